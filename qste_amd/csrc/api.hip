@@ -51,8 +51,9 @@ int mfma_backward_pair(const void*, int, const uint8_t*, int64_t, const uint16_t
                        const float*, float*, const EvidencePlan&, float*, hipStream_t);
 int launch_transpose_bits(const uint8_t*, uint8_t*, int64_t, int64_t, int64_t, int64_t, hipStream_t);
 int launch_f32_to_16(const float*, uint16_t*, int64_t, int64_t, int, hipStream_t);
-int gemv_linear_forward(const void*, int, const uint8_t*, const float*, const float*, void*, int64_t,
-                        int64_t, int64_t, hipStream_t);
+size_t gemv_forward_workspace(int64_t, int64_t, int64_t, int);
+int gemv_linear_forward(const void*, int, const uint8_t*, const float*, const float*, void*, int64_t, int64_t,
+                        int64_t, void*, size_t, hipStream_t);
 int launch_swiglu_forward(const void*, const void*, int, void*, uint8_t*, float*, float*, int64_t, int64_t,
                           hipStream_t);
 int launch_swiglu_backward(const void*, const void*, const void*, int, void*, void*, int64_t, hipStream_t);
@@ -131,7 +132,7 @@ BackwardLayout backward_layout(int64_t samples, int64_t rows, int64_t cols, bool
 
 int forward_dispatch(const void* x, int dtype, const uint8_t* packed, const float* scale,
                      const float* bias, void* y, int64_t m, int64_t rows, int64_t cols, hipStream_t s) {
-  int rc = gemv_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, s);
+  int rc = gemv_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, nullptr, 0, s);
   if (rc != 1) return rc;
   rc = mfma_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, s);
   if (rc != 1) return rc;
@@ -229,6 +230,7 @@ int qste_packed_linear_affine(const void* x, int dtype, const uint8_t* packed, c
 }
 
 size_t qste_packed_linear_affine_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int dtype) {
+  if (const size_t skinny = gemv_forward_workspace(m, rows, cols, dtype)) return skinny;
   return dtype == QSTE_F32 ? f32_forward_workspace(m, rows, cols) : mfma_forward_split_workspace(m, rows, cols, dtype);
 }
 
@@ -239,6 +241,11 @@ int qste_packed_linear_affine_ws(const void* x, int dtype, const uint8_t* packed
   if (m < 0 || rows < 0 || cols < 0) return QSTE_E_SHAPE;
   if (m * rows == 0) return 0;
   if (!y || !scale || (cols > 0 && (!x || !packed))) return QSTE_E_NULL;
+  if (cols > 0) {
+    const int rc = gemv_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, workspace, workspace_bytes,
+                                       as_stream(stream));
+    if (rc != 1) return rc;
+  }
   if (dtype == QSTE_F32 && cols > 0) {
     const int rc = mfma_f32_forward(static_cast<const float*>(x), packed, scale, bias, static_cast<float*>(y), m,
                                     rows, cols, workspace, workspace_bytes, as_stream(stream));

@@ -1465,6 +1465,14 @@ inline size_t up256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 }  // namespace limbs
 
+// The limbs of x [rows, cols] as rows of their own: out [3 rows, cols], row
+// 3r + i limb i (hi, mid, lo) of row r.
+int launch_limbs(const float* x, int64_t rows, int64_t cols, uint16_t* out, hipStream_t stream) {
+  limbs::split_kernel<<<limbs::grid_for(rows * cols), 256, 0, stream>>>(x, rows, cols, nullptr, nullptr, out, 3 * cols,
+                                                                        cols);
+  return static_cast<int>(hipGetLastError());
+}
+
 int launch_transpose_bits(const uint8_t*, uint8_t*, int64_t, int64_t, int64_t, int64_t, hipStream_t);
 
 // Whether a product of these sizes takes the limbs (enough rows of output to

@@ -1,60 +1,65 @@
-// Skinny-M forward (decode): y[m, n] = (sum_k x[m, k] sign[n, k]) * scale[n]
-// + bias[n] for M <= 16 bf16 rows (fallback.py:95-108; the small-batch path of
-// the reference GPU backend, cuda.py:198-501).
+// Skinny forward (decode and small batches): y[m, n] = (sum_k x[m, k]
+// sign[n, k]) * scale[n] + bias[n] for up to 64 rows of bf16 / fp16 x, or up
+// to 21 rows of fp32 x as three bf16 limbs each (fallback.py:95-108; the
+// small-batch path of the reference GPU backend, cuda.py:198-501).
 //
-// The weight bits (R * C / 8 bytes) are the only large operand and are read
-// once from HBM, so the kernel has to stream them at memory speed.  Two costs
-// stand in the way on CDNA4, and the design answers both:
+// The weight bits (N * K / 8 bytes) are the only large operand and each bit
+// is used for a few rows only, so what the kernel spends per bit decides its
+// time.  Expanding bits to +-1 operands costs the VALU one instruction per
+// pair of weights at best (the matrix cores then wait for it).  Here the
+// bits never become operand values:
 //
-// * Sign expansion.  Turning bits into +-1 bf16 costs at least two VALU ops per
-//   element pair with a shift-and-mask scheme (about 6 us of VALU time at
-//   M=1 for the config-5 matrix, more than the 3.7 us of HBM time).  Here a
-//   bit becomes a bf16 of value v0 + 0.5 * bit with ONE v_and_or_b32 per
-//   element pair: from one of four shifted copies of a weight dword (w << 4,
-//   w, w >> 4, w >> 8), bit a in 4..7 of each 16-bit half is OR-ed into the
-//   mantissa (a = 4..6) or the exponent LSB (a = 7) of the power-of-two base
-//   v0 = 4, 2, 1, 0.5, whose bit a is clear; every set bit therefore adds
-//   exactly 0.5.  With v0(k) = 4, 2, 1, 0.5 for k mod 4 = 0..3 the MFMA sums
-//       acc[m, n] = sum_k x[m, k] v0(k) + 0.5 * sum_{k: bit} x[m, k]
-//   and with C[m] = sum_k x[m, k] v0(k), S[m] = sum_k x[m, k]:
-//       sum_k x[m, k] sign[n, k] = 2 * sum_{bit} x - S = 4 * acc - (4 C + S).
-//   C and S come from one more MFMA per x fragment against the bases (column
-//   0) and ones (column 1).  All values involved are exact in bf16; since
-//   v0 <= 8 * 0.5, the cancellation costs about 3 of fp32's 24 bits.
-// * Sharing x.  Each wave keeps its x fragments in registers and uses every
-//   one for 7-8 weight blocks of 16 rows (not once per block from LDS).
+// * Weights as the sparsity indexes of v_smfmac_f32_16x16x64.  That
+//   instruction multiplies a 4:2 sparse A (its nonzero values and a 2-bit
+//   index per value that says which element of its group of four it is)
+//   with a dense B.  B holds every x twice, negated and plain, as the pair
+//   (-x[k], x[k]); the two nonzeros of a group pick one element of each of
+//   its two pairs.  All of A's values are 1.0, and the index of a value is
+//   its weight bit (plus 2 for the second pair of the group): bit set picks
+//   x[k], clear picks -x[k].  So 16 consecutive even (or odd) bits of a
+//   weight dword, masked and OR-ed with the constant second-pair bits, are
+//   the index operand as they are: 3 VALU instructions turn 32 weights of a
+//   lane into the operands of 4 MFMAs, against 20 for bit expansion.  The
+//   products are exact (x or -x), the sums the MFMA's fp32 sums.
+// * x fragments (pairs) are formed once per 32 columns from LDS and used for
+//   NBW blocks of 16 weight rows.
 //
-// Work split: a workgroup of 8 waves owns 16 * NBW weight rows (NBW chosen so
-// the grid is about one workgroup per CU); its waves split K in chunks of 512
-// columns (lane group q of a wave reads 16 bytes = 128 columns of each row),
-// all weight loads of a wave are issued before its first MFMA, and the 8
-// partial accumulators are summed through LDS in a fixed order.  The x rows
-// of a chunk reach the wave through its own LDS rows (direct buffer->LDS
-// loads of one contiguous kilobyte per row) instead of per-lane 16-byte loads
-// that touch 16 rows of x each.
+// MFMA layout: lane l holds A row l%16, nonzeros e = 0..7 of logical k
+// 16(l/16) + 2e, + 2e + 1; B column l%16, values i = 0..7 at logical k
+// 8(l/16) + i and i = 8..15 at 32 + 8(l/16) + i - 8; the accumulator's
+// register j holds D[4(l/16) + j][l%16].  D's rows are weight rows and its
+// columns rows of x, so each lane ends with four consecutive outputs of one
+// row of y.  A lane group g's index dword covers columns 128g + 32j + 0..31
+// of a 512-column chunk (j: which of its four dwords): the even bits are two
+// MFMAs (the low half, then the high half of the index register), the odd
+// bits two more.
 //
-// MFMA 16x16x32 bf16 layout: lane l holds A[l%16][8(l/16) + i] and
-// B[8(l/16) + i][l%16]; accumulator register j holds D[4(l/16) + j][l%16].
-// Which k each of a lane group's 8 slots stands for is free as long as A and
-// B agree: for a weight dword w (32 columns from k0), MFMA u (0..3) takes the
-// copy w_u = w << 4, w, w >> 4, w >> 8, and its slot pair a' (0..3) holds
-// columns k0 + 4u + a' (low half, bit 4 + a' of w_u) and k0 + 16 + 4u + a'
-// (high half, bit 20 + a' of w_u).
+// Work split: a workgroup of 8 waves owns 16 * NBW weight rows over one of
+// `splits` ranges of K; its waves take the range's 512-column chunks in
+// turn, each wave with x rows of its own in LDS (no barrier until the end),
+// and the 8 partial accumulators are summed through LDS in wave order.  With
+// splits > 1 the range sums go to a caller workspace and a second kernel adds
+// them in range order: every workgroup reads all of x's rows over its range,
+// so at many rows of x and few rows of weights x's traffic from L2 is what
+// splitting K saves.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace qste {
 namespace gemv {
 
-typedef short bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x16_t __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x8 __attribute__((ext_vector_type(8)));
 
 constexpr int WAVES = 8;
 constexpr int THREADS = 64 * WAVES;
 constexpr int CHUNK_K = 512;  // columns per wave chunk (4 lane groups x 128)
-constexpr int DEPTH = 2;      // weight loads in flight per wave (swept 2-16: fewer requests per wave keep the
-                              // CUs' streams interleaved; 2 is fastest at M = 4 and 16)
 constexpr uint32_t kRsrcWord3 = 0x00020000u;
 constexpr uint32_t kOob = 0x80000000u;  // an offset past every buffer: reads zero
 
@@ -67,333 +72,602 @@ __device__ __forceinline__ u32x4 ld128(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 0));
 }
 
-// a literal held in a VGPR (VOP3 instructions take at most one SGPR and no
-// literal on gfx9, so the base of each v_and_or_b32 lives in a VGPR)
-template <uint32_t V>
-__device__ __forceinline__ uint32_t vreg() {
-  uint32_t v;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(v) : "i"(V));
-  return v;
-}
-
-// Per activation dtype: the 16-bit pairs of the bases v0 = 4, 2, 1, 0.5,
-// the position of slot a' = 0's bit in each half-word (bf16: bits 4..7,
-// fp16: bits 7..10 -- the top three mantissa bits and the exponent LSB in
-// both, which add exactly 0.5 to bases 4, 2, 1, 0.5, whose bit there is
-// clear), the pair of ones, and the MFMA.
+// Per 16-bit type: the pair of ones and the sparse MFMA (H: which half of the
+// index register).
 template <int DT>
-struct Dec;
+struct Op;
 
 template <>
-struct Dec<QSTE_BF16> {
-  static constexpr uint32_t base[4] = {0x40804080u, 0x40004000u, 0x3F803F80u, 0x3F003F00u};
-  static constexpr int pos = 4;
+struct Op<QSTE_BF16> {
   static constexpr uint32_t ones = 0x3F803F80u;
-  static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
+  template <int H>
+  static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x8 b, f32x4 c, uint32_t index) {
+    return __builtin_amdgcn_smfmac_f32_16x16x64_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                     __builtin_bit_cast(bf16x16_t, b), c, static_cast<int>(index), 0,
+                                                     H);
   }
-  static __device__ __forceinline__ uint16_t store(float v) { return f32_to_bf16(v); }
 };
 
 template <>
-struct Dec<QSTE_F16> {
-  static constexpr uint32_t base[4] = {0x44004400u, 0x40004000u, 0x3C003C00u, 0x38003800u};
-  static constexpr int pos = 7;
+struct Op<QSTE_F16> {
   static constexpr uint32_t ones = 0x3C003C00u;
-  static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
-                                                  0, 0);
+  template <int H>
+  static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x8 b, f32x4 c, uint32_t index) {
+    return __builtin_amdgcn_smfmac_f32_16x16x64_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x16_t, b),
+                                                    c, static_cast<int>(index), 0, H);
   }
-  static __device__ __forceinline__ uint16_t store(float v) { return f32_to_f16(v); }
 };
-
-// Copy u (0..3) of a weight dword: the column 4u + a' (low half) and
-// 16 + 4u + a' (high half) bits moved to position pos + a' of each half.
-template <int POS>
-__device__ __forceinline__ uint32_t weight_copy(uint32_t w, int u) {
-  const int shift = POS - 4 * u;  // compile-time after unrolling
-  return shift >= 0 ? w << shift : w >> -shift;
-}
-
-// Workgroup barrier that waits only for this wave's LDS operations.
-// (__syncthreads() also waits for every outstanding global load, which here
-// would make the prologue wait for the whole weight stream.)
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 
 typedef __attribute__((address_space(3))) void lds_t;
-constexpr int XP = 1024 + 16;  // LDS bytes per staged x row: conflict-free 16-byte reads across 16 rows
 
-template <int NBW, int MP>
-struct Smem {
-  static constexpr int x_bytes = WAVES * MP * XP;
-  static constexpr int red_bytes = WAVES * (NBW + 1) * 64 * 16;
-  static constexpr int bytes = x_bytes > red_bytes ? x_bytes : red_bytes;
+// Wait until at most N of this wave's vector-memory loads are in flight.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  // s_waitcnt fields: vmcnt [3:0] and [15:14], expcnt [6:4] (7: none), lgkmcnt [11:8] (15: none)
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | (((N >> 4) & 3) << 14) | 0xF70);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// What a launch is given besides the operands.
+struct Args {
+  const uint16_t* x;    // [xr, K] 16-bit rows (fp32: three limb rows per row)
+  const uint8_t* bits;  // [N, K / 8]
+  const float* scale;
+  const float* bias;    // may be null
+  void* y;              // [xr / limbs, N] (16-bit, or fp32 with limbs)
+  float* partial;       // splits > 1: [splits][xr][N]
+  int xr;               // rows of x
+  int limbs;            // 1, or 3 (y in fp32, row m = rows 3m .. 3m + 2 of x)
+  int splits;
+  int chunks_per_split;
+  int64_t N, K;
 };
 
-// NBW weight blocks of 16 rows per workgroup; x rows staged MP (>= M, a
-// power of two) at a time.
-template <int DT, int NBW, int MP>
-__global__ __launch_bounds__(THREADS, 1) void decode_kernel(const uint16_t* __restrict__ x,
-                                                            const uint8_t* __restrict__ bits,
-                                                            const float* __restrict__ scale,
-                                                            const float* __restrict__ bias,
-                                                            uint16_t* __restrict__ y, int M, int64_t N,
-                                                            int64_t K) {
-  __shared__ __attribute__((aligned(16))) uint8_t smem[Smem<NBW, MP>::bytes];
-  __shared__ float dsum[16];
+// Four outputs n .. n + 3 of row m from their sums.
+template <int OUT>
+__device__ __forceinline__ void finish4(const Args& p, int64_t m, int64_t n, f32x4 v, const float* sc,
+                                        const float* bi, bool vec) {
+  float r[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    r[j] = v[j] * sc[j];
+    r[j] = r[j] + bi[j];
+  }
+  const int64_t at = m * p.N + n;
+  if constexpr (OUT == QSTE_F32) {
+    float* y = static_cast<float*>(p.y);
+    if (vec) {
+      *reinterpret_cast<float4*>(y + at) = make_float4(r[0], r[1], r[2], r[3]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n + j < p.N) y[at + j] = r[j];
+    }
+  } else {
+    uint16_t* y = static_cast<uint16_t*>(p.y);
+    uint16_t h[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h[j] = OUT == QSTE_F16 ? f32_to_f16(r[j]) : f32_to_bf16(r[j]);
+    if (vec) {
+      *reinterpret_cast<uint2*>(y + at) = make_uint2(h[0] | (static_cast<uint32_t>(h[1]) << 16),
+                                                     h[2] | (static_cast<uint32_t>(h[3]) << 16));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n + j < p.N) y[at + j] = h[j];
+    }
+  }
+}
+
+// XR rows of x are staged (>= p.xr: 4 or a multiple of 16; rows past p.xr
+// are left as they are, their outputs are never stored), NBW blocks of 16
+// weight rows per workgroup.  RESIDENT: a chunk's fragments are all formed
+// first and the blocks streamed past them.
+template <int XR, int NBW, bool RESIDENT>
+struct Cfg {
+  static constexpr int MT = (XR + 15) / 16;                     // MFMA columns / 16
+  static constexpr int STAGES = XR <= 16 ? 1 : 4;               // x stages per chunk
+  static constexpr int JS = 4 / STAGES;
+  // one stage: whole chunks of a row (1 KB and a pad: the 16 rows of a
+  // fragment read cover all banks), or 256 bytes of a row (16-byte piece i of
+  // row r at slot i ^ (r % 16))
+  static constexpr int PITCH = STAGES == 1 ? 1040 : 256;
+  // chunks of x in LDS at a time: below 16 rows there is room for two, which
+  // takes x's latency out of a wave's chain of chunks
+  static constexpr int XBUF = XR < 16 && !RESIDENT ? 2 : 1;
+  static constexpr int x_bytes = XBUF * XR * PITCH;             // per wave
+  static constexpr int red_bytes = WAVES * NBW * MT * 64 * 16;
+  static constexpr int bytes = WAVES * x_bytes > red_bytes ? WAVES * x_bytes : red_bytes;
+  // weight loads in flight: a chunk's, or two where blocks are streamed (the
+  // CUs' streams stay interleaved; 4 in flight: 4-6% slower at M = 1)
+  static constexpr int D = !RESIDENT ? NBW : (NBW < 2 ? NBW : 2);
+};
+
+template <int DT, int XR, int NBW, bool RESIDENT>
+__global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
+  using C = Cfg<XR, NBW, RESIDENT>;
+  static_assert(!RESIDENT || XR <= 16, "fragments of one tile fit the registers");
+  constexpr int MT = C::MT, JS = C::JS, D = C::D;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[C::bytes];
+  __shared__ float epi[2][16 * NBW];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, q = lane >> 4;
-  const int64_t pb = K / 8;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * (16 * NBW);
-  const int nchunks = static_cast<int>((K + CHUNK_K - 1) / CHUNK_K);
+  const int64_t K = p.K, pb = K / 8;
+  // consecutive workgroups land on different XCDs: with the range as the
+  // fastest index, an XCD's workgroups read few ranges of x
+  const int range = static_cast<int>(blockIdx.x) % p.splits;
+  const int64_t n0 = static_cast<int64_t>(static_cast<int>(blockIdx.x) / p.splits) * (16 * NBW);
+  const int c_first = range * p.chunks_per_split;
+  const int c_all = static_cast<int>((K + CHUNK_K - 1) / CHUNK_K);
+  const int c_last = min(c_first + p.chunks_per_split, c_all);
 
-  // rows past N and x rows past M read zero through the buffer bounds
-  const __amdgpu_buffer_rsrc_t rb = rsrc(bits, N * pb);
-  const __amdgpu_buffer_rsrc_t rx = rsrc(x, static_cast<int64_t>(M) * K * 2);
+  // rows past N read zero through the buffer bounds
+  const __amdgpu_buffer_rsrc_t rb = rsrc(p.bits, p.N * pb);
+  const __amdgpu_buffer_rsrc_t rx = rsrc(p.x, static_cast<int64_t>(p.xr) * K * 2);
   uint32_t boff[NBW];
 #pragma unroll
   for (int b = 0; b < NBW; ++b) boff[b] = static_cast<uint32_t>((n0 + 16 * b + l16) * pb + 16 * q);
 
-  using T = Dec<DT>;
-  uint32_t base[4];
-  base[0] = vreg<T::base[0]>(); base[1] = vreg<T::base[1]>();
-  base[2] = vreg<T::base[2]>(); base[3] = vreg<T::base[3]>();
-  // B of the C/S product (the same for every MFMA): column 0 the bases,
-  // column 1 ones, the rest zero
-  const uint32_t cs_one = l16 == 1 ? T::ones : 0u;
-  u32x4 cf;
-  cf.x = l16 == 0 ? base[0] : cs_one;
-  cf.y = l16 == 0 ? base[1] : cs_one;
-  cf.z = l16 == 0 ? base[2] : cs_one;
-  cf.w = l16 == 0 ? base[3] : cs_one;
-
-  f32x4 acc[NBW];
+  uint8_t* xs = smem + wave * C::x_bytes;
+  auto issue_x = [&](int c, int stage, int buf = 0) {
+    // columns past K (a last chunk that K ends inside) read zero
+    if constexpr (C::STAGES == 1) {
+      const uint32_t off =
+          c < c_last && CHUNK_K * c + 8 * lane < K ? 1024u * static_cast<uint32_t>(c) + 16u * lane : kOob;
+      auto row = [&](int r, uint32_t at) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_t*)(xs + (buf * XR + r) * C::PITCH), 16,
+                                                 static_cast<int>(at), static_cast<int>(r * K * 2), 0, 0);
+      };
+      if constexpr (C::XBUF > 1) {  // always XR loads: the waits below count them
 #pragma unroll
-  for (int b = 0; b < NBW; ++b) acc[b] = f32x4{};
-  f32x4 acc_cs = f32x4{};
+        for (int r = 0; r < XR; ++r) row(r, r < p.xr ? off : kOob);
+      } else {
+        for (int r = 0; r < p.xr; ++r) row(r, off);
+      }
+    } else {
+      const int col = CHUNK_K * c + 128 * stage;
+#pragma unroll
+      for (int r = 0; r < XR; r += 4) {
+        if (r >= p.xr) break;
+        const int row = r + (lane >> 4), piece = (lane & 15) ^ (row & 15);
+        const uint32_t off = col + 8 * piece < K ? static_cast<uint32_t>((lane >> 4) * K * 2 + 16 * piece) : kOob;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_t*)(xs + r * C::PITCH), 16, static_cast<int>(off),
+                                                 static_cast<int>(r * K * 2 + 2 * static_cast<int64_t>(col)), 0, 0);
+      }
+    }
+  };
+  // The weights of a lane group g cover columns 128g + 32j of the chunk with
+  // dword j where a stage holds whole chunks, and 128j + 32g (the 4 x 4
+  // transpose of groups and dwords, by_stage below) where stage j holds
+  // columns 128j .. + 127.  This lane's x of dword j, tile mt, half-dword H
+  // and logical k half h: 8 columns at 16H + 8(q%2) of the 32 columns of
+  // group 2h + q/2.
+  auto read_x = [&](int j, int mt, int H, int h, int buf = 0) {
+    const int g = 2 * h + (q >> 1);
+    if constexpr (C::STAGES == 1) {
+      const int row = buf * XR + (XR >= 16 ? l16 : l16 % XR);
+      return *reinterpret_cast<const u32x4*>(xs + row * C::PITCH + 256 * g + 64 * j + 32 * H + 16 * (q & 1));
+    } else {
+      const int row = 16 * mt + l16, piece = (4 * g + 2 * H + (q & 1)) ^ l16;
+      return *reinterpret_cast<const u32x4*>(xs + row * C::PITCH + 16 * piece);
+    }
+  };
+  auto by_stage = [&](u32x4 w) {
+    if constexpr (C::STAGES == 1) return w;
+    const auto a = __builtin_amdgcn_permlane16_swap(w[0], w[1], false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(w[2], w[3], false, false);
+    const auto e = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+    const auto o = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+    return u32x4{e[0], o[0], e[1], o[1]};
+  };
 
-  // the epilogue's row scale and bias, fetched now so their latency is not
-  // paid after the reduction (thread t finishes column n0 + 16 (t / 64) + t % 16)
-  const int64_t n_out = n0 + 16 * (tid >> 6) + (tid & 15);
-  float out_scale = 0.0f, out_bias = 0.0f;
-  if (tid < 64 * NBW && n_out < N) {
-    out_scale = scale[n_out];
-    out_bias = bias ? bias[n_out] : 0.0f;
+  u32x4 W[NBW];
+  auto issue_w1 = [&](int c, int b) { return ld128(rb, c < c_last ? boff[b] + 64u * static_cast<uint32_t>(c) : kOob); };
+
+  f32x4 acc[NBW][MT];
+#pragma unroll
+  for (int b = 0; b < NBW; ++b)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[b][mt] = f32x4{};
+  const u32x4 ones = {Op<DT>::ones, Op<DT>::ones, Op<DT>::ones, Op<DT>::ones};
+  auto pairs = [&](uint32_t v, int odd) {  // (-x, x) of the even or the odd one of two columns
+    return __builtin_amdgcn_perm(v, v ^ 0x80008000u, odd ? 0x07060302u : 0x05040100u);
+  };
+  auto even_index = [](uint32_t w) { return (w & 0x55555555u) | 0x88888888u; };
+  auto odd_index = [](uint32_t w) { return ((w >> 1) & 0x55555555u) | 0x88888888u; };
+
+  int c = c_first + wave;
+  if (c < c_last) {
+    issue_x(c, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < D; ++b) W[b] = issue_w1(c, b);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (C::XBUF > 1) issue_x(c + WAVES, 0, 1);
+    __builtin_amdgcn_sched_barrier(0);
   }
-
-  // x rows of a chunk go to this wave's own LDS rows with one direct
-  // buffer->LDS load per row (1 KB, lane-contiguous, so every instruction
-  // reads one contiguous kilobyte); no other wave touches them, so no
-  // workgroup barrier is needed
-  uint8_t* xr = smem + wave * MP * XP;
-  auto issue_x = [&](int c) {
-    // lane l brings columns 512c + 8l .. + 7; columns past K (a last chunk
-    // that K ends inside) and rows past M read zero
-    const bool live = c < nchunks && CHUNK_K * c + 8 * lane < K;
-    const uint32_t off = static_cast<uint32_t>(c) * 1024u + 16u * lane;
+  // the epilogue's row scale and bias, fetched while the first loads fly
+  float out_scale = 0.0f, out_bias = 0.0f;
+  if (tid < 16 * NBW && n0 + tid < p.N) {
+    out_scale = p.scale[n0 + tid];
+    out_bias = p.bias ? p.bias[n0 + tid] : 0.0f;
+  }
+  if constexpr (RESIDENT) {
+    for (; c < c_last; c += WAVES) {
+      wait_vm<D>();  // all but the newest loads, the weights in flight: x is in LDS
+      u32x8 f[4][2][2];
 #pragma unroll
-    for (int m = 0; m < MP; ++m)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_t*)(xr + m * XP), 16,
-                                               live ? off + static_cast<uint32_t>(m * K * 2) : kOob, 0, 0, 0);
-  };
-  // this lane's 128 columns of its x row.  Lanes of rows past MP read row
-  // l16 % MP instead: output rows m >= M are never stored, and an MFMA output
-  // row depends only on the same row of A, so those rows may hold any finite
-  // values (and identical addresses are broadcast by the LDS)
-  auto read_x = [&](u32x4 (&Xd)[16]) {
-    const uint8_t* src = xr + (l16 & (MP - 1)) * XP + 256 * q;
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) Xd[i] = *reinterpret_cast<const u32x4*>(src + 16 * i);
-    // the next chunk's direct loads overwrite these rows: the values must
-    // live in registers from here on, not be re-read from LDS later
+        for (int H = 0; H < 2; ++H) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(Xd[i]));
-  };
-  // The 16 x fragments of a chunk (one per 32-column group j and MFMA u;
-  // slot pair a' holds columns 4u + a' and 16 + 4u + a' of the group),
-  // permuted once and used for every weight block of the chunk.
-  auto fragments = [&](const u32x4 (&Xd)[16], u32x4 (&af)[16]) {
+          for (int h = 0; h < 2; ++h) {
+            const u32x4 v = read_x(j, 0, H, h);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      uint32_t xg[16];  // columns k0 + 2i, k0 + 2i + 1 of group j
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) xg[i] = Xd[4 * j + i / 4][i % 4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        af[4 * j + u].x = __builtin_amdgcn_perm(xg[8 + 2 * u], xg[2 * u], 0x05040100u);
-        af[4 * j + u].y = __builtin_amdgcn_perm(xg[8 + 2 * u], xg[2 * u], 0x07060302u);
-        af[4 * j + u].z = __builtin_amdgcn_perm(xg[9 + 2 * u], xg[2 * u + 1], 0x05040100u);
-        af[4 * j + u].w = __builtin_amdgcn_perm(xg[9 + 2 * u], xg[2 * u + 1], 0x07060302u);
-      }
-    }
-  };
-  auto block = [&](const u32x4 (&af)[16], const u32x4& Bd, int b) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t w = Bd[j];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint32_t wu = weight_copy<T::pos>(w, u);
-        constexpr uint32_t m0 = 0x00010001u << T::pos;
-        u32x4 bf;
-        bf.x = (wu & m0) | base[0];
-        bf.y = (wu & (m0 << 1)) | base[1];
-        bf.z = (wu & (m0 << 2)) | base[2];
-        bf.w = (wu & (m0 << 3)) | base[3];
-        acc[b] = T::mma(af[4 * j + u], bf, acc[b]);
-      }
-    }
-  };
-
-  // Chunks wave and wave + 8 (all of K up to 8192; larger K loops), their
-  // 2 * NBW weight blocks streamed through a ring of DEPTH loads in flight:
-  // the load of block i + DEPTH is issued when block i is consumed.  (All
-  // loads at once would make every block complete only at the end of the
-  // whole transfer, leaving no compute to overlap with it.)
-  constexpr int STEPS = 2 * NBW;
-  constexpr int D = DEPTH < STEPS ? DEPTH : STEPS;
-  for (int c0 = wave; c0 < nchunks; c0 += 2 * WAVES) {
-    const int c1 = c0 + WAVES;
-    u32x4 X[16], af[16], Bs[STEPS];
-    auto issue_step = [&](int i) {
-      const int c = i < NBW ? c0 : c1, b = i < NBW ? i : i - NBW;
-      Bs[i] = ld128(rb, c < nchunks ? boff[b] + 64u * static_cast<uint32_t>(c) : kOob);
-    };
-    issue_x(c0);
-#pragma unroll
-    for (int i = 0; i < D; ++i) issue_step(i);
-    __builtin_amdgcn_sched_barrier(0);
-    read_x(X);
-    // the x rows are read before the next chunk's rows overwrite them
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    __builtin_amdgcn_sched_barrier(0);
-    issue_x(c1);
-    __builtin_amdgcn_sched_barrier(0);
-    fragments(X, af);
-#pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-      if (i + D < STEPS) issue_step(i + D);
-      if (i == NBW) {
-        read_x(X);
-        fragments(X, af);
-      }
+              for (int o = 0; o < 2; ++o) f[j][H][o][4 * h + i] = pairs(v[i], o);
+          }
+          asm volatile("" : "+v"(f[j][H][0]), "+v"(f[j][H][1]));
+        }
+      // the x rows are in registers from here on: the next chunk's may land
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
       __builtin_amdgcn_sched_barrier(0);
-      block(af, Bs[i], i < NBW ? i : i - NBW);
-      if (i == NBW - 1 || i == STEPS - 1) {
-#pragma unroll
-        for (int f = 0; f < 16; ++f) acc_cs = T::mma(af[f], cf, acc_cs);
-      }
+      if (c + WAVES < c_last) issue_x(c + WAVES, 0);
       __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < NBW; ++b) {
+        const u32x4 w = W[b];
+        auto next = [&] {  // the load D blocks ahead
+          if (b + D < NBW) W[b + D] = issue_w1(c, b + D);
+          else W[b + D - NBW] = issue_w1(c + WAVES, b + D - NBW);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        if (D < NBW) next();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t e = even_index(w[j]), o = odd_index(w[j]);
+          acc[b][0] = Op<DT>::template mma<0>(ones, f[j][0][0], acc[b][0], e);
+          acc[b][0] = Op<DT>::template mma<0>(ones, f[j][0][1], acc[b][0], o);
+          acc[b][0] = Op<DT>::template mma<1>(ones, f[j][1][0], acc[b][0], e);
+          acc[b][0] = Op<DT>::template mma<1>(ones, f[j][1][1], acc[b][0], o);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (D == NBW) next();
+      }
     }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
+  } else {
+    u32x4 Wn[NBW];
+    for (int buf = 0; c < c_last; c += WAVES, buf ^= C::XBUF - 1) {
+      const int cn = c + WAVES;
+      if constexpr (C::STAGES > 1) {
+        wait_vm<0>();
+#pragma unroll
+        for (int b = 0; b < NBW; ++b) W[b] = by_stage(W[b]);
+      }
+#pragma unroll
+      for (int st = 0; st < C::STAGES; ++st) {
+        // the next chunk's weights go out behind this chunk's last x stage
+        // (loads complete in order: x must not wait for weights not needed yet)
+        if (st == C::STAGES - 1) {
+#pragma unroll
+          for (int b = 0; b < NBW; ++b) Wn[b] = issue_w1(cn, b);
+          // all but the loads just issued (and the x of the chunk after
+          // this one, issued before them): the stage is in LDS
+          wait_vm<NBW + (C::XBUF - 1) * XR>();
+        } else {
+          wait_vm<0>();
+        }
+#pragma unroll
+        for (int jj = 0; jj < JS; ++jj) {
+          const int j = JS * st + jj;
+          u32x4 raw[MT][2][2];
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int H = 0; H < 2; ++H)
+#pragma unroll
+              for (int h = 0; h < 2; ++h) raw[mt][H][h] = read_x(j, mt, H, h, buf);
+          if (jj == JS - 1) {
+            // the stage is in registers from here on: the next one's direct
+            // loads may overwrite it
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+              for (int H = 0; H < 2; ++H)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(raw[mt][H][h]));
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+            __builtin_amdgcn_sched_barrier(0);
+            if (st + 1 < C::STAGES) issue_x(c, st + 1);
+            else if (C::XBUF > 1) issue_x(cn + WAVES, 0, buf);
+            else if (cn < c_last) issue_x(cn, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          uint32_t index[NBW][2];
+#pragma unroll
+          for (int b = 0; b < NBW; ++b) {
+            index[b][0] = even_index(W[b][j]);
+            index[b][1] = odd_index(W[b][j]);
+          }
+          auto half = [&](auto half_index) {
+            constexpr int H = decltype(half_index)::value;
+            u32x8 f[MT][2];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+              for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int o = 0; o < 2; ++o) f[mt][o][i] = pairs(raw[mt][H][i >> 2][i & 3], o);
+#pragma unroll
+            for (int o = 0; o < 2; ++o)
+#pragma unroll
+              for (int b = 0; b < NBW; ++b)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                  acc[b][mt] = Op<DT>::template mma<H>(ones, f[mt][o], acc[b][mt], index[b][o]);
+          };
+          half(std::integral_constant<int, 0>{});
+          half(std::integral_constant<int, 1>{});
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < NBW; ++b) W[b] = Wn[b];
+    }
   }
 
   // partial sums of the 8 waves, added in wave order
-  __syncthreads();
-  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [WAVES][NBW + 1][64]
-#pragma unroll
-  for (int b = 0; b < NBW; ++b) red[(wave * (NBW + 1) + b) * 64 + lane] = acc[b];
-  red[(wave * (NBW + 1) + NBW) * 64 + lane] = acc_cs;
-  __syncthreads();
-  if (tid < 16) {
-    // row m = tid: C at (lane 16(m/4), reg m%4), S at the next lane
-    const int src = 16 * (tid >> 2), j = tid & 3;
-    float c = 0.0f, s = 0.0f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      c += red[(w * (NBW + 1) + NBW) * 64 + src][j];
-      s += red[(w * (NBW + 1) + NBW) * 64 + src + 1][j];
-    }
-    dsum[tid] = 4.0f * c + s;
+  if (tid < 16 * NBW) {
+    epi[0][tid] = out_scale;
+    epi[1][tid] = out_bias;
   }
   __syncthreads();
-  if (tid < 64 * NBW) {
-    const int b = tid >> 6, l = tid & 63;
-    f32x4 v = red[b * 64 + l];
+  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [WAVES][NBW * MT][64]
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) v += red[(w * (NBW + 1) + b) * 64 + l];
-    const int64_t n = n_out;
-    if (n < N) {
-      const float sc = out_scale;
-      const float bi = out_bias;
+  for (int b = 0; b < NBW; ++b)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int m = 4 * (l >> 4) + j;
-        if (m < M) {
-          float r = 4.0f * v[j] - dsum[m];
-          r = r * sc;
-          r = r + bi;
-          y[static_cast<int64_t>(m) * N + n] = T::store(r);
-        }
+    for (int mt = 0; mt < MT; ++mt) red[(wave * NBW * MT + b * MT + mt) * 64 + lane] = acc[b][mt];
+  __syncthreads();
+  auto total = [&](int b, int row, int g) {  // x row `row`, weight rows 16b + 4g + 0..3
+    const int at = (b * MT + (row >> 4)) * 64 + 16 * g + (row & 15);
+    f32x4 v = red[at];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) v += red[w * NBW * MT * 64 + at];
+    return v;
+  };
+  const bool full = (p.N & 3) == 0;
+  if (p.splits > 1) {
+    float* part = p.partial + static_cast<int64_t>(range) * p.xr * p.N;
+    for (int i = tid; i < NBW * p.xr * 4; i += THREADS) {
+      const int g = i & 3, b = (i >> 2) % NBW, row = (i >> 2) / NBW;
+      const int64_t n = n0 + 16 * b + 4 * g;
+      if (n >= p.N) continue;
+      const f32x4 v = total(b, row, g);
+      float* d = part + static_cast<int64_t>(row) * p.N + n;
+      if (full) {
+        *reinterpret_cast<f32x4*>(d) = v;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (n + j < p.N) d[j] = v[j];
       }
     }
+    return;
+  }
+  const int rows = p.xr / p.limbs;
+  const int align = p.limbs == 3 ? 15 : 7;
+  const bool vec = full && (reinterpret_cast<uintptr_t>(p.y) & align) == 0;
+  for (int i = tid; i < NBW * rows * 4; i += THREADS) {
+    const int g = i & 3, b = (i >> 2) % NBW, m = (i >> 2) / NBW;
+    const int64_t n = n0 + 16 * b + 4 * g;
+    if (n >= p.N) continue;
+    const float* sc = &epi[0][16 * b + 4 * g];
+    const float* bi = &epi[1][16 * b + 4 * g];
+    if (p.limbs == 3) {
+      const f32x4 v = (total(b, 3 * m + 2, g) + total(b, 3 * m + 1, g)) + total(b, 3 * m, g);
+      finish4<QSTE_F32>(p, m, n, v, sc, bi, vec);
+    } else {
+      finish4<DT>(p, m, n, total(b, m, g), sc, bi, vec);
+    }
   }
 }
 
-template <int DT, int NBW, int MP>
-void launch(const void* x, const uint8_t* packed, const float* scale, const float* bias, void* y, int64_t m,
-            int64_t rows, int64_t cols, hipStream_t stream) {
-  const int grid = static_cast<int>((rows + 16 * NBW - 1) / (16 * NBW));
-  decode_kernel<DT, NBW, MP><<<grid, THREADS, 0, stream>>>(static_cast<const uint16_t*>(x), packed, scale, bias,
-                                                        static_cast<uint16_t*>(y), static_cast<int>(m), rows,
-                                                        cols);
+// splits > 1: the range sums added in range order (and each row's limbs,
+// smallest first), then scale, bias and one rounding; four outputs a thread.
+template <int OUT>
+__global__ __launch_bounds__(256) void combine_kernel(Args p) {
+  const int64_t quads = (p.N + 3) / 4, rows = p.xr / p.limbs;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= rows * quads) return;
+  const int64_t m = i / quads, n = 4 * (i - m * quads);
+  const bool full = (p.N & 3) == 0;
+  float sc[4], bi[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    sc[j] = n + j < p.N ? p.scale[n + j] : 0.0f;
+    bi[j] = n + j < p.N && p.bias ? p.bias[n + j] : 0.0f;
+  }
+  f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int l = p.limbs - 1; l >= 0; --l) {
+    f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = 0; s < p.splits; ++s) {
+      const float* d = p.partial + (static_cast<int64_t>(s) * p.xr + m * p.limbs + l) * p.N + n;
+      if (full) {
+        t += *reinterpret_cast<const f32x4*>(d);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (n + j < p.N) t[j] += d[j];
+      }
+    }
+    v = v + t;
+  }
+  const bool vec = full && (reinterpret_cast<uintptr_t>(p.y) & (OUT == QSTE_F32 ? 15 : 7)) == 0;
+  finish4<OUT>(p, m, n, v, sc, bi, vec);
 }
 
-template <int DT, int NBW>
-void launch_m(const void* x, const uint8_t* packed, const float* scale, const float* bias, void* y, int64_t m,
-              int64_t rows, int64_t cols, hipStream_t stream) {
-  if (m <= 1) launch<DT, NBW, 1>(x, packed, scale, bias, y, m, rows, cols, stream);
-  else if (m <= 2) launch<DT, NBW, 2>(x, packed, scale, bias, y, m, rows, cols, stream);
-  else if (m <= 4) launch<DT, NBW, 4>(x, packed, scale, bias, y, m, rows, cols, stream);
-  else if (m <= 8) launch<DT, NBW, 8>(x, packed, scale, bias, y, m, rows, cols, stream);
-  else launch<DT, NBW, 16>(x, packed, scale, bias, y, m, rows, cols, stream);
+template <int DT, int XR, int NBW>
+void launch(const Args& p, bool resident, hipStream_t stream) {
+  const int groups = static_cast<int>((p.N + 16 * NBW - 1) / (16 * NBW));
+  if constexpr (XR <= 16) {
+    if (resident) {
+      skinny_kernel<DT, XR, NBW, true><<<groups * p.splits, THREADS, 0, stream>>>(p);
+      return;
+    }
+  }
+  skinny_kernel<DT, XR, NBW, false><<<groups * p.splits, THREADS, 0, stream>>>(p);
+}
+
+// Weight blocks per workgroup at most: what the waves' accumulators and their
+// image in LDS at the end have room for.
+constexpr int most_blocks(int xr) { return xr <= 32 ? 8 : (xr <= 48 ? 6 : 4); }
+
+template <int DT, int XR, int NBW = 1>
+void launch_nbw(int nbw, const Args& p, bool resident, hipStream_t stream) {
+  if constexpr (NBW < most_blocks(XR)) {
+    if (nbw > NBW) return launch_nbw<DT, XR, NBW + 1>(nbw, p, resident, stream);
+  }
+  launch<DT, XR, NBW>(p, resident, stream);
 }
 
 template <int DT>
-void launch_dt(int64_t nbw, const void* x, const uint8_t* packed, const float* scale, const float* bias, void* y,
-               int64_t m, int64_t rows, int64_t cols, hipStream_t stream) {
-  switch (nbw) {
-    case 1: launch_m<DT, 1>(x, packed, scale, bias, y, m, rows, cols, stream); break;
-    case 2: launch_m<DT, 2>(x, packed, scale, bias, y, m, rows, cols, stream); break;
-    case 3: launch_m<DT, 3>(x, packed, scale, bias, y, m, rows, cols, stream); break;
-    case 4: launch_m<DT, 4>(x, packed, scale, bias, y, m, rows, cols, stream); break;
-    case 5: launch_m<DT, 5>(x, packed, scale, bias, y, m, rows, cols, stream); break;
-    case 6: launch_m<DT, 6>(x, packed, scale, bias, y, m, rows, cols, stream); break;
-    case 7: launch_m<DT, 7>(x, packed, scale, bias, y, m, rows, cols, stream); break;
-    default: launch_m<DT, 8>(x, packed, scale, bias, y, m, rows, cols, stream); break;
-  }
+void launch_xr(int nbw, const Args& p, bool resident, hipStream_t stream) {
+  if (p.xr <= 4) launch_nbw<DT, 4>(nbw, p, resident, stream);
+  else if (p.xr <= 16) launch_nbw<DT, 16>(nbw, p, resident, stream);
+  else if (p.xr <= 32) launch_nbw<DT, 32>(nbw, p, resident, stream);
+  else if (p.xr <= 48) launch_nbw<DT, 48>(nbw, p, resident, stream);
+  else launch_nbw<DT, 64>(nbw, p, resident, stream);
 }
+
+// Rows of x a launch takes: four tiles of 16, or 21 rows of three limbs.
+constexpr int64_t kRows16 = 64, kRows32 = 21;
+
+struct Plan {
+  int nbw, splits, chunks_per_split;
+};
+
+// Weight blocks per workgroup and ranges of K for xr rows of x.
+//
+// Blocks: the workgroups of one round over the 256 CUs as even as the most
+// blocks a workgroup can hold allows.  Ranges: with 1 to 2 blocks per
+// workgroup, forming fragments from x (0.087 us per chunk and tile of 16
+// rows: 192 VALU instructions) and x's reads from L2 (0.0085 us per chunk and
+// row) bound the kernel, not the weights; S ranges cut both S-fold, and cost
+// a second launch and the sums' round trip.  Measured, one range against the
+// best split: 8192 x 28672, M = 16: 19.9 / 17.9 us, M = 40: 40.6 / 31.9;
+// 4096 x 14336, M = 24: 14.4 / 13.0, M = 16: 9.8 / 10.4 (not split); three
+// blocks and more (14336 x 4096, M = 40: 11.8 / 20.8) are never split.
+Plan plan_of(int64_t xr, int64_t rows, int64_t cols, bool may_split) {
+  const int64_t blocks = (rows + 15) / 16, chunks = (cols + CHUNK_K - 1) / CHUNK_K;
+  const int64_t most = most_blocks(static_cast<int>(xr)), tiles = (xr + 15) / 16;
+  int64_t splits = 1, per = chunks;
+  if (may_split && blocks <= 2 * 256) {
+    double best = 0.0;
+    for (int64_t s = 2; s <= 4 && 2 * s <= chunks; s *= 2) {
+      const int64_t cps = (chunks + s - 1) / s, ns = (chunks + cps - 1) / cps;
+      if ((blocks * ns + 255) / 256 > most) continue;  // a second round
+      const double saved = static_cast<double>(chunks - cps) * (0.087 * tiles + 0.0085 * xr);
+      const double cost = 4.5 + static_cast<double>(ns * xr * rows) * 8.0 / 4e6;
+      if (saved - cost > best) {
+        best = saved - cost;
+        splits = ns;
+        per = cps;
+      }
+    }
+  }
+  const int64_t work = blocks * splits, rounds = (work + 256 * most - 1) / (256 * most);
+  int64_t nbw = (work + 256 * rounds - 1) / (256 * rounds);
+  return Plan{static_cast<int>(nbw < 1 ? 1 : nbw), static_cast<int>(splits), static_cast<int>(per)};
+}
+
+// Rows of 16-bit x that m rows make (three limbs for an fp32 row), 0 when
+// the product is not for this path.
+int64_t x_rows(int dtype, int64_t m, int64_t rows, int64_t cols) {
+  const int64_t most = dtype == QSTE_F32 ? kRows32 : kRows16;
+  if (m < 1 || m > most || rows < 1 || cols < 128 || cols % 128 != 0) return 0;
+  const int64_t xr = dtype == QSTE_F32 ? 3 * m : m;
+  // 32-bit buffer offsets, with room for the padded last block and the
+  // out-of-range marker
+  return (rows + 128) * (cols / 8) < (int64_t{1} << 31) && xr * cols * 2 < (int64_t{1} << 31) ? xr : 0;
+}
+
+template <int DT>
+int run(const Args& p, const Plan& plan, bool fp32, hipStream_t stream) {
+  // streaming blocks past resident fragments pays from three blocks on
+  // (28672 x 8192, M = 1: 10.3 against 12.7 us; 4096 x 4096, one block: 3.9
+  // both ways; 4096 x 14336: 7.7 against 7.2)
+  launch_xr<DT>(plan.nbw, p, plan.nbw >= 3, stream);
+  int rc = static_cast<int>(hipGetLastError());
+  if (rc || p.splits == 1) return rc;
+  const int64_t items = p.xr / p.limbs * ((p.N + 3) / 4);
+  const int grid = static_cast<int>((items + 255) / 256);
+  if (fp32) combine_kernel<QSTE_F32><<<grid, 256, 0, stream>>>(p);
+  else combine_kernel<DT><<<grid, 256, 0, stream>>>(p);
+  return static_cast<int>(hipGetLastError());
+}
+
+size_t up256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 }  // namespace gemv
 
-// Returns 1 when the call is not for this path.
-int gemv_linear_forward(const void* x, int dtype, const uint8_t* packed, const float* scale,
-                        const float* bias, void* y, int64_t m, int64_t rows, int64_t cols,
+int launch_limbs(const float*, int64_t, int64_t, uint16_t*, hipStream_t);
+
+// Workspace of a product on this path: fp32 x's limbs, and the range sums of
+// the plan (past 16 rows of two ranges at least, so that the size does not
+// depend on where the plan's line lies); 0 where none is needed or the
+// product is not for this path.
+size_t gemv_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
+  const int64_t xr = gemv::x_rows(dtype, m, rows, cols);
+  if (xr == 0) return 0;
+  const gemv::Plan plan = gemv::plan_of(xr, rows, cols, true);
+  int64_t ranges = plan.splits > 1 ? plan.splits : 0;
+  if (m > 16 && ranges < 2) ranges = 2;
+  return (dtype == QSTE_F32 ? gemv::up256(static_cast<size_t>(xr * cols) * 2) : 0) +
+         static_cast<size_t>(ranges * xr * rows) * sizeof(float);
+}
+
+// Returns 1 when the call is not for this path (fp32 needs its workspace; 16
+// bit runs in one range without one).
+int gemv_linear_forward(const void* x, int dtype, const uint8_t* packed, const float* scale, const float* bias,
+                        void* y, int64_t m, int64_t rows, int64_t cols, void* workspace, size_t workspace_bytes,
                         hipStream_t stream) {
-  if ((dtype != QSTE_BF16 && dtype != QSTE_F16) || m < 1 || m > 16 || rows < 1 || cols < 128 || cols % 128 != 0 ||
-      (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(packed) & 15))
+  const int64_t xr = gemv::x_rows(dtype, m, rows, cols);
+  const bool fp32 = dtype == QSTE_F32;
+  if (xr == 0 || (reinterpret_cast<uintptr_t>(x) & 15) ||
+      (reinterpret_cast<uintptr_t>(packed) & 15))
     return 1;
-  // 32-bit buffer offsets, with room for the padded last block and the
-  // out-of-range marker
-  const int64_t pb = cols / 8;
-  if ((rows + 128) * pb >= (int64_t{1} << 31) || m * cols * 2 >= (int64_t{1} << 31)) return 1;
-  // about one workgroup per CU: 16 * NBW rows each, NBW in 1..8
-  int64_t nbw = (rows + 16 * 256 - 1) / (16 * 256);
-  if (nbw < 1) nbw = 1;
-  if (nbw > 8) nbw = 8;
-  if (dtype == QSTE_F16)
-    gemv::launch_dt<QSTE_F16>(nbw, x, packed, scale, bias, y, m, rows, cols, stream);
-  else
-    gemv::launch_dt<QSTE_BF16>(nbw, x, packed, scale, bias, y, m, rows, cols, stream);
-  return static_cast<int>(hipGetLastError());
+  const bool room = workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+                    workspace_bytes >= gemv_forward_workspace(m, rows, cols, dtype);
+  if (fp32 && !room) return 1;
+  const gemv::Plan plan = gemv::plan_of(xr, rows, cols, room);
+  gemv::Args p{};
+  p.x = static_cast<const uint16_t*>(x);
+  p.bits = packed;
+  p.scale = scale;
+  p.bias = bias;
+  p.y = y;
+  p.xr = static_cast<int>(xr);
+  p.limbs = fp32 ? 3 : 1;
+  p.splits = plan.splits;
+  p.chunks_per_split = plan.chunks_per_split;
+  p.N = rows;
+  p.K = cols;
+  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  if (fp32) {
+    uint16_t* xl = reinterpret_cast<uint16_t*>(ws);
+    const int rc = launch_limbs(static_cast<const float*>(x), m, cols, xl, stream);
+    if (rc) return rc;
+    p.x = xl;
+    ws += gemv::up256(static_cast<size_t>(p.xr * cols) * 2);
+  }
+  p.partial = reinterpret_cast<float*>(ws);
+  return dtype == QSTE_F16 ? gemv::run<QSTE_F16>(p, plan, false, stream)
+                           : gemv::run<QSTE_BF16>(p, plan, fp32, stream);
 }
 
 }  // namespace qste

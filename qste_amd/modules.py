@@ -72,9 +72,8 @@ class PackedLinear(nn.Module):
     result back to the input dtype (modules.py:114-120).  Widening bf16/fp16
     to fp32 is exact, so the input goes to the kernel in its own dtype; the
     kernels multiply exact +-1 operands, accumulate in fp32 and round once to
-    the input dtype.  The decode kernel (bf16, at most 16 rows) accumulates a
-    biased operand and subtracts the bias, which costs a few of fp32's bits
-    relative to sum |x|: well below the output's bf16 rounding.
+    the input dtype.  The kernel for few rows (at most 64, 21 in fp32) selects
+    x or -x by the weight bit, exactly.
     """
 
     def __init__(self, packed: Tensor, scale: Tensor, columns: int, bias: Tensor | None):

@@ -1,0 +1,118 @@
+"""The skinny forward past 16 rows, in fp32, and over split ranges of K.
+
+Against the float64 oracle: every product is exact (x or -x), so the only
+errors are fp32 sums and one output rounding.  A sum of n terms in any order
+is within (n - 1) * 2^-24 * sum |x| of the exact one; the longest chain here
+is the MFMAs of a wave's chunks, the 8 waves, the ranges and the limbs, under
+K / 8 + 64 additions (an MFMA adds 32 columns, internally rounded at most
+that often).  fp32 outputs take scale and bias with two more roundings; 16-bit
+outputs one rounding to the dtype.
+
+Sizes sit where the kernel's layout can go wrong: row counts at the edges of
+its 4-, 16-, 32-, 48- and 64-row instances, K inside a 512-column chunk and
+over several chunks of a wave, N inside a block of 16 and of a workgroup,
+output rows whose start is not 16-byte aligned, one to eight blocks, and plans
+that split K (the C entry without a workspace runs the same call unsplit)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+HALF_ULP = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12, torch.float32: 2.0 ** -24}
+
+
+@pytest.fixture(autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+def _problem(rows, cols, m, dtype, seed):
+    rng = np.random.default_rng(seed)
+    packed = rng.integers(0, 256, size=(rows, cols // 8), dtype=np.uint8)
+    x = torch.from_numpy(rng.standard_normal((m, cols)).astype(np.float32)).to(dtype).float().numpy()
+    scale = (np.abs(rng.standard_normal(rows)) * 0.02 + 0.01).astype(np.float32)
+    bias = (rng.standard_normal(rows) * 0.1).astype(np.float32)
+    return packed, x, scale, bias
+
+
+def _check(got, x, packed, scale, bias, cols):
+    want = oracle.linear_fwd(x, packed, scale, bias, cols)
+    err = np.abs(got.double().cpu().numpy() - want)
+    mag = np.abs(x).astype(np.float64).sum(axis=1)[:, None] * scale.astype(np.float64)[None, :]
+    bound = (cols / 8 + 64) * 2.0 ** -24 * mag + 2.0 ** -23 * (np.abs(want) + np.abs(bias)[None, :])
+    if got.dtype != torch.float32:
+        bound = bound + 2 * HALF_ULP[got.dtype] * np.abs(want) + 1e-7
+    assert np.all(err <= bound), np.max(err / bound)
+
+
+SHAPES = [(300, 1024, 17), (4097, 896, 33), (129, 4224, 48), (1000, 8192, 49), (16, 128, 64), (9001, 640, 32),
+          (4096, 14336, 24), (1026, 5120, 40), (8200, 1152, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols,m", SHAPES)
+def test_rows_past_sixteen(rows, cols, m, dtype):
+    from qste_amd import kernels
+
+    print(f"skinny {rows}x{cols} m={m} {dtype}", flush=True)
+    packed, x, scale, bias = _problem(rows, cols, m, dtype, rows + cols + m)
+    tx, tp = torch.from_numpy(x).to(DEV, dtype), torch.from_numpy(packed).to(DEV)
+    ts, tb = torch.from_numpy(scale).to(DEV), torch.from_numpy(bias).to(DEV)
+    _check(kernels.packed_linear_affine(tx, tp, ts, tb, cols), x, packed, scale, bias, cols)
+    plain = torch.empty(m, rows, dtype=dtype, device=DEV)
+    rc = kernels._lib.load().qste_packed_linear_affine(
+        tx.data_ptr(), CODE[dtype], tp.data_ptr(), ts.data_ptr(), tb.data_ptr(), plain.data_ptr(), m, rows, cols,
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    _check(plain, x, packed, scale, bias, cols)
+
+
+@pytest.mark.parametrize("rows,cols,m", [(300, 1024, 1), (17, 384, 2), (2048, 2048, 5), (129, 4224, 6), (1, 640, 16),
+                                         (4097, 896, 21), (1000, 8192, 11), (8192, 16384, 4)])
+def test_fp32_rows(rows, cols, m):
+    """fp32 x as three limbs; one row holds an infinity, whose outputs are
+    infinities after the weights' signs."""
+
+    from qste_amd import kernels
+
+    packed, x, scale, bias = _problem(rows, cols, m, torch.float32, rows + cols + m)
+    tp, ts, tb = torch.from_numpy(packed).to(DEV), torch.from_numpy(scale).to(DEV), torch.from_numpy(bias).to(DEV)
+    got = kernels.packed_linear_affine(torch.from_numpy(x).to(DEV), tp, ts, tb, cols)
+    _check(got, x, packed, scale, bias, cols)
+    x[m - 1, cols - 3] = np.inf
+    got = kernels.packed_linear_affine(torch.from_numpy(x).to(DEV), tp, ts, tb, cols).cpu().numpy()
+    bit = (packed[:, (cols - 3) // 8] >> ((cols - 3) % 8)) & 1
+    assert np.array_equal(got[m - 1], np.where(bit == 1, np.inf, -np.inf).astype(np.float32))
+    if m > 1:
+        _check(torch.from_numpy(got[:m - 1]), x[:m - 1], packed, scale, bias, cols)
+
+
+@pytest.mark.parametrize("rows,cols,m", [(8192, 28672, 16), (1000, 8192, 64), (4096, 14336, 24)])
+def test_split_plans_are_deterministic(rows, cols, m):
+    """Shapes whose plan splits K: two calls agree bit for bit, and with the
+    unsplit call up to fp32 summation order (at most one ulp, on few)."""
+
+    from qste_amd import kernels
+
+    g = torch.Generator(device=DEV).manual_seed(m)
+    tp = torch.randint(0, 256, (rows, cols // 8), generator=g, device=DEV, dtype=torch.uint8)
+    ts = torch.rand(rows, generator=g, device=DEV) * 0.02 + 0.01
+    tx = torch.randn(m, cols, generator=g, device=DEV).to(torch.bfloat16)
+    a = kernels.packed_linear_affine(tx, tp, ts, None, cols)
+    assert torch.equal(a, kernels.packed_linear_affine(tx, tp, ts, None, cols))
+    plain = torch.empty_like(a)
+    assert kernels._lib.load().qste_packed_linear_affine(
+        tx.data_ptr(), 2, tp.data_ptr(), ts.data_ptr(), None, plain.data_ptr(), m, rows, cols,
+        torch.cuda.current_stream().cuda_stream) == 0
+    a, plain = a.float(), plain.float()
+    assert (a != plain).float().mean() < 0.01
+    assert torch.all((a - plain).abs() <= plain.abs() * 2.0 ** -7 + 1e-6)
