@@ -37,18 +37,22 @@ int mfma_linear_forward(const void*, int, const uint8_t*, const float*, const fl
                         int64_t, int64_t, hipStream_t);
 int mfma_linear_dgrad(const void*, int, const uint8_t*, const float*, void*, int64_t, int64_t, int64_t,
                       hipStream_t);
-int mfma_linear_dgrad_t(const void*, int, const uint8_t*, int64_t, const uint16_t*, void*, int64_t, int64_t,
+int mfma_linear_dgrad_t(const void*, int64_t, int, const uint8_t*, int64_t, const uint16_t*, void*, int64_t, int64_t,
                         int64_t, hipStream_t);
 int mfma_evidence(const void*, int, const uint8_t*, const float*, float*, int64_t, int64_t, int64_t,
                   const float*, const float*, const uint8_t*, float*, const EvidencePlan*, float*, hipStream_t);
-int mfma_evidence_t(const void*, int, const uint8_t*, int64_t, const uint16_t*, float*, int64_t, int64_t, int64_t,
-                    const float*, const float*, const uint8_t*, float*, const EvidencePlan*, float*, hipStream_t);
+int mfma_evidence_t(const void*, int64_t, int, const uint8_t*, int64_t, const uint16_t*, float*, int64_t, int64_t,
+                    int64_t, const float*, const float*, const uint8_t*, int64_t, float*, const EvidencePlan*, float*,
+                    hipStream_t);
 int64_t mfma_evidence_tiles(int64_t cols);
-bool mfma_pair_ok(const void*, int, int64_t, int64_t, int64_t);
+bool mfma_backward_ok(const void*, int64_t, int, int64_t, int64_t, int64_t);
 EvidencePlan mfma_evidence_plan(int64_t, int64_t, int64_t, bool);
-int mfma_backward_pair(const void*, int, const uint8_t*, int64_t, const uint16_t*, float*, const uint8_t*, int64_t,
-                       const uint16_t*, const uint8_t*, void*, int64_t, int64_t, int64_t, const float*,
-                       const float*, float*, const EvidencePlan&, float*, hipStream_t);
+int mfma_backward_pair(const void*, int64_t, int, const uint8_t*, int64_t, const uint16_t*, float*, const uint8_t*,
+                       int64_t, const uint16_t*, const uint8_t*, int64_t, void*, int64_t, int64_t, int64_t,
+                       const float*, const float*, float*, const EvidencePlan&, float*, hipStream_t);
+int launch_pad_rows(const void*, void*, int64_t, int64_t, int64_t, hipStream_t);
+int launch_colsums_pad(const void*, int, const float*, int64_t, int64_t, int64_t, uint16_t*, float*, float*, float*,
+                       float*, hipStream_t);
 int launch_transpose_bits(const uint8_t*, uint8_t*, int64_t, int64_t, int64_t, int64_t, hipStream_t);
 int launch_f32_to_16(const float*, uint16_t*, int64_t, int64_t, int, hipStream_t);
 size_t gemv_forward_workspace(int64_t, int64_t, int64_t, int);
@@ -86,15 +90,39 @@ inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 inline bool dtype_ok(int d) { return d == QSTE_F32 || d == QSTE_F16 || d == QSTE_BF16; }
 inline size_t align_up(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
+inline int64_t up64(int64_t v) { return (v + 63) / 64 * 64; }
+
+// A 16-bit layer whose rows or columns are no multiple of 64 runs its backward
+// on the matrix cores too, from zero-padded copies (of dy where rows are
+// ragged, of the weight signs where columns are), once the products are worth
+// the copies' launches.  Measured, scalar kernels / matrix cores, in us: 64
+// samples of 300 x 300 (2^22.5 multiply-adds) 78 / 74, 64 of 300 x 130
+// (2^21.3) 75 / about the same, 256 of 300 x 300 120 / 78, 512 of 1000 x 1000
+// 245 / 80, 2048 of 1000 x 3000 698 / 110.
+constexpr int64_t kRaggedWork = int64_t{1} << 22;
+bool ragged_backward(int dtype, int64_t samples, int64_t rows, int64_t cols) {
+  return (dtype == QSTE_BF16 || dtype == QSTE_F16) && (rows % 64 != 0 || cols % 64 != 0) && samples > 0 && rows > 0 &&
+         cols > 0 && static_cast<double>(samples) * rows * cols >= static_cast<double>(kRaggedWork) &&
+         static_cast<double>(samples) * up64(rows) * 2 < 4294967296.0;
+}
+
 struct BackwardLayout {
-  size_t v_part, db_part, v, gs_part, w_t, x_t, s16, xs16, partial, limbs, limb_bytes, total;
+  size_t v_part, db_part, v, gs_part, w_t, x_t, s16, xs16, partial, limbs, limb_bytes, dy_pad, w_pad, total;
   int64_t chunks, tiles;
   int64_t w_t_pitch, x_t_pitch;  // bytes per row of the transposed sign copies
 };
 
-// with_limbs: room for fp32 dy's bf16 limbs (the dX and evidence products
-// take turns in it)
-BackwardLayout backward_layout(int64_t samples, int64_t rows, int64_t cols, bool with_limbs = false) {
+// What the workspace has room for besides the scalar kernels' needs: fp32
+// dy's bf16 limbs (the dX and evidence products take turns in them), or the
+// padded copies of a ragged 16-bit layer.
+enum LayoutKind { LAYOUT_PLAIN, LAYOUT_LIMBS, LAYOUT_RAGGED };
+
+LayoutKind layout_kind(int dtype, int64_t samples, int64_t rows, int64_t cols) {
+  if (dtype == QSTE_F32) return LAYOUT_LIMBS;
+  return ragged_backward(dtype, samples, rows, cols) ? LAYOUT_RAGGED : LAYOUT_PLAIN;
+}
+
+BackwardLayout backward_layout(int64_t samples, int64_t rows, int64_t cols, LayoutKind kind = LAYOUT_PLAIN) {
   BackwardLayout l{};
   l.chunks = colsum_chunks(samples);
   int64_t tiles = simt_evidence_tiles(cols);
@@ -102,8 +130,9 @@ BackwardLayout backward_layout(int64_t samples, int64_t rows, int64_t cols, bool
   if (mt > tiles) tiles = mt;
   l.tiles = tiles;
   size_t at = 0;
-  l.v_part = at; at += align_up(sizeof(float) * static_cast<size_t>((l.chunks > 0 ? l.chunks : 1) * rows));
-  l.db_part = at; at += align_up(sizeof(float) * static_cast<size_t>((l.chunks > 0 ? l.chunks : 1) * rows));
+  const int64_t part_rows = (l.chunks > 0 ? l.chunks : 1) * (kind == LAYOUT_RAGGED ? up64(rows) : rows);
+  l.v_part = at; at += align_up(sizeof(float) * static_cast<size_t>(part_rows));
+  l.db_part = at; at += align_up(sizeof(float) * static_cast<size_t>(part_rows));
   l.v = at; at += align_up(sizeof(float) * static_cast<size_t>(rows));
   l.gs_part = at; at += align_up(sizeof(float) * static_cast<size_t>(tiles * rows));
   // transposed signs (bits along K, rows padded to 64-bit words) and bf16
@@ -121,11 +150,16 @@ BackwardLayout backward_layout(int64_t samples, int64_t rows, int64_t cols, bool
   if (alone > partial) partial = alone;
   l.partial = at; at += align_up(static_cast<size_t>(partial));
   l.limb_bytes = 0;
-  if (with_limbs) {
+  if (kind == LAYOUT_LIMBS) {
     const size_t d = f32_dgrad_workspace(samples, rows, cols), e = f32_evidence_workspace(samples, rows, cols);
     l.limb_bytes = d > e ? d : e;
   }
   l.limbs = at; at += align_up(l.limb_bytes);
+  l.dy_pad = at;
+  if (kind == LAYOUT_RAGGED && rows % 64 != 0) at += align_up(sizeof(uint16_t) * static_cast<size_t>(samples * up64(rows)));
+  l.w_pad = at;
+  // (padded to 128 columns: the copy writes 16 bytes at a time)
+  if (kind == LAYOUT_RAGGED && cols % 64 != 0) at += align_up(static_cast<size_t>(rows * ((cols + 127) / 128 * 16)));
   l.total = at;
   return l;
 }
@@ -229,9 +263,35 @@ int qste_packed_linear_affine(const void* x, int dtype, const uint8_t* packed, c
   return forward_dispatch(x, dtype, packed, scale, bias, y, m, rows, cols, as_stream(stream));
 }
 
-size_t qste_packed_linear_affine_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int dtype) {
+namespace {
+
+// A 16-bit forward whose columns no matrix path takes (a multiple of 64; of
+// 128 up to 64 rows) runs it on copies of x and the signs that are padded
+// with zeros (a zero x times either sign adds nothing).  The scalar kernel's
+// time is its K chain, about 2.3 us per 16 columns; the copies and the product
+// take 9-13 us up to 64 rows (64 x 300 x 130: 23.5 -> 12.3, 32 x 65 x 65: 14.2
+// -> 9.4) and 24-29 us on 256-row tiles (128 x 300 x 300: 45 -> 24, 2048 x 1000
+// x 3000: 503 -> 46, but 1000 x 130 x 130: 24 / 26): hence the two lines.
+int64_t padded_forward_cols(int64_t m, int64_t rows, int64_t cols, int dtype) {
+  if ((dtype != QSTE_BF16 && dtype != QSTE_F16) || m <= 0 || rows <= 0 || cols <= (m <= 64 ? 64 : 160))
+    return 0;
+  const int64_t unit = m <= 64 ? 128 : 64;
+  // the copies are rows of whole 16-byte words of signs
+  return cols % unit == 0 ? 0 : (cols + 127) / 128 * 128;
+}
+
+size_t plain_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
   if (const size_t skinny = gemv_forward_workspace(m, rows, cols, dtype)) return skinny;
   return dtype == QSTE_F32 ? f32_forward_workspace(m, rows, cols) : mfma_forward_split_workspace(m, rows, cols, dtype);
+}
+
+}  // namespace
+
+size_t qste_packed_linear_affine_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int dtype) {
+  if (const int64_t pc = padded_forward_cols(m, rows, cols, dtype))
+    return align_up(static_cast<size_t>(m * pc) * 2) + align_up(static_cast<size_t>(rows * pc / 8)) +
+           plain_forward_workspace(m, rows, pc, dtype);
+  return plain_forward_workspace(m, rows, cols, dtype);
 }
 
 int qste_packed_linear_affine_ws(const void* x, int dtype, const uint8_t* packed, const float* scale,
@@ -241,6 +301,19 @@ int qste_packed_linear_affine_ws(const void* x, int dtype, const uint8_t* packed
   if (m < 0 || rows < 0 || cols < 0) return QSTE_E_SHAPE;
   if (m * rows == 0) return 0;
   if (!y || !scale || (cols > 0 && (!x || !packed))) return QSTE_E_NULL;
+  const int64_t pc = padded_forward_cols(m, rows, cols, dtype);
+  if (pc && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+      workspace_bytes >= qste_packed_linear_affine_workspace_bytes(m, rows, cols, dtype)) {
+    hipStream_t s = as_stream(stream);
+    const size_t xb = align_up(static_cast<size_t>(m * pc) * 2), wb = align_up(static_cast<size_t>(rows * pc / 8));
+    char* xp = static_cast<char*>(workspace);
+    char* wp = xp + xb;
+    int rc = launch_pad_rows(x, xp, m, 2 * cols, 2 * pc, s);
+    if (rc) return rc;
+    if ((rc = launch_pad_rows(packed, wp, rows, (cols + 7) / 8, pc / 8, s))) return rc;
+    return qste_packed_linear_affine_ws(xp, dtype, reinterpret_cast<uint8_t*>(wp), scale, bias, y, m, rows, pc,
+                                        wp + wb, workspace_bytes - xb - wb, stream);
+  }
   if (cols > 0) {
     const int rc = gemv_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, workspace, workspace_bytes,
                                        as_stream(stream));
@@ -329,12 +402,12 @@ int qste_packed_row_inner(const float* matrix, const uint8_t* packed, float* out
 
 size_t qste_linear_backward_workspace_bytes(int64_t samples, int64_t rows, int64_t cols) {
   if (samples < 0 || rows < 0 || cols < 0) return 0;
-  return backward_layout(samples, rows, cols).total;
+  return backward_layout(samples, rows, cols, layout_kind(QSTE_BF16, samples, rows, cols)).total;
 }
 
 size_t qste_linear_backward_workspace_bytes_dtype(int64_t samples, int64_t rows, int64_t cols, int dtype) {
   if (samples < 0 || rows < 0 || cols < 0) return 0;
-  return backward_layout(samples, rows, cols, dtype == QSTE_F32).total;
+  return backward_layout(samples, rows, cols, layout_kind(dtype, samples, rows, cols)).total;
 }
 
 namespace {
@@ -350,11 +423,12 @@ int linear_backward_impl(const void* dy, int dtype, const uint8_t* packed_x, con
   if (samples < 0 || rows <= 0 || cols <= 0) return QSTE_E_SHAPE;
   if (!evidence || !grad_scale || !scale || !packed_w) return QSTE_E_NULL;
   if (samples > 0 && (!dy || !packed_x || !x_offset || !x_scale)) return QSTE_E_NULL;
-  // fp32 takes its products through bf16 limbs when the workspace has room
-  // for them (qste_linear_backward_workspace_bytes_dtype), the SIMT kernels
-  // otherwise
-  BackwardLayout l = backward_layout(samples, rows, cols, dtype == QSTE_F32);
-  if (workspace_bytes < l.total) l = backward_layout(samples, rows, cols);
+  // fp32 takes its products through bf16 limbs and ragged 16-bit layers
+  // theirs through padded copies when the workspace has room for them
+  // (qste_linear_backward_workspace_bytes_dtype), the SIMT kernels otherwise
+  LayoutKind kind = layout_kind(dtype, samples, rows, cols);
+  BackwardLayout l = backward_layout(samples, rows, cols, kind);
+  if (workspace_bytes < l.total) l = backward_layout(samples, rows, cols, kind = LAYOUT_PLAIN);
   if (!workspace || workspace_bytes < l.total) return QSTE_E_WORKSPACE;
   hipStream_t s = as_stream(stream);
   char* base = static_cast<char*>(workspace);
@@ -364,60 +438,71 @@ int linear_backward_impl(const void* dy, int dtype, const uint8_t* packed_x, con
   float* gs_part = reinterpret_cast<float*>(base + l.gs_part);
   int rc;
   if (samples > 0) {
+    // rows of dy the matrix products read: dy itself, or its padded copy
+    const bool ragged = kind == LAYOUT_RAGGED;
+    const bool pad_dy = ragged && rows % 64 != 0;
+    const void* dy_m = pad_dy ? static_cast<const void*>(base + l.dy_pad) : dy;
+    const int64_t ldy = pad_dy ? up64(rows) : rows;
+    const bool matrix = (ragged || (rows % 64 == 0 && cols % 64 == 0)) &&
+                        mfma_backward_ok(dy_m, ldy, dtype, samples, rows, cols);
     // the offset correction's column sums, unless the caller brings them
     // (with a bias gradient to form, dy is read for both anyway)
-    if (offset_dot && !grad_bias) {
-      v = const_cast<float*>(offset_dot);  // only read from here on
+    if (matrix && pad_dy) {
+      if ((rc = launch_colsums_pad(dy, dtype, x_offset, samples, rows, ldy, reinterpret_cast<uint16_t*>(base + l.dy_pad),
+                                   v_part, grad_bias ? db_part : nullptr, v, grad_bias, s)))
+        return rc;
+      if (offset_dot && !grad_bias) v = const_cast<float*>(offset_dot);  // only read from here on
+    } else if (offset_dot && !grad_bias) {
+      v = const_cast<float*>(offset_dot);
     } else if ((rc = launch_colsums(dy, dtype, x_offset, samples, rows, v_part, grad_bias ? db_part : nullptr, v,
                                     grad_bias, s))) {
       return rc;
     }
-    // MFMA path: the plan runs evidence and dgrad in one launch (from
-    // transposed copies of the signs and bf16 copies of the scales) or as
-    // two, and splits evidence tiles over K where that shortens the work
+    // MFMA path: the plan runs evidence and dgrad in one launch or as two,
+    // and splits evidence tiles over K where that shortens the work.  Both
+    // read transposed copies of the signs (bits along K) and 16-bit copies
+    // of the scales
     bool dgrad_done = false;
-    if (mfma_pair_ok(dy, dtype, samples, rows, cols)) {
+    if (matrix) {
       const EvidencePlan plan = mfma_evidence_plan(samples, rows, cols, dx != nullptr);
       float* partial = reinterpret_cast<float*>(base + l.partial);
       uint8_t* w_t = reinterpret_cast<uint8_t*>(base + l.w_t);
+      uint8_t* x_t = reinterpret_cast<uint8_t*>(base + l.x_t);
       uint16_t* s16 = reinterpret_cast<uint16_t*>(base + l.s16);
+      uint16_t* xs16 = reinterpret_cast<uint16_t*>(base + l.xs16);
       const int64_t pb = (cols + 7) / 8;
-      if (plan.pair) {
-        uint8_t* x_t = reinterpret_cast<uint8_t*>(base + l.x_t);
-        uint16_t* xs16 = reinterpret_cast<uint16_t*>(base + l.xs16);
+      // the evidence epilogue reads the signs of W in whole dwords
+      const uint8_t* w_epi = packed_w;
+      int64_t w_epi_pb = pb;
+      if (cols % 64 != 0) {
+        w_epi = reinterpret_cast<const uint8_t*>(base + l.w_pad);
+        w_epi_pb = (cols + 127) / 128 * 16;
+        if ((rc = launch_pad_rows(packed_w, base + l.w_pad, rows, pb, w_epi_pb, s))) return rc;
+      }
+      if (dx) {
         if ((rc = launch_transpose_bits(packed_w, w_t, rows, cols, pb, l.w_t_pitch, s))) return rc;
+        if ((rc = launch_f32_to_16(scale, s16, rows, up64(rows), dtype, s))) return rc;
+      }
+      if (plan.pair) {
         if ((rc = launch_transpose_bits(packed_x, x_t, samples, cols, pb, l.x_t_pitch, s))) return rc;
-        if ((rc = launch_f32_to_16(scale, s16, rows, (rows + 63) / 64 * 64, dtype, s))) return rc;
-        if ((rc = launch_f32_to_16(x_scale, xs16, samples, (samples + 63) / 64 * 64, dtype, s))) return rc;
-        rc = mfma_backward_pair(dy, dtype, x_t, l.x_t_pitch, xs16, evidence, w_t, l.w_t_pitch, s16, packed_w, dx,
-                                samples, rows, cols, v, scale, gs_part, plan, partial, s);
+        if ((rc = launch_f32_to_16(x_scale, xs16, samples, up64(samples), dtype, s))) return rc;
+        rc = mfma_backward_pair(dy_m, ldy, dtype, x_t, l.x_t_pitch, xs16, evidence, w_t, l.w_t_pitch, s16, w_epi,
+                                w_epi_pb, dx, samples, rows, cols, v, scale, gs_part, plan, partial, s);
         if (rc == 0) return launch_sum_partials(gs_part, mfma_evidence_tiles(cols), rows, grad_scale, s);
         if (rc != 1) return rc;
       } else {
         if (dx) {
-          // dgrad from transposed signs (bits along K, bf16 scales)
-          if ((rc = launch_transpose_bits(packed_w, w_t, rows, cols, pb, l.w_t_pitch, s))) return rc;
-          if ((rc = launch_f32_to_16(scale, s16, rows, (rows + 63) / 64 * 64, dtype, s))) return rc;
-          rc = mfma_linear_dgrad_t(dy, dtype, w_t, l.w_t_pitch, s16, dx, samples, rows, cols, s);
+          rc = mfma_linear_dgrad_t(dy_m, ldy, dtype, w_t, l.w_t_pitch, s16, dx, samples, rows, cols, s);
           if (rc == 1) rc = dgrad_dispatch(dy, dtype, packed_w, scale, dx, samples, rows, cols, s);
           if (rc) return rc;
         }
         dgrad_done = true;
-        // the evidence from a transposed copy of x's signs (bits along K,
-        // bf16 scales), as the pair reads them
-        uint8_t* x_t = reinterpret_cast<uint8_t*>(base + l.x_t);
-        uint16_t* xs16 = reinterpret_cast<uint16_t*>(base + l.xs16);
         if ((rc = launch_transpose_bits(packed_x, x_t, samples, cols, pb, l.x_t_pitch, s))) return rc;
-        if ((rc = launch_f32_to_16(x_scale, xs16, samples, (samples + 63) / 64 * 64, dtype, s))) return rc;
-        rc = mfma_evidence_t(dy, dtype, x_t, l.x_t_pitch, xs16, evidence, samples, rows, cols, v, scale, packed_w,
-                             gs_part, &plan, partial, s);
+        if ((rc = launch_f32_to_16(x_scale, xs16, samples, up64(samples), dtype, s))) return rc;
+        rc = mfma_evidence_t(dy_m, ldy, dtype, x_t, l.x_t_pitch, xs16, evidence, samples, rows, cols, v, scale, w_epi,
+                             w_epi_pb, gs_part, &plan, partial, s);
         if (rc == 0) return launch_sum_partials(gs_part, mfma_evidence_tiles(cols), rows, grad_scale, s);
         if (rc != 1) return rc;
-        int64_t tiles = 0;
-        if ((rc = evidence_dispatch(dy, dtype, packed_x, x_scale, evidence, samples, rows, cols, v, scale,
-                                    packed_w, gs_part, &plan, partial, &tiles, s)))
-          return rc;
-        return launch_sum_partials(gs_part, tiles, rows, grad_scale, s);
       }
     }
     if (dtype == QSTE_F32 && l.limb_bytes > 0) {

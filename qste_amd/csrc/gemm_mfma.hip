@@ -855,8 +855,8 @@ __global__ __launch_bounds__(THREADS, 1) void backward_pair_kernel(Params pe, Pa
 // summed in range order + m_add[m]; E = E0 * m_scale[m]; and the
 // scale-gradient partials sum_c E0 * sign_w over each 64-column slot, in
 // the slots the fused epilogue writes ([WAVES_N * tiles_n][M]).  One wave
-// per tile row (4 columns per lane, 16-byte accesses; N % 64 == 0 on this
-// path), a 16-lane group per slot; workgroups of 4 rows x split tiles.
+// per tile row (4 columns per lane, 16-byte accesses where N allows them), a
+// 16-lane group per slot; workgroups of 4 rows x split tiles.
 __global__ __launch_bounds__(THREADS) void evidence_combine_kernel(Split sp, const float* __restrict__ m_add,
                                                                    const float* __restrict__ m_scale,
                                                                    const uint8_t* __restrict__ w_bits, int64_t w_pb,
@@ -883,11 +883,19 @@ __global__ __launch_bounds__(THREADS) void evidence_combine_kernel(Split sp, con
     }
     const float add = m_add ? m_add[row] : 0.0f, mul = m_scale ? m_scale[row] : 1.0f;
     const float e0[4] = {acc.x + add, acc.y + add, acc.z + add, acc.w + add};
-    *reinterpret_cast<float4*>(ev + row * N + col) = make_float4(e0[0] * mul, e0[1] * mul, e0[2] * mul, e0[3] * mul);
+    if ((N & 3) == 0) {
+      *reinterpret_cast<float4*>(ev + row * N + col) =
+          make_float4(e0[0] * mul, e0[1] * mul, e0[2] * mul, e0[3] * mul);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (col + q < N) ev[row * N + col + q] = e0[q] * mul;
+    }
     if (w_bits) {
       const uint32_t nib = (w_bits[row * w_pb + (col >> 3)] >> (col & 7)) & 0xFu;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) signed_e0 += ((nib >> q) & 1u) ? e0[q] : -e0[q];
+      for (int q = 0; q < 4; ++q)
+        if (col + q < N) signed_e0 += ((nib >> q) & 1u) ? e0[q] : -e0[q];
     }
   }
 #pragma unroll
@@ -984,6 +992,15 @@ static bool evidence_ok(const void* dy, int dtype, const uint8_t* packed_x, int6
          aligned16(dy) && aligned16(packed_x) && fits32(samples * rows * 2) && fits32(samples * cols / 8);
 }
 
+// A layer's backward from transposed sign copies: dy rows `ldy` apart (rows
+// rounded up to 64, zero behind the data, so K steps end on zeros), any
+// rows and cols.
+static bool backward_operands_ok(const void* dy, int64_t ldy, int dtype, const uint8_t* bits_t, int64_t t_pitch,
+                                 int64_t samples, int64_t rows, int64_t cols) {
+  return mfma_dtype(dtype) && ldy % 64 == 0 && ldy >= rows && rows > 0 && cols > 0 && samples > 0 && aligned16(dy) &&
+         aligned16(bits_t) && fits32(samples * ldy * 2) && fits32(cols * t_pitch);
+}
+
 static mfma::Params dgrad_params(const void* dy, const uint8_t* packed, const float* row_scale, void* dx,
                                  int64_t m, int64_t rows, int64_t cols) {
   mfma::Params p{};
@@ -1014,10 +1031,10 @@ static mfma::Params evidence_params(const void* dy, const uint8_t* packed_x, con
 
 // The combine pass of a split evidence: workgroups of 4 tile rows x split tiles.
 static int launch_combine(const mfma::wide::Split& sp, const float* m_add, const float* m_scale,
-                          const uint8_t* w_bits, float* ev, float* gs_partial, int64_t rows, int64_t cols,
-                          hipStream_t stream) {
+                          const uint8_t* w_bits, int64_t w_pb, float* ev, float* gs_partial, int64_t rows,
+                          int64_t cols, hipStream_t stream) {
   const dim3 grid(mfma::wide::BM / (mfma::wide::THREADS / kWave), static_cast<unsigned>(sp.tiles_e - sp.tiles_full));
-  mfma::wide::evidence_combine_kernel<<<grid, mfma::wide::THREADS, 0, stream>>>(sp, m_add, m_scale, w_bits, cols / 8,
+  mfma::wide::evidence_combine_kernel<<<grid, mfma::wide::THREADS, 0, stream>>>(sp, m_add, m_scale, w_bits, w_pb,
                                                                                ev, gs_partial, rows, cols);
   return static_cast<int>(hipGetLastError());
 }
@@ -1128,16 +1145,17 @@ int mfma_linear_dgrad(const void* dy, int dtype, const uint8_t* packed, const fl
 // forward.  Measured 6-10% faster than bits along N at config 4's shapes;
 // the results are identical (the same bf16 operand values, the same
 // accumulation order).
-int mfma_linear_dgrad_t(const void* dy, int dtype, const uint8_t* w_t, int64_t w_t_pitch, const uint16_t* scale16,
-                        void* dx, int64_t m, int64_t rows, int64_t cols, hipStream_t stream) {
-  if (!dgrad_ok(dy, dtype, w_t, m, rows, cols) || !fits32(cols * w_t_pitch) || !aligned16(w_t)) return 1;
+int mfma_linear_dgrad_t(const void* dy, int64_t ldy, int dtype, const uint8_t* w_t, int64_t w_t_pitch,
+                        const uint16_t* scale16, void* dx, int64_t m, int64_t rows, int64_t cols,
+                        hipStream_t stream) {
+  if (!backward_operands_ok(dy, ldy, dtype, w_t, w_t_pitch, m, rows, cols)) return 1;
   mfma::Params p{};
   p.a = static_cast<const uint16_t*>(dy);
   p.bits = w_t;
   p.kscale16 = scale16;
   p.out = dx;
-  p.M = m; p.N = cols; p.K = rows;
-  p.lda = rows; p.pb = w_t_pitch;
+  p.M = m; p.N = cols; p.K = ldy;
+  p.lda = ldy; p.pb = w_t_pitch;
   p.a_rows = m; p.bit_rows = cols;
   if (dtype == QSTE_F16)
     mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K_SCALED, mfma::EPI_PLAIN, QSTE_F16>
@@ -1168,7 +1186,7 @@ int mfma_evidence(const void* dy, int dtype, const uint8_t* packed_x, const floa
       mfma::wide::evidence_split_kernel<mfma::B_BITS_ALONG_N, QSTE_BF16><<<grid, mfma::wide::THREADS, 0, stream>>>(p, sp);
     int rc = static_cast<int>(hipGetLastError());
     if (rc) return rc;
-    return launch_combine(sp, m_add, m_scale, w_bits, ev, gs_partial, rows, cols, stream);
+    return launch_combine(sp, m_add, m_scale, w_bits, cols / 8, ev, gs_partial, rows, cols, stream);
   }
   if (dtype == QSTE_F16)
     mfma::wide::wide_kernel<mfma::A_ROWS_K, mfma::B_BITS_ALONG_N, mfma::EPI_EVIDENCE, QSTE_F16>
@@ -1187,20 +1205,20 @@ int mfma_evidence(const void* dy, int dtype, const uint8_t* packed_x, const floa
 // values and K order as mfma_evidence: the results are identical.  Measured
 // ~2% faster than bits along N at config 4's gate and up evidence, the
 // transposes included.
-int mfma_evidence_t(const void* dy, int dtype, const uint8_t* x_t, int64_t x_t_pitch, const uint16_t* x_scale16,
-                    float* ev, int64_t samples, int64_t rows, int64_t cols, const float* m_add, const float* m_scale,
-                    const uint8_t* w_bits, float* gs_partial, const EvidencePlan* plan, float* partial,
-                    hipStream_t stream) {
-  if (!evidence_ok(dy, dtype, x_t, samples, rows, cols) || !fits32(cols * x_t_pitch) || !aligned16(x_t)) return 1;
+int mfma_evidence_t(const void* dy, int64_t ldy, int dtype, const uint8_t* x_t, int64_t x_t_pitch,
+                    const uint16_t* x_scale16, float* ev, int64_t samples, int64_t rows, int64_t cols,
+                    const float* m_add, const float* m_scale, const uint8_t* w_bits, int64_t w_pb, float* gs_partial,
+                    const EvidencePlan* plan, float* partial, hipStream_t stream) {
+  if (!backward_operands_ok(dy, ldy, dtype, x_t, x_t_pitch, samples, rows, cols)) return 1;
   mfma::Params p{};
   p.a = static_cast<const uint16_t*>(dy);
   p.bits = x_t;
   p.kscale16 = x_scale16;
   p.out = ev;
   p.M = rows; p.N = cols; p.K = samples;
-  p.lda = rows; p.pb = x_t_pitch;
+  p.lda = ldy; p.pb = x_t_pitch;
   p.a_rows = samples; p.bit_rows = cols;
-  p.m_add = m_add; p.m_scale = m_scale; p.w_bits = w_bits; p.w_pb = cols / 8; p.gs_partial = gs_partial;
+  p.m_add = m_add; p.m_scale = m_scale; p.w_bits = w_bits; p.w_pb = w_pb; p.gs_partial = gs_partial;
   const int te = wide_grid(rows, cols);
   if (plan && plan->splits > 1 && aligned16(ev)) {  // the combine pass stores 16 bytes at a time
     if (!partial) return QSTE_E_WORKSPACE;
@@ -1214,7 +1232,7 @@ int mfma_evidence_t(const void* dy, int dtype, const uint8_t* x_t, int64_t x_t_p
           <<<grid, mfma::wide::THREADS, 0, stream>>>(p, sp);
     int rc = static_cast<int>(hipGetLastError());
     if (rc) return rc;
-    return launch_combine(sp, m_add, m_scale, w_bits, ev, gs_partial, rows, cols, stream);
+    return launch_combine(sp, m_add, m_scale, w_bits, w_pb, ev, gs_partial, rows, cols, stream);
   }
   if (dtype == QSTE_F16)
     mfma::wide::wide_kernel<mfma::A_ROWS_K, mfma::B_BITS_ALONG_K_SCALED, mfma::EPI_EVIDENCE, QSTE_F16>
@@ -1225,11 +1243,12 @@ int mfma_evidence_t(const void* dy, int dtype, const uint8_t* x_t, int64_t x_t_p
   return static_cast<int>(hipGetLastError());
 }
 
-// Whether mfma_backward_pair takes a call (workspace copies are 256-byte
-// aligned, so only the caller's operands are checked here).
-bool mfma_pair_ok(const void* dy, int dtype, int64_t samples, int64_t rows, int64_t cols) {
-  return mfma_dtype(dtype) && cols % 64 == 0 && rows % 64 == 0 && rows > 0 && cols > 0 && samples > 0 &&
-         aligned16(dy) && fits32(samples * rows * 2) && fits32(samples * cols / 8) && fits32(rows * cols / 8);
+// Whether a layer's backward runs on the matrix cores from `ldy` columns of dy
+// (workspace copies are 256-byte aligned, so only dy itself is checked here).
+bool mfma_backward_ok(const void* dy, int64_t ldy, int dtype, int64_t samples, int64_t rows, int64_t cols) {
+  const int64_t c64 = (cols + 63) / 64 * 64;
+  return mfma_dtype(dtype) && rows > 0 && cols > 0 && samples > 0 && ldy % 64 == 0 && aligned16(dy) &&
+         fits32(samples * ldy * 2) && fits32(samples * c64 / 8) && fits32(rows * c64 / 8);
 }
 
 // ---------------------------------------------------------------------------
@@ -1348,13 +1367,13 @@ EvidencePlan mfma_evidence_plan(int64_t samples, int64_t rows, int64_t cols, boo
 // to a multiple of 64 entries.  `plan` is mfma_evidence_plan's for the
 // shape (with pair set); its split tiles need plan.partial_bytes at
 // `partial`.  Returns 1 when either product is not for this path.
-int mfma_backward_pair(const void* dy, int dtype, const uint8_t* x_t, int64_t x_t_pitch, const uint16_t* x_scale16,
-                       float* ev, const uint8_t* w_t, int64_t w_t_pitch, const uint16_t* scale16,
-                       const uint8_t* packed_w, void* dx, int64_t samples, int64_t rows, int64_t cols,
-                       const float* m_add, const float* scale, float* gs_partial, const EvidencePlan& plan,
-                       float* partial, hipStream_t stream) {
-  if (!evidence_ok(dy, dtype, x_t, samples, rows, cols) || !fits32(cols * x_t_pitch) || !dx ||
-      !dgrad_ok(dy, dtype, w_t, samples, rows, cols) || !fits32(cols * w_t_pitch))
+int mfma_backward_pair(const void* dy, int64_t ldy, int dtype, const uint8_t* x_t, int64_t x_t_pitch,
+                       const uint16_t* x_scale16, float* ev, const uint8_t* w_t, int64_t w_t_pitch,
+                       const uint16_t* scale16, const uint8_t* packed_w, int64_t w_pb, void* dx, int64_t samples,
+                       int64_t rows, int64_t cols, const float* m_add, const float* scale, float* gs_partial,
+                       const EvidencePlan& plan, float* partial, hipStream_t stream) {
+  if (!dx || !backward_operands_ok(dy, ldy, dtype, x_t, x_t_pitch, samples, rows, cols) ||
+      !backward_operands_ok(dy, ldy, dtype, w_t, w_t_pitch, samples, rows, cols))
     return 1;
   if (plan.splits > 1 && !partial) return QSTE_E_WORKSPACE;
   mfma::Params pe{};
@@ -1363,16 +1382,16 @@ int mfma_backward_pair(const void* dy, int dtype, const uint8_t* x_t, int64_t x_
   pe.kscale16 = x_scale16;
   pe.out = ev;
   pe.M = rows; pe.N = cols; pe.K = samples;
-  pe.lda = rows; pe.pb = x_t_pitch;
+  pe.lda = ldy; pe.pb = x_t_pitch;
   pe.a_rows = samples; pe.bit_rows = cols;
-  pe.m_add = m_add; pe.m_scale = scale; pe.w_bits = packed_w; pe.w_pb = cols / 8; pe.gs_partial = gs_partial;
+  pe.m_add = m_add; pe.m_scale = scale; pe.w_bits = packed_w; pe.w_pb = w_pb; pe.gs_partial = gs_partial;
   mfma::Params pd{};
   pd.a = static_cast<const uint16_t*>(dy);
   pd.bits = w_t;
   pd.kscale16 = scale16;
   pd.out = dx;
-  pd.M = samples; pd.N = cols; pd.K = rows;
-  pd.lda = rows; pd.pb = w_t_pitch;
+  pd.M = samples; pd.N = cols; pd.K = ldy;
+  pd.lda = ldy; pd.pb = w_t_pitch;
   pd.a_rows = samples; pd.bit_rows = cols;
   const int te = wide_grid(rows, cols), td = wide_grid(samples, cols);
   const bool split = plan.splits > 1 && aligned16(ev);  // the combine pass stores 16 bytes at a time
@@ -1388,7 +1407,7 @@ int mfma_backward_pair(const void* dy, int dtype, const uint8_t* x_t, int64_t x_
   }
   int rc = static_cast<int>(hipGetLastError());
   if (rc || !split) return rc;
-  return launch_combine(sp, m_add, scale, packed_w, ev, gs_partial, rows, cols, stream);
+  return launch_combine(sp, m_add, scale, packed_w, w_pb, ev, gs_partial, rows, cols, stream);
 }
 
 // ---------------------------------------------------------------------------
