@@ -35,10 +35,11 @@ int launch_coordinate_update(const float*, int8_t*, uint8_t*, int8_t*, uint16_t*
 // MFMA paths (gemm_mfma.hip): return 1 when the shape/dtype is not theirs.
 int mfma_linear_forward(const void*, int, const uint8_t*, const float*, const float*, void*, int64_t,
                         int64_t, int64_t, hipStream_t);
-int mfma_linear_dgrad(const void*, int, const uint8_t*, const float*, void*, int64_t, int64_t, int64_t,
+int mfma_linear_dgrad(const void*, int, const uint8_t*, const float*, void*, int64_t, int64_t, int64_t, float*,
                       hipStream_t);
 int mfma_linear_dgrad_t(const void*, int64_t, int, const uint8_t*, int64_t, const uint16_t*, void*, int64_t, int64_t,
-                        int64_t, hipStream_t);
+                        int64_t, float*, hipStream_t);
+int64_t mfma_dgrad_split_bytes(int64_t, int64_t, int64_t);
 int mfma_evidence(const void*, int, const uint8_t*, const float*, float*, int64_t, int64_t, int64_t,
                   const float*, const float*, const uint8_t*, float*, const EvidencePlan*, float*, hipStream_t);
 int mfma_evidence_t(const void*, int64_t, int, const uint8_t*, int64_t, const uint16_t*, float*, int64_t, int64_t,
@@ -148,6 +149,9 @@ BackwardLayout backward_layout(int64_t samples, int64_t rows, int64_t cols, Layo
   int64_t partial = mfma_evidence_plan(samples, rows, cols, true).partial_bytes;
   const int64_t alone = mfma_evidence_plan(samples, rows, cols, false).partial_bytes;
   if (alone > partial) partial = alone;
+  // dX as a launch of its own runs before the evidence, in the same space
+  const int64_t dgrad = mfma_dgrad_split_bytes(samples, rows, cols);
+  if (dgrad > partial) partial = dgrad;
   l.partial = at; at += align_up(static_cast<size_t>(partial));
   l.limb_bytes = 0;
   if (kind == LAYOUT_LIMBS) {
@@ -174,8 +178,8 @@ int forward_dispatch(const void* x, int dtype, const uint8_t* packed, const floa
 }
 
 int dgrad_dispatch(const void* dy, int dtype, const uint8_t* packed, const float* row_scale, void* dx,
-                   int64_t m, int64_t rows, int64_t cols, hipStream_t s) {
-  int rc = mfma_linear_dgrad(dy, dtype, packed, row_scale, dx, m, rows, cols, s);
+                   int64_t m, int64_t rows, int64_t cols, hipStream_t s, float* partial = nullptr) {
+  int rc = mfma_linear_dgrad(dy, dtype, packed, row_scale, dx, m, rows, cols, partial, s);
   if (rc != 1) return rc;
   return simt_linear_dgrad(dy, dtype, packed, row_scale, dx, m, rows, cols, s);
 }
@@ -265,20 +269,26 @@ int qste_packed_linear_affine(const void* x, int dtype, const uint8_t* packed, c
 
 namespace {
 
-// A 16-bit forward whose columns no matrix path takes (a multiple of 64; of
-// 128 up to 64 rows) runs it on copies of x and the signs that are padded
+// A forward whose columns no matrix path takes (a multiple of 64; of 128 up to
+// 64 rows, 21 of fp32) runs it on copies of x and the signs that are padded
 // with zeros (a zero x times either sign adds nothing).  The scalar kernel's
 // time is its K chain, about 2.3 us per 16 columns; the copies and the product
 // take 9-13 us up to 64 rows (64 x 300 x 130: 23.5 -> 12.3, 32 x 65 x 65: 14.2
 // -> 9.4) and 24-29 us on 256-row tiles (128 x 300 x 300: 45 -> 24, 2048 x 1000
 // x 3000: 503 -> 46, but 1000 x 130 x 130: 24 / 26): hence the two lines.
 int64_t padded_forward_cols(int64_t m, int64_t rows, int64_t cols, int dtype) {
-  if ((dtype != QSTE_BF16 && dtype != QSTE_F16) || m <= 0 || rows <= 0 || cols <= (m <= 64 ? 64 : 160))
-    return 0;
-  const int64_t unit = m <= 64 ? 128 : 64;
+  if (m <= 0 || rows <= 0) return 0;
+  if (dtype == QSTE_F32) {
+    // past 21 rows the limb copies pad by themselves
+    if (m > 21 || cols <= 64 || cols % 128 == 0) return 0;
+  } else {
+    if (cols <= (m <= 64 ? 64 : 160) || cols % (m <= 64 ? 128 : 64) == 0) return 0;
+  }
   // the copies are rows of whole 16-byte words of signs
-  return cols % unit == 0 ? 0 : (cols + 127) / 128 * 128;
+  return (cols + 127) / 128 * 128;
 }
+
+size_t elem_bytes(int dtype) { return dtype == QSTE_F32 ? 4 : 2; }
 
 size_t plain_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
   if (const size_t skinny = gemv_forward_workspace(m, rows, cols, dtype)) return skinny;
@@ -289,7 +299,7 @@ size_t plain_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype)
 
 size_t qste_packed_linear_affine_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int dtype) {
   if (const int64_t pc = padded_forward_cols(m, rows, cols, dtype))
-    return align_up(static_cast<size_t>(m * pc) * 2) + align_up(static_cast<size_t>(rows * pc / 8)) +
+    return align_up(static_cast<size_t>(m * pc) * elem_bytes(dtype)) + align_up(static_cast<size_t>(rows * pc / 8)) +
            plain_forward_workspace(m, rows, pc, dtype);
   return plain_forward_workspace(m, rows, cols, dtype);
 }
@@ -305,10 +315,10 @@ int qste_packed_linear_affine_ws(const void* x, int dtype, const uint8_t* packed
   if (pc && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
       workspace_bytes >= qste_packed_linear_affine_workspace_bytes(m, rows, cols, dtype)) {
     hipStream_t s = as_stream(stream);
-    const size_t xb = align_up(static_cast<size_t>(m * pc) * 2), wb = align_up(static_cast<size_t>(rows * pc / 8));
+    const size_t eb = elem_bytes(dtype), xb = align_up(static_cast<size_t>(m * pc) * eb), wb = align_up(static_cast<size_t>(rows * pc / 8));
     char* xp = static_cast<char*>(workspace);
     char* wp = xp + xb;
-    int rc = launch_pad_rows(x, xp, m, 2 * cols, 2 * pc, s);
+    int rc = launch_pad_rows(x, xp, m, static_cast<int64_t>(eb) * cols, static_cast<int64_t>(eb) * pc, s);
     if (rc) return rc;
     if ((rc = launch_pad_rows(packed, wp, rows, (cols + 7) / 8, pc / 8, s))) return rc;
     return qste_packed_linear_affine_ws(xp, dtype, reinterpret_cast<uint8_t*>(wp), scale, bias, y, m, rows, pc,
@@ -332,7 +342,8 @@ int qste_packed_linear_affine_ws(const void* x, int dtype, const uint8_t* packed
 }
 
 size_t qste_packed_transpose_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int dtype) {
-  return dtype == QSTE_F32 ? f32_dgrad_workspace(m, rows, cols) : 0;
+  if (dtype == QSTE_F32) return f32_dgrad_workspace(m, rows, cols);
+  return rows % 64 == 0 && cols % 64 == 0 ? static_cast<size_t>(mfma_dgrad_split_bytes(m, rows, cols)) : 0;
 }
 
 int qste_packed_transpose_ws(const void* dy, int dtype, const uint8_t* packed, const float* row_scale, void* dx,
@@ -347,7 +358,10 @@ int qste_packed_transpose_ws(const void* dy, int dtype, const uint8_t* packed, c
                                   cols, workspace, workspace_bytes, as_stream(stream));
     if (rc != 1) return rc;
   }
-  return dgrad_dispatch(dy, dtype, packed, row_scale, dx, m, rows, cols, as_stream(stream));
+  const bool room = dtype != QSTE_F32 && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+                    static_cast<int64_t>(workspace_bytes) >= mfma_dgrad_split_bytes(m, rows, cols);
+  return dgrad_dispatch(dy, dtype, packed, row_scale, dx, m, rows, cols, as_stream(stream),
+                        room ? static_cast<float*>(workspace) : nullptr);
 }
 
 int qste_packed_transpose(const void* dy, int dtype, const uint8_t* packed, const float* row_scale,
@@ -492,8 +506,8 @@ int linear_backward_impl(const void* dy, int dtype, const uint8_t* packed_x, con
         if (rc != 1) return rc;
       } else {
         if (dx) {
-          rc = mfma_linear_dgrad_t(dy_m, ldy, dtype, w_t, l.w_t_pitch, s16, dx, samples, rows, cols, s);
-          if (rc == 1) rc = dgrad_dispatch(dy, dtype, packed_w, scale, dx, samples, rows, cols, s);
+          rc = mfma_linear_dgrad_t(dy_m, ldy, dtype, w_t, l.w_t_pitch, s16, dx, samples, rows, cols, partial, s);
+          if (rc == 1) rc = dgrad_dispatch(dy, dtype, packed_w, scale, dx, samples, rows, cols, s, partial);
           if (rc) return rc;
         }
         dgrad_done = true;

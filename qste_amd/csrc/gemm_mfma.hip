@@ -729,6 +729,12 @@ __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0,
             // the outputs again (0.3-3% faster per launch than plain stores)
             const u32x4 w = {v.x, v.y, v.z, v.w};
             __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(y + grow * p.N + gcol));
+          } else if (gcol + 8 <= p.N) {
+            // rows off 16-byte boundaries: one unaligned store
+            struct __attribute__((packed)) Unaligned16 {
+              uint32_t w[4];
+            };
+            *reinterpret_cast<Unaligned16*>(y + grow * p.N + gcol) = Unaligned16{{v.x, v.y, v.z, v.w}};
           } else {
             const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
 #pragma unroll
@@ -902,23 +908,30 @@ __global__ __launch_bounds__(THREADS) void evidence_combine_kernel(Split sp, con
   for (int o = 8; o >= 1; o >>= 1) signed_e0 += __shfl_xor(signed_e0, o, kWave);
   if (gs_partial && lane % 16 == 0) gs_partial[(static_cast<int64_t>(tn) * WAVES_N + lane / 16) * M + row] = signed_e0;
 }
-// Split-K forward for products with few output tiles and a long K chain
-// (fp32 limbs at small M): workgroup w covers tile w % tiles over K range
-// w / tiles (ks_steps K steps) and stores its bare accumulators in slab w of
-// `partial` (BM x BN fp32 each) for forward_combine_kernel.
-template <int DT>
-__global__ __launch_bounds__(THREADS, 1) void forward_split_kernel(Params p, int tiles, int ks_steps,
+// Split-K product (forward or dX) for few output tiles and a long K chain:
+// workgroup w covers tile w % tiles over K range w / tiles (ks_steps K steps)
+// and stores its bare accumulators in slab w of `partial` (BM x BN fp32 each)
+// for forward_combine_kernel.
+template <int BKIND, int DT>
+__global__ __launch_bounds__(THREADS, 1) void product_split_kernel(Params p, int tiles, int ks_steps,
                                                                    float* partial) {
-  using SZ = StageSizes<A_ROWS_M, B_BITS_ALONG_K>;
+  using SZ = StageSizes<A_ROWS_M, BKIND>;
   QSTE_WIDE_STAGES(SZ::a, SZ::b, SZ::s)
   const int w = static_cast<int>(blockIdx.x), i = w % tiles, j = w / tiles;
   const int64_t k0 = static_cast<int64_t>(j) * ks_steps * BK;
   Params q = p;
-  q.a = p.a + k0;          // columns k0 .. of every dense row (lda unchanged)
-  q.bits = p.bits + k0 / 8;  // bits k0 .. of every packed row (pb unchanged)
+  q.a = p.a + k0;  // columns k0 .. of every dense row (lda unchanged)
+  if (BKIND == B_BITS_ALONG_N) {
+    q.bits = p.bits + k0 * p.pb;  // packed rows k0 ..
+    q.bit_rows = p.bit_rows - k0;
+    if (p.kscale) q.kscale = p.kscale + k0;
+  } else {
+    q.bits = p.bits + k0 / 8;  // bits k0 .. of every packed row (pb unchanged)
+    if (BKIND == B_BITS_ALONG_K_SCALED) q.kscale16 = p.kscale16 + k0;
+  }
   q.K = p.K - k0 < static_cast<int64_t>(ks_steps) * BK ? p.K - k0 : static_cast<int64_t>(ks_steps) * BK;
   q.out = partial + static_cast<int64_t>(w) * (BM * BN);
-  wide_tile<A_ROWS_M, B_BITS_ALONG_K, EPI_PARTIAL, DT>(q, i, A0, A1, A2, A3, B0, B1, B2, B3, Sc);
+  wide_tile<A_ROWS_M, BKIND, EPI_PARTIAL, DT>(q, i, A0, A1, A2, A3, B0, B1, B2, B3, Sc);
 }
 
 // y = (the K ranges' accumulators summed in range order) * scale[n] +
@@ -944,17 +957,34 @@ __global__ __launch_bounds__(THREADS) void forward_combine_kernel(const float* _
     const float4 v = *reinterpret_cast<const float4*>(src + static_cast<int64_t>(j) * tiles * (BM * BN));
     acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
   }
-  const float a[4] = {acc.x, acc.y, acc.z, acc.w};
+  const int64_t col0 = static_cast<int64_t>(tn) * BN + lcol;
+  float v[4] = {acc.x, acc.y, acc.z, acc.w};
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int64_t col = static_cast<int64_t>(tn) * BN + lcol + q;
+    const int64_t col = col0 + q;
     if (col < N) {
-      float v = a[q] * (n_scale ? n_scale[col] : 1.0f);
-      v = v + (n_bias ? n_bias[col] : 0.0f);
+      v[q] = v[q] * (n_scale ? n_scale[col] : 1.0f);
+      v[q] = v[q] + (n_bias ? n_bias[col] : 0.0f);
+    }
+  }
+  const int64_t at = row * N + col0;
+  // N a multiple of 4 keeps every quad of an aligned output aligned
+  const bool vec = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+  if (vec && col0 < N) {
+    if constexpr (OUT == QSTE_F32)
+      *reinterpret_cast<float4*>(static_cast<float*>(out) + at) = make_float4(v[0], v[1], v[2], v[3]);
+    else
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + at) =
+          make_uint2(round16x2<OUT>(v[0], v[1]), round16x2<OUT>(v[2], v[3]));
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (col0 + q < N) {
       if constexpr (OUT == QSTE_F32)
-        static_cast<float*>(out)[row * N + col] = v;
+        static_cast<float*>(out)[at + q] = v[q];
       else
-        static_cast<uint16_t*>(out)[row * N + col] = round16<OUT>(v);
+        static_cast<uint16_t*>(out)[at + q] = round16<OUT>(v[q]);
     }
   }
 }
@@ -970,6 +1000,8 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // bf16 and fp16 take the MFMA path (fp32 stays on the fp32 SIMT kernel)
 static bool mfma_dtype(int dtype) { return dtype == QSTE_BF16 || dtype == QSTE_F16; }
+
+EvidencePlan mfma_evidence_plan(int64_t samples, int64_t rows, int64_t cols, bool with_dgrad);
 
 // Buffer offsets are 32-bit: every operand must stay under 4 GiB.
 static bool fits32(int64_t bytes) { return bytes < (int64_t{1} << 32); }
@@ -1061,15 +1093,15 @@ int mfma_linear_forward(const void* x, int dtype, const uint8_t* packed, const f
 }
 
 // K ranges of a forward with `tiles` output tiles and nk K steps: a product
-// with fewer tiles than half the device's 256 CUs and a long K chain is cut
-// into up to 16 ranges of at least 4 K steps (one round of workgroups),
-// else 1.
+// with fewer tiles than half the device's 256 CUs and a K chain of 12 steps or
+// more is cut into up to 16 ranges of at least 4 K steps (one round of
+// workgroups), else 1.
 struct SplitK {
   int splits, ks_steps;
 };
 static SplitK forward_split_plan(int tiles, int nk) {
   int s = 1;
-  if (tiles > 0 && 2 * tiles <= 256 && nk >= 16) {
+  if (tiles > 0 && 2 * tiles <= 256 && nk >= 12) {
     s = 16;
     if (s > 256 / tiles) s = 256 / tiles;
     if (s > nk / 4) s = nk / 4;
@@ -1078,6 +1110,25 @@ static SplitK forward_split_plan(int tiles, int nk) {
   const int ks = (nk + s - 1) / s;
   return {(nk + ks - 1) / ks, ks};
 }
+static size_t split_bytes(const SplitK& sp, int tiles) {
+  return sp.splits > 1 ? static_cast<size_t>(sp.splits) * tiles * mfma::wide::BM * mfma::wide::BN * sizeof(float) : 0;
+}
+
+// A product cut into the plan's K ranges and combined: scale and bias per
+// column (or null), stored as OUT.
+template <int BKIND, int DT, int OUT>
+static int launch_split(const mfma::Params& p, const SplitK& sp, float* partial, hipStream_t stream) {
+  const int tiles = wide_grid(p.M, p.N);
+  mfma::wide::product_split_kernel<BKIND, DT>
+      <<<tiles * sp.splits, mfma::wide::THREADS, 0, stream>>>(p, tiles, sp.ks_steps, partial);
+  const int rc = static_cast<int>(hipGetLastError());
+  if (rc) return rc;
+  const dim3 grid(mfma::wide::BM / (mfma::wide::THREADS / kWave), static_cast<unsigned>(tiles));
+  mfma::wide::forward_combine_kernel<OUT><<<grid, mfma::wide::THREADS, 0, stream>>>(
+      partial, tiles, sp.splits, p.n_scale, p.n_bias, p.out, p.M, p.N);
+  return static_cast<int>(hipGetLastError());
+}
+
 // The 16-bit forward with few output tiles (M past the decode GEMV's 16, a
 // round of 256-row tiles or less) over a long K: K ranges as for the fp32
 // limbs, their accumulators in a caller workspace, then scale, bias and one
@@ -1085,9 +1136,7 @@ static SplitK forward_split_plan(int tiles, int nk) {
 size_t mfma_forward_split_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
   if (!mfma_dtype(dtype) || m <= 16 || rows <= 0 || cols <= 0 || cols % 64 != 0) return 0;
   const int tiles = wide_grid(m, rows);
-  const SplitK sp = forward_split_plan(tiles, static_cast<int>(cols / mfma::wide::BK));
-  return sp.splits > 1 ? static_cast<size_t>(sp.splits) * tiles * mfma::wide::BM * mfma::wide::BN * sizeof(float)
-                       : 0;
+  return split_bytes(forward_split_plan(tiles, static_cast<int>(cols / mfma::wide::BK)), tiles);
 }
 
 // Returns 1 when the call is not for this path (shape, or too little workspace).
@@ -1104,31 +1153,42 @@ int mfma_linear_forward_split(const void* x, int dtype, const uint8_t* packed, c
   p.M = m; p.N = rows; p.K = cols;
   p.lda = cols; p.pb = cols / 8;
   p.a_rows = m; p.bit_rows = rows;
-  const int tiles = wide_grid(m, rows);
-  const SplitK sp = forward_split_plan(tiles, static_cast<int>(cols / mfma::wide::BK));
+  p.out = y;
+  p.n_scale = scale; p.n_bias = bias;
+  const SplitK sp = forward_split_plan(wide_grid(m, rows), static_cast<int>(cols / mfma::wide::BK));
   float* partial = static_cast<float*>(workspace);
-  if (dtype == QSTE_F16)
-    mfma::wide::forward_split_kernel<QSTE_F16>
-        <<<tiles * sp.splits, mfma::wide::THREADS, 0, stream>>>(p, tiles, sp.ks_steps, partial);
-  else
-    mfma::wide::forward_split_kernel<QSTE_BF16>
-        <<<tiles * sp.splits, mfma::wide::THREADS, 0, stream>>>(p, tiles, sp.ks_steps, partial);
-  int rc = static_cast<int>(hipGetLastError());
-  if (rc) return rc;
-  const dim3 grid(mfma::wide::BM / (mfma::wide::THREADS / kWave), static_cast<unsigned>(tiles));
-  if (dtype == QSTE_F16)
-    mfma::wide::forward_combine_kernel<QSTE_F16>
-        <<<grid, mfma::wide::THREADS, 0, stream>>>(partial, tiles, sp.splits, scale, bias, y, m, rows);
-  else
-    mfma::wide::forward_combine_kernel<QSTE_BF16>
-        <<<grid, mfma::wide::THREADS, 0, stream>>>(partial, tiles, sp.splits, scale, bias, y, m, rows);
-  return static_cast<int>(hipGetLastError());
+  return dtype == QSTE_F16
+             ? launch_split<mfma::B_BITS_ALONG_K, QSTE_F16, QSTE_F16>(p, sp, partial, stream)
+             : launch_split<mfma::B_BITS_ALONG_K, QSTE_BF16, QSTE_BF16>(p, sp, partial, stream);
 }
 
+// The input gradient as a launch of its own, where its tiles are few: K cut
+// into ranges as the forward's is (2046 x 768 from 50257 rows, 24 tiles of 786
+// K steps: 934 -> 142 us).  dgrad_cut does not look at the layer's plan,
+// which weighs its time; a layer whose evidence and input gradient share one
+// launch is not cut, and the product called alone is cut as the layer's is,
+// so the two agree bit for bit.
+static SplitK dgrad_cut(int64_t m, int64_t rows, int64_t cols) {
+  return forward_split_plan(wide_grid(m, cols), static_cast<int>((rows + mfma::wide::BK - 1) / mfma::wide::BK));
+}
+static SplitK dgrad_split(int64_t m, int64_t rows, int64_t cols) {
+  if (mfma_evidence_plan(m, rows, cols, true).pair) return {1, 0};
+  return dgrad_cut(m, rows, cols);
+}
+int64_t mfma_dgrad_split_bytes(int64_t m, int64_t rows, int64_t cols) {
+  if (m <= 0 || rows <= 0 || cols <= 0) return 0;
+  return static_cast<int64_t>(split_bytes(dgrad_split(m, rows, cols), wide_grid(m, cols)));
+}
+
+// `partial`: mfma_dgrad_split_bytes of space, or null (unsplit)
 int mfma_linear_dgrad(const void* dy, int dtype, const uint8_t* packed, const float* row_scale, void* dx,
-                      int64_t m, int64_t rows, int64_t cols, hipStream_t stream) {
+                      int64_t m, int64_t rows, int64_t cols, float* partial, hipStream_t stream) {
   if (!dgrad_ok(dy, dtype, packed, m, rows, cols)) return 1;
   const mfma::Params p = dgrad_params(dy, packed, row_scale, dx, m, rows, cols);
+  const SplitK sp = partial ? dgrad_split(m, rows, cols) : SplitK{1, 0};
+  if (sp.splits > 1)
+    return dtype == QSTE_F16 ? launch_split<mfma::B_BITS_ALONG_N, QSTE_F16, QSTE_F16>(p, sp, partial, stream)
+                             : launch_split<mfma::B_BITS_ALONG_N, QSTE_BF16, QSTE_BF16>(p, sp, partial, stream);
   if (dtype == QSTE_F16)
     mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_N, mfma::EPI_PLAIN, QSTE_F16>
         <<<wide_grid(m, cols), mfma::wide::THREADS, 0, stream>>>(p);
@@ -1144,9 +1204,9 @@ int mfma_linear_dgrad(const void* dy, int dtype, const uint8_t* packed, const fl
 // are one byte and each expansion is one shift-and-OR per pair, as in the
 // forward.  Measured 6-10% faster than bits along N at config 4's shapes;
 // the results are identical (the same bf16 operand values, the same
-// accumulation order).
+// accumulation order).  With `partial` given, K is cut as dgrad_split says.
 int mfma_linear_dgrad_t(const void* dy, int64_t ldy, int dtype, const uint8_t* w_t, int64_t w_t_pitch,
-                        const uint16_t* scale16, void* dx, int64_t m, int64_t rows, int64_t cols,
+                        const uint16_t* scale16, void* dx, int64_t m, int64_t rows, int64_t cols, float* partial,
                         hipStream_t stream) {
   if (!backward_operands_ok(dy, ldy, dtype, w_t, w_t_pitch, m, rows, cols)) return 1;
   mfma::Params p{};
@@ -1157,6 +1217,11 @@ int mfma_linear_dgrad_t(const void* dy, int64_t ldy, int dtype, const uint8_t* w
   p.M = m; p.N = cols; p.K = ldy;
   p.lda = ldy; p.pb = w_t_pitch;
   p.a_rows = m; p.bit_rows = cols;
+  const SplitK sp = dgrad_split(m, rows, cols);
+  if (partial && sp.splits > 1)
+    return dtype == QSTE_F16
+               ? launch_split<mfma::B_BITS_ALONG_K_SCALED, QSTE_F16, QSTE_F16>(p, sp, partial, stream)
+               : launch_split<mfma::B_BITS_ALONG_K_SCALED, QSTE_BF16, QSTE_BF16>(p, sp, partial, stream);
   if (dtype == QSTE_F16)
     mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K_SCALED, mfma::EPI_PLAIN, QSTE_F16>
         <<<wide_grid(m, cols), mfma::wide::THREADS, 0, stream>>>(p);
@@ -1303,7 +1368,15 @@ static EvidencePlan compute_plan(int64_t samples, int64_t rows, int64_t cols, bo
   EvidencePlan best{0, static_cast<int>(te), 1, static_cast<int>(nk), 0};
   if (samples <= 0 || rows <= 0 || cols <= 0) return best;
   const int64_t dgrad[1][2] = {{td, nkd + kTileOverhead}};
-  const double dgrad_alone = td ? static_cast<double>(list_schedule(dgrad, 1)) : 0.0;
+  double dgrad_alone = td ? static_cast<double>(list_schedule(dgrad, 1)) : 0.0;
+  if (const int64_t splits = td ? dgrad_cut(samples, rows, cols).splits : 1; splits > 1) {
+    // as its own launch dX cuts K where its tiles are few
+    const int64_t ks = (nkd + splits - 1) / splits;
+    const int64_t ranges[1][2] = {{td * splits, ks + kTileOverhead}};
+    const double cut = static_cast<double>(list_schedule(ranges, 1)) +
+                       static_cast<double>((splits + 1) * td * kTileBytes) / kBytesPerStep + 2.0;
+    if (cut < dgrad_alone) dgrad_alone = cut;
+  }
   double best_cost = -1.0;
   for (int S = 1; S <= 8; S *= 2) {
     const int64_t ks = (nk + S - 1) / S;
@@ -1428,50 +1501,79 @@ int mfma_backward_pair(const void* dy, int64_t ldy, int dtype, const uint8_t* x_
 namespace limbs {
 
 // out[plane * p + r * ld + c] for the three limbs p of x[r, c] (times
-// row_mul[r] or col_mul[c] when given)
+// row_mul[r] or col_mul[c] when given), c < `padded` (a multiple of 4, as ld
+// and plane are), zero from `cols` on; four columns a thread.
 __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ x, int64_t rows, int64_t cols,
                                                     const float* __restrict__ row_mul,
                                                     const float* __restrict__ col_mul, uint16_t* __restrict__ out,
-                                                    int64_t ld, int64_t plane) {
-  const int64_t n = rows * cols;
+                                                    int64_t ld, int64_t plane, int64_t padded) {
+  const int64_t per = padded / 4, n = rows * per;
+  const bool vec = (cols & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t r = i / cols, c = i - r * cols;
-    float v = x[i];
-    if (row_mul) v = v * row_mul[r];
-    if (col_mul) v = v * col_mul[c];
-    uint16_t hi = f32_to_bf16(v);
-    const bool finite = __builtin_isfinite(v);
-    // a finite value that rounds past bf16's largest finite one keeps its
-    // top 16 bits instead (truncation: the residual is exact as well); an
-    // infinite or NaN value is carried by hi alone, its other limbs zero,
-    // so the products see the same inf or NaN the fp32 operand holds
-    if (finite && (hi & 0x7F80u) == 0x7F80u) hi = static_cast<uint16_t>(__float_as_uint(v) >> 16);
-    const float r1 = finite ? v - bf16_to_f32(hi) : 0.0f;
-    const uint16_t mid = f32_to_bf16(r1);
-    const float r2 = r1 - bf16_to_f32(mid);
-    const uint16_t lo = f32_to_bf16(r2);
+    const int64_t r = i / per, c = 4 * (i - r * per);
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (vec && c < cols) {
+      const float4 q = *reinterpret_cast<const float4*>(x + r * cols + c);
+      v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (c + k < cols) v[k] = x[r * cols + c + k];
+    }
+    uint16_t h[3][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float f = v[k];
+      if (row_mul) f = f * row_mul[r];
+      if (col_mul && c + k < cols) f = f * col_mul[c + k];
+      uint16_t hi = f32_to_bf16(f);
+      const bool finite = __builtin_isfinite(f);
+      // a finite value that rounds past bf16's largest finite one keeps its
+      // top 16 bits instead (truncation: the residual is exact as well); an
+      // infinite or NaN value is carried by hi alone, its other limbs zero,
+      // so the products see the same inf or NaN the fp32 operand holds
+      if (finite && (hi & 0x7F80u) == 0x7F80u) hi = static_cast<uint16_t>(__float_as_uint(f) >> 16);
+      const float r1 = finite ? f - bf16_to_f32(hi) : 0.0f;
+      const uint16_t mid = f32_to_bf16(r1);
+      h[0][k] = hi;
+      h[1][k] = mid;
+      h[2][k] = f32_to_bf16(r1 - bf16_to_f32(mid));
+    }
     uint16_t* o = out + r * ld + c;
-    o[0] = hi;
-    o[plane] = mid;
-    o[2 * plane] = lo;
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+      *reinterpret_cast<uint2*>(o + p * plane) = make_uint2(h[p][0] | (static_cast<uint32_t>(h[p][1]) << 16),
+                                                            h[p][2] | (static_cast<uint32_t>(h[p][3]) << 16));
   }
 }
 
 // out[plane * p + r * out_ld + j] = in[r * in_ld + j] for p = 0, 1, 2 and
-// j < bytes (the packed signs repeated for each limb); in may be plane 0 of
-// out itself, which is then left as it is
+// j < bytes, zero for j < `padded` (a multiple of 8, as out_ld and plane are):
+// the packed signs repeated for each limb; in may be plane 0 of out itself
+// (bytes == padded then), which is left as it is
 __global__ __launch_bounds__(256) void repeat_kernel(const uint8_t* in, int64_t rows, int64_t bytes, int64_t in_ld,
-                                                     uint8_t* out, int64_t out_ld, int64_t plane) {
-  const int64_t n = rows * bytes;
+                                                     uint8_t* out, int64_t out_ld, int64_t plane, int64_t padded) {
+  struct __attribute__((packed)) Unaligned8 {
+    uint64_t w;
+  };
+  const int64_t per = padded / 8, n = rows * per;
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t r = i / bytes, j = i - r * bytes;
-    const uint8_t v = in[r * in_ld + j];
+    const int64_t r = i / per, j = 8 * (i - r * per);
+    const uint8_t* src = in + r * in_ld + j;
+    uint64_t v = 0;
+    if (j + 8 <= bytes) {
+      v = reinterpret_cast<const Unaligned8*>(src)->w;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (j + k < bytes) v |= static_cast<uint64_t>(src[k]) << (8 * k);
+    }
     uint8_t* o = out + r * out_ld + j;
-    if (o != in + r * in_ld + j) o[0] = v;
-    o[plane] = v;
-    o[2 * plane] = v;
+    if (o != src) *reinterpret_cast<uint64_t*>(o) = v;
+    *reinterpret_cast<uint64_t*>(o + plane) = v;
+    *reinterpret_cast<uint64_t*>(o + 2 * plane) = v;
   }
 }
 
@@ -1487,16 +1589,28 @@ inline size_t up256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 // The limbs of x [rows, cols] as rows of their own: out [3 rows, cols], row
 // 3r + i limb i (hi, mid, lo) of row r.
 int launch_limbs(const float* x, int64_t rows, int64_t cols, uint16_t* out, hipStream_t stream) {
-  limbs::split_kernel<<<limbs::grid_for(rows * cols), 256, 0, stream>>>(x, rows, cols, nullptr, nullptr, out, 3 * cols,
-                                                                        cols);
+  limbs::split_kernel<<<limbs::grid_for(rows * cols / 4), 256, 0, stream>>>(x, rows, cols, nullptr, nullptr, out,
+                                                                            3 * cols, cols, cols);
   return static_cast<int>(hipGetLastError());
 }
 
 int launch_transpose_bits(const uint8_t*, uint8_t*, int64_t, int64_t, int64_t, int64_t, hipStream_t);
 
-// Whether a product of these sizes takes the limbs (enough rows of output to
-// fill 256-row tiles; below that the fp32 SIMT kernels are as fast)
-static bool f32_limbs_worth(int64_t m) { return m >= 128; }
+// Whether an [m, n] product over k takes the limbs.  From 128 rows and for
+// whole 64-column steps always; else where an estimate in us says so.  The
+// scalar kernel: its serial chain or its rate, the limbs: their copies, the
+// K ranges and the combine pass.  Measured, scalar / limbs: 24 x 2048 over
+// 2048 250 / 29, 64 x 300 over 300 45 / 20, 24 x 300 over 200 30 / about 20,
+// 2048 x 1000 over 3000 499 / 66, dX of 300 x 1000 over 64 10.7 / 47 (taken
+// for its whole steps as before).
+static bool f32_limbs_worth(int64_t m, int64_t n, int64_t k) {
+  if (m >= 128 && k % 64 == 0) return true;
+  const double flops = 2.0 * static_cast<double>(m) * n * k;
+  const double chain = 0.135 * k, rate = flops / 50e6;
+  return (chain > rate ? chain : rate) > 26.0 + flops / 350e6;
+}
+
+static int64_t up64(int64_t v) { return (v + 63) / 64 * 64; }
 
 // The limbs of the dense operand (6 bytes per fp32 value) are held to this
 // many bytes of workspace: the forward and dX products run over chunks of
@@ -1504,136 +1618,131 @@ static bool f32_limbs_worth(int64_t m) { return m >= 128; }
 // fit takes the fp32 SIMT kernels.
 constexpr size_t kLimbBudget = static_cast<size_t>(512) << 20;
 
-// Output rows per chunk of a product over k: all m when they fit the budget,
-// else a multiple of the 256-row tile (0 when not even one tile fits).
+// Output rows per chunk of a product over k (rounded up to 64 in the copies):
+// all m when they fit the budget, else a multiple of the 256-row tile (0 when
+// not even one tile fits).
 static int64_t f32_chunk_rows(int64_t m, int64_t k) {
-  const int64_t fit = static_cast<int64_t>(kLimbBudget / (static_cast<size_t>(k) * 3 * 2));
+  const int64_t fit = static_cast<int64_t>(kLimbBudget / (static_cast<size_t>(up64(k)) * 3 * 2));
   return fit >= m ? m : fit / mfma::wide::BM * mfma::wide::BM;
 }
 
-static SplitK f32_forward_split(int64_t m, int64_t rows, int64_t cols) {
-  return forward_split_plan(wide_grid(m, rows), static_cast<int>(3 * cols / mfma::wide::BK));
+static SplitK f32_split(int64_t m, int64_t n, int64_t k) {
+  return forward_split_plan(wide_grid(m, n), static_cast<int>(3 * up64(k) / mfma::wide::BK));
 }
 
-static size_t f32_forward_partial(int64_t m, int64_t rows, int64_t cols) {
-  const SplitK sp = f32_forward_split(m, rows, cols);
-  return sp.splits > 1 ? static_cast<size_t>(sp.splits) * wide_grid(m, rows) * mfma::wide::BM * mfma::wide::BN *
-                             sizeof(float)
-                       : 0;
-}
+static size_t f32_partial(int64_t m, int64_t n, int64_t k) { return split_bytes(f32_split(m, n, k), wide_grid(m, n)); }
 
-size_t f32_forward_workspace(int64_t m, int64_t rows, int64_t cols) {
-  if (m <= 0 || rows <= 0 || cols <= 0 || cols % 64 != 0 || !f32_limbs_worth(m)) return 0;
-  const int64_t mc = f32_chunk_rows(m, cols);
+// Workspace of an [m, n] product over k through the limbs (0: not for it):
+// the dense limbs of a chunk, the signs three times, and the split-K partials
+// of a full chunk or of the last, shorter one.
+static size_t f32_product_workspace(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0 || !f32_limbs_worth(m, n, k)) return 0;
+  const int64_t mc = f32_chunk_rows(m, k);
   if (mc == 0) return 0;
-  // the split-K partials of a full chunk or of the last, shorter one
-  size_t partial = f32_forward_partial(mc, rows, cols);
+  size_t partial = f32_partial(mc, n, k);
   if (m % mc) {
-    const size_t tail = f32_forward_partial(m % mc, rows, cols);
+    const size_t tail = f32_partial(m % mc, n, k);
     if (tail > partial) partial = tail;
   }
-  return limbs::up256(static_cast<size_t>(mc) * 3 * cols * 2) +
-         limbs::up256(static_cast<size_t>(rows) * 3 * cols / 8) + partial;
+  return limbs::up256(static_cast<size_t>(mc) * 3 * up64(k) * 2) +
+         limbs::up256(static_cast<size_t>(n) * 3 * up64(k) / 8) + partial;
 }
 
-// y [m, rows] fp32 = (x @ sign^T) * scale + bias through the limbs, over
-// chunks of f32_chunk_rows rows of x.  Returns 1 when the call is not for
-// this path (shape, or too little workspace).
-int mfma_f32_forward(const float* x, const uint8_t* packed, const float* scale, const float* bias, float* y,
-                     int64_t m, int64_t rows, int64_t cols, void* workspace, size_t workspace_bytes,
-                     hipStream_t stream) {
-  const size_t need = f32_forward_workspace(m, rows, cols);
-  if (need == 0 || !workspace || workspace_bytes < need) return 1;
-  const int64_t k3 = 3 * cols, kb = cols / 8, mc = f32_chunk_rows(m, cols);
-  if (!fits32(mc * k3 * 2) || !fits32(rows * k3 / 8)) return 1;
-  uint16_t* a = static_cast<uint16_t*>(workspace);
-  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(mc) * k3 * 2);
-  float* partial = reinterpret_cast<float*>(b + limbs::up256(static_cast<size_t>(rows) * k3 / 8));
-  limbs::repeat_kernel<<<limbs::grid_for(rows * kb), 256, 0, stream>>>(packed, rows, kb, kb, b, 3 * kb, kb);
+// out [m, n] = (dense [m, k] * col_mul) @ signs^T * scale + bias over chunks
+// of rows of the dense operand; the signs (bits along k, [n][3 up64(k) / 8],
+// planes of up64(k) / 8) are at `b` already.
+static int f32_product(const float* dense, const float* col_mul, const uint8_t* b, const float* scale,
+                       const float* bias, float* out, int64_t m, int64_t n, int64_t k, uint16_t* a, float* partial,
+                       hipStream_t stream) {
+  const int64_t kp = up64(k), mc = f32_chunk_rows(m, k);
   for (int64_t i0 = 0; i0 < m; i0 += mc) {
     const int64_t mi = m - i0 < mc ? m - i0 : mc;
-    float* yi = y + i0 * rows;
-    limbs::split_kernel<<<limbs::grid_for(mi * cols), 256, 0, stream>>>(x + i0 * cols, mi, cols, nullptr, nullptr, a,
-                                                                        k3, cols);
+    limbs::split_kernel<<<limbs::grid_for(mi * kp / 4), 256, 0, stream>>>(dense + i0 * k, mi, k, nullptr, col_mul, a,
+                                                                          3 * kp, kp, kp);
     mfma::Params p{};
     p.a = a;
     p.bits = b;
-    p.out = yi;
-    p.M = mi; p.N = rows; p.K = k3;
-    p.lda = k3; p.pb = 3 * kb;
-    p.a_rows = mi; p.bit_rows = rows;
+    p.out = out + i0 * n;
+    p.M = mi; p.N = n; p.K = 3 * kp;
+    p.lda = 3 * kp; p.pb = 3 * kp / 8;
+    p.a_rows = mi; p.bit_rows = n;
     p.n_scale = scale; p.n_bias = bias;
-    const SplitK sp = f32_forward_split(mi, rows, cols);
-    const int tiles = wide_grid(mi, rows);
+    const SplitK sp = f32_split(mi, n, k);
+    int rc;
     if (sp.splits > 1) {
-      mfma::wide::forward_split_kernel<QSTE_BF16>
-          <<<tiles * sp.splits, mfma::wide::THREADS, 0, stream>>>(p, tiles, sp.ks_steps, partial);
-      int rc = static_cast<int>(hipGetLastError());
-      if (rc) return rc;
-      const dim3 grid(mfma::wide::BM / (mfma::wide::THREADS / kWave), static_cast<unsigned>(tiles));
-      mfma::wide::forward_combine_kernel<QSTE_F32>
-          <<<grid, mfma::wide::THREADS, 0, stream>>>(partial, tiles, sp.splits, scale, bias, yi, mi, rows);
+      rc = launch_split<mfma::B_BITS_ALONG_K, QSTE_BF16, QSTE_F32>(p, sp, partial, stream);
     } else {
       mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD_F32, QSTE_BF16>
-          <<<tiles, mfma::wide::THREADS, 0, stream>>>(p);
+          <<<wide_grid(mi, n), mfma::wide::THREADS, 0, stream>>>(p);
+      rc = static_cast<int>(hipGetLastError());
     }
-    const int rc = static_cast<int>(hipGetLastError());
     if (rc) return rc;
   }
   return 0;
 }
 
-size_t f32_dgrad_workspace(int64_t m, int64_t rows, int64_t cols) {
-  if (m <= 0 || rows <= 0 || cols <= 0 || rows % 64 != 0 || !f32_limbs_worth(m)) return 0;
-  const int64_t mc = f32_chunk_rows(m, rows);
-  if (mc == 0) return 0;
-  return limbs::up256(static_cast<size_t>(mc) * 3 * rows * 2) +
-         limbs::up256(static_cast<size_t>(cols) * 3 * rows / 8);
+size_t f32_forward_workspace(int64_t m, int64_t rows, int64_t cols) { return f32_product_workspace(m, rows, cols); }
+
+// y [m, rows] fp32 = (x @ sign^T) * scale + bias through the limbs.  Returns 1
+// when the call is not for this path (shape, or too little workspace).
+int mfma_f32_forward(const float* x, const uint8_t* packed, const float* scale, const float* bias, float* y,
+                     int64_t m, int64_t rows, int64_t cols, void* workspace, size_t workspace_bytes,
+                     hipStream_t stream) {
+  const size_t need = f32_forward_workspace(m, rows, cols);
+  if (need == 0 || !workspace || workspace_bytes < need || !aligned16(workspace)) return 1;
+  const int64_t kp = up64(cols), kb = kp / 8, mc = f32_chunk_rows(m, cols), pb = (cols + 7) / 8;
+  if (!fits32(mc * 3 * kp * 2) || !fits32(rows * 3 * kb)) return 1;
+  uint16_t* a = static_cast<uint16_t*>(workspace);
+  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(mc) * 3 * kp * 2);
+  float* partial = reinterpret_cast<float*>(b + limbs::up256(static_cast<size_t>(rows) * 3 * kb));
+  limbs::repeat_kernel<<<limbs::grid_for(rows * kb / 8), 256, 0, stream>>>(packed, rows, pb, pb, b, 3 * kb, kb, kb);
+  return f32_product(x, nullptr, b, scale, bias, y, m, rows, cols, a, partial, stream);
 }
 
+size_t f32_dgrad_workspace(int64_t m, int64_t rows, int64_t cols) { return f32_product_workspace(m, cols, rows); }
+
 // dx [m, cols] fp32 = dy @ (row_scale * sign) through the limbs: dy scaled
-// by the row scale along K, the signs transposed (bits along K); over chunks
-// of f32_chunk_rows rows of dy.
+// by the row scale along K, the signs transposed (bits along K).
 int mfma_f32_dgrad(const float* dy, const uint8_t* packed, const float* row_scale, float* dx, int64_t m,
                    int64_t rows, int64_t cols, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   const size_t need = f32_dgrad_workspace(m, rows, cols);
-  if (need == 0 || !workspace || workspace_bytes < need) return 1;
-  const int64_t k3 = 3 * rows, kb = rows / 8, mc = f32_chunk_rows(m, rows);
-  if (!fits32(mc * k3 * 2) || !fits32(cols * k3 / 8)) return 1;
+  if (need == 0 || !workspace || workspace_bytes < need || !aligned16(workspace)) return 1;
+  const int64_t kp = up64(rows), kb = kp / 8, mc = f32_chunk_rows(m, rows);
+  if (!fits32(mc * 3 * kp * 2) || !fits32(cols * 3 * kb)) return 1;
   uint16_t* a = static_cast<uint16_t*>(workspace);
-  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(mc) * k3 * 2);
-  // the transposed signs into plane 0 of each row of b (its pitch 3 * kb is
-  // a multiple of 8 as rows % 64 == 0), then repeated into planes 1 and 2
-  int rc = launch_transpose_bits(packed, b, rows, cols, (cols + 7) / 8, 3 * kb, stream);
+  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(mc) * 3 * kp * 2);
+  float* partial = reinterpret_cast<float*>(b + limbs::up256(static_cast<size_t>(cols) * 3 * kb));
+  // the transposed signs into plane 0 of each row of b (zero past `rows`),
+  // then repeated into planes 1 and 2
+  const int rc = launch_transpose_bits(packed, b, rows, cols, (cols + 7) / 8, 3 * kb, stream);
   if (rc) return rc;
-  limbs::repeat_kernel<<<limbs::grid_for(cols * kb), 256, 0, stream>>>(b, cols, kb, 3 * kb, b, 3 * kb, kb);
-  for (int64_t i0 = 0; i0 < m; i0 += mc) {
-    const int64_t mi = m - i0 < mc ? m - i0 : mc;
-    limbs::split_kernel<<<limbs::grid_for(mi * rows), 256, 0, stream>>>(dy + i0 * rows, mi, rows, nullptr, row_scale,
-                                                                        a, k3, rows);
-    mfma::Params p{};
-    p.a = a;
-    p.bits = b;
-    p.out = dx + i0 * cols;
-    p.M = mi; p.N = cols; p.K = k3;
-    p.lda = k3; p.pb = 3 * kb;
-    p.a_rows = mi; p.bit_rows = cols;
-    mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD_F32, QSTE_BF16>
-        <<<wide_grid(mi, cols), mfma::wide::THREADS, 0, stream>>>(p);
-    if ((rc = static_cast<int>(hipGetLastError()))) return rc;
-  }
-  return 0;
+  limbs::repeat_kernel<<<limbs::grid_for(cols * kb / 8), 256, 0, stream>>>(b, cols, kb, 3 * kb, b, 3 * kb, kb, kb);
+  return f32_product(dy, row_scale, b, nullptr, nullptr, dx, m, cols, rows, a, partial, stream);
+}
+
+// Whether the evidence takes the limbs; its K is the samples.  From 128 rows
+// and for whole 64-column tiles always; ragged ones by the same kind of
+// estimate (scalar / limbs: 256 samples of 1000 x 1000 36 / 45, 512 of 300 x
+// 300 64 / 59, 2048 of 1000 x 3000 407 / 156).
+static bool f32_evidence_worth(int64_t samples, int64_t rows, int64_t cols) {
+  if (rows % 64 == 0 && cols % 64 == 0) return rows >= 128;
+  const double flops = 2.0 * static_cast<double>(samples) * rows * cols;
+  const double chain = 4.0 + 0.118 * samples, rate = flops / 42e6, limb_chain = 0.058 * samples,
+               limb_rate = flops / 400e6;
+  return (chain > rate ? chain : rate) > 30.0 + (limb_chain > limb_rate ? limb_chain : limb_rate);
 }
 
 size_t f32_evidence_workspace(int64_t samples, int64_t rows, int64_t cols) {
-  if (samples <= 0 || rows <= 0 || cols <= 0 || rows % 64 != 0 || cols % 64 != 0 || !f32_limbs_worth(rows))
-    return 0;
+  if (samples <= 0 || rows <= 0 || cols <= 0 || !f32_evidence_worth(samples, rows, cols)) return 0;
   // K is the samples here: the fused epilogue needs the whole sum in one
   // pass, so a product whose limbs exceed the budget is not split up
-  const size_t a = static_cast<size_t>(3 * samples) * rows * 2;
+  const size_t a = static_cast<size_t>(3 * samples) * up64(rows) * 2;
   if (a > kLimbBudget) return 0;
-  return limbs::up256(a) + limbs::up256(static_cast<size_t>(3 * samples) * (cols / 8));
+  return limbs::up256(a) + limbs::up256(static_cast<size_t>(3 * samples) * (up64(cols) / 8)) +
+         (cols % 64 ? limbs::up256(static_cast<size_t>(rows) * ((cols + 127) / 128 * 16)) : 0);
 }
+
+int launch_pad_rows(const void*, void*, int64_t, int64_t, int64_t, hipStream_t);
 
 // The evidence of fp32 dy through the limbs: dy scaled by the sample scale,
 // its limbs stacked along the samples (rows of K), the sample signs repeated
@@ -1643,16 +1752,25 @@ int mfma_f32_evidence(const float* dy, const uint8_t* packed_x, const float* x_s
                       int64_t rows, int64_t cols, const float* m_add, const float* m_scale, const uint8_t* w_bits,
                       float* gs_partial, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   const size_t need = f32_evidence_workspace(samples, rows, cols);
-  if (need == 0 || !workspace || workspace_bytes < need) return 1;
-  const int64_t k3 = 3 * samples, cb = cols / 8;
-  if (!fits32(k3 * rows * 2) || !fits32(k3 * cb)) return 1;
+  if (need == 0 || !workspace || workspace_bytes < need || !aligned16(workspace)) return 1;
+  const int64_t k3 = 3 * samples, rp = up64(rows), cb = up64(cols) / 8, pb = (cols + 7) / 8;
+  if (!fits32(k3 * rp * 2) || !fits32(k3 * cb)) return 1;
   uint16_t* a = static_cast<uint16_t*>(workspace);
-  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(k3) * rows * 2);
-  limbs::split_kernel<<<limbs::grid_for(samples * rows), 256, 0, stream>>>(dy, samples, rows, x_scale, nullptr, a,
-                                                                          rows, samples * rows);
-  limbs::repeat_kernel<<<limbs::grid_for(samples * cb), 256, 0, stream>>>(packed_x, samples, cb, cb, b, cb,
-                                                                         samples * cb);
+  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(k3) * rp * 2);
+  limbs::split_kernel<<<limbs::grid_for(samples * rp / 4), 256, 0, stream>>>(dy, samples, rows, x_scale, nullptr, a,
+                                                                             rp, samples * rp, rp);
+  limbs::repeat_kernel<<<limbs::grid_for(samples * cb / 8), 256, 0, stream>>>(packed_x, samples, pb, pb, b, cb,
+                                                                             samples * cb, cb);
   mfma::Params p = evidence_params(a, b, nullptr, ev, k3, rows, cols, m_add, m_scale, w_bits, gs_partial);
+  p.lda = rp;
+  p.pb = cb;
+  if (cols % 64 != 0 && w_bits) {  // the epilogue reads the signs of W in whole dwords
+    uint8_t* wp = b + limbs::up256(static_cast<size_t>(k3) * cb);
+    p.w_pb = (cols + 127) / 128 * 16;
+    const int rc = launch_pad_rows(w_bits, wp, rows, pb, p.w_pb, stream);
+    if (rc) return rc;
+    p.w_bits = wp;
+  }
   mfma::wide::wide_kernel<mfma::A_ROWS_K, mfma::B_BITS_ALONG_N, mfma::EPI_EVIDENCE, QSTE_BF16>
       <<<wide_grid(rows, cols), mfma::wide::THREADS, 0, stream>>>(p);
   return static_cast<int>(hipGetLastError());

@@ -143,3 +143,52 @@ def test_offset_dot_is_taken():
     assert rel(ev2.cpu().numpy(), ev.cpu().numpy()) <= 1e-6 and rel(gs2.cpu().numpy(), gs.cpu().numpy()) <= 1e-4
     _, ev3, _, _ = kernels.linear_backward(*args, need_bias=False, offset_dot=dot + 1)
     assert rel(ev3.cpu().numpy(), ev.cpu().numpy()) > 1e-3
+
+
+F32 = [(300, 300, 24), (2048, 2048, 24), (65, 1000, 700), (1000, 1001, 600), (1001, 1000, 64), (4100, 130, 130),
+       (256, 256, 256), (300, 300, 1300)]
+
+
+@pytest.mark.parametrize("rows,cols,m", F32)
+@pytest.mark.parametrize("need_input", [True, False])
+def test_fp32_layer(rows, cols, m, need_input):
+    """fp32 layers of few rows, odd sizes and few output tiles (K in ranges):
+    exact limb products, so only fp32 sums of up to 3 * 4100 terms and the
+    scale's rounding separate them from the oracle (1e-6 in the 2-norm)."""
+
+    from qste_amd import kernels
+
+    print(f"fp32 {rows}x{cols} m={m}", flush=True)
+    rng = np.random.default_rng(rows + cols + m)
+    packed = oracle.pack_coordinate(rng.integers(-127, 128, size=(rows, cols)).astype(np.int8))
+    x = rng.standard_normal((m, cols)).astype(np.float32)
+    dy = rng.standard_normal((m, rows)).astype(np.float32)
+    scale = (np.abs(rng.standard_normal(rows)) * 0.02 + 0.01).astype(np.float32)
+    bias = (rng.standard_normal(rows) * 0.1).astype(np.float32)
+    y = kernels.packed_linear_affine(t(x), t(packed), t(scale), t(bias), cols).cpu().numpy()
+    assert rel(y, oracle.linear_fwd(x, packed, scale, bias, cols)) <= 1e-6
+    xbits, off, xs = oracle.pack_affine_rows(x)
+    dx, ev, gs, db = kernels.linear_backward(t(dy), t(xbits), t(off), t(xs), t(packed), t(scale), cols,
+                                             need_bias=True, need_input=need_input)
+    e0 = oracle.evidence(dy, xbits, cols, xs) + oracle.offset_correction(dy, off)[:, None]
+    assert rel(ev.cpu().numpy(), e0 * scale[:, None]) <= 1e-6
+    assert rel(gs.cpu().numpy(), oracle.row_inner(e0.astype(np.float32), packed, cols)) <= 1e-4
+    assert rel(db.cpu().numpy(), dy.astype(np.float64).sum(0)) <= 1e-6
+    if need_input:
+        assert rel(dx.cpu().numpy(), oracle.linear_dgrad(dy, packed, cols, scale)) <= 1e-6
+
+
+@pytest.mark.parametrize("rows,cols,m", [(6400, 256, 257), (4097, 130, 300), (16384, 512, 64)])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_input_gradient_in_ranges(rows, cols, m, dt):
+    """Few dX tiles over many rows: K in ranges, combined (one rounding)."""
+
+    from qste_amd import kernels
+
+    packed, x, dy, scale, _ = problem(rows, cols, m, dt, rows + m)
+    xbits, off, xs = oracle.pack_affine_rows(x)
+    dx, _, _, _ = kernels.linear_backward(t(dy, DT[dt]), t(xbits), t(off), t(xs), t(packed), t(scale), cols,
+                                          need_bias=False)
+    want = rnd(oracle.linear_dgrad(dy, packed, cols, rnd(scale, dt)), dt)
+    got = dx.float().cpu().numpy()
+    assert rel(got, want) <= 1e-3 and np.mean(got != want) < 0.02
