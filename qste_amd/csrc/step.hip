@@ -24,7 +24,8 @@
 //   final    (prologue: step size 1/rms(m) * lr) stochastic rounding, momentum
 //            requantization, sign repack and flip count, 8 columns (one
 //            packed byte) per thread
-//   finish   new block scales into place, flip total
+//   finish   new block scales into place, flip total (the row path's final
+//            pass does both itself)
 //
 // Float semantics follow the specification operation by operation: every
 // element-wise product and sum rounds in fp32 (this file is compiled with
@@ -51,7 +52,7 @@ namespace qste {
 namespace step {
 
 constexpr int kThreads = 256;
-constexpr int kStrip = 64;        // rows per stats workgroup
+constexpr int kStrip = 64;        // rows per stats workgroup at most
 constexpr int kColChunk = 1024;   // columns per stats workgroup (4 per thread)
 constexpr int kUsqGroups = 1024;
 constexpr int kMomentGroups = kUsqGroups;  // the momentum partials share the usq layout
@@ -105,6 +106,7 @@ struct Work {
   float* s_rcp;        // [blocks] 1 / max(s_new, 1e-12), correctly rounded (row path)
   int64_t* flips_part; // [kFinalGroups]
   int64_t nstrips, nchunks;
+  int strip;           // rows per stats workgroup off the row path (<= kStrip)
   int64_t parts;       // slots of usq_part and msq_part written (<= kUsqGroups)
   int64_t fparts;      // slots of flips_part written (<= kFinalGroups)
 };
@@ -205,9 +207,9 @@ __global__ __launch_bounds__(kThreads) void stats_kernel(const float* __restrict
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int64_t chunk = blockIdx.x;
-  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * kStrip;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * w.strip;
   const int64_t c0 = chunk * kColChunk + threadIdx.x * 4;
-  const int rows_here = static_cast<int>(p.rows - r0 < kStrip ? p.rows - r0 : kStrip);
+  const int rows_here = static_cast<int>(p.rows - r0 < w.strip ? p.rows - r0 : w.strip);
   double col_acc[4] = {0.0, 0.0, 0.0, 0.0};
   const bool full4 = p.vec && c0 + 4 <= p.cols;
   for (int rr0 = 0; rr0 < rows_here; rr0 += 4) {
@@ -271,8 +273,9 @@ __global__ __launch_bounds__(kThreads) void stats_kernel(const float* __restrict
 // statistic (finished by the next pass).
 __global__ __launch_bounds__(kThreads) void colrow_kernel(uint16_t* __restrict__ col_v,
                                                           uint16_t* __restrict__ row_v, Params p, Work w,
-                                                          int col_groups) {
+                                                          int col_groups, int64_t* flips_out) {
   const bool on = enabled(p);
+  if (blockIdx.x == 0 && threadIdx.x == 0 && flips_out) *flips_out = 0;  // the row path's final pass adds to it
   if (static_cast<int>(blockIdx.x) >= col_groups) {
     __shared__ double red[kThreads / kWave];
     const int64_t group = static_cast<int64_t>(blockIdx.x) - col_groups;
@@ -299,8 +302,20 @@ __global__ __launch_bounds__(kThreads) void colrow_kernel(uint16_t* __restrict__
   const int cl = threadIdx.x & 15, sg = threadIdx.x >> 4;
   const int64_t c = blockIdx.x * 16ll + cl;
   double s = 0.0;
-  if (c < p.cols)
-    for (int64_t k = sg; k < w.nstrips; k += 16) s += w.col_part[k * p.cols + c];
+  if (c < p.cols) {
+    // eight strips' loads in flight: one at a time the 64 of a thread at 1024
+    // strips were a chain of L2 latencies (22 us at 3072 x 768)
+    constexpr int kBatch = 8;
+    int64_t k = sg;
+    for (; k + 16 * (kBatch - 1) < w.nstrips; k += 16 * kBatch) {
+      double v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) v[u] = w.col_part[(k + 16 * u) * p.cols + c];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) s += v[u];
+    }
+    for (; k < w.nstrips; k += 16) s += w.col_part[k * p.cols + c];
+  }
   part[sg][cl] = s;
   __syncthreads();
   if (threadIdx.x < 16 && c < p.cols) {
@@ -598,6 +613,52 @@ __global__ __launch_bounds__(kThreads) void elem_row_kernel(const float* __restr
                                                             const uint16_t* __restrict__ moment_scale,
                                                             Params p, Work w) {
   __shared__ double red[kThreads / kWave];
+  const bool with_m = MOMENT || p.spec;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int64_t chunk = blockIdx.y;
+  const int64_t c0 = chunk * kRowChunk;
+  const int ns = chunk_slots(p.cols, c0);
+  const int gsize = static_cast<int>(p.block_size >> 2);  // lanes per momentum block
+  // loads are unconditional (straight-line code keeps the compiler's waits
+  // per load): slots past the chunk's end re-read its last slot, rows past
+  // the end the last row, and those results are dropped
+  int64_t sc[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) sc[k] = c0 + 4 * lane + 256 * (k < ns ? k : ns - 1);
+  struct RowIn {
+    float4 v[4];
+    uint32_t q4[4];
+    uint16_t so[4];
+    float row;  // the row factor (MOMENT) or the new row statistic
+  };
+  auto load_row = [&](int64_t r, RowIn& in) {
+    const int64_t rb = r * p.cols;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      in.v[k] = *reinterpret_cast<const float4*>(g + rb + sc[k]);
+      if (with_m) {
+        in.q4[k] = *reinterpret_cast<const uint32_t*>(moment_q + rb + sc[k]);
+        in.so[k] = moment_scale[(rb + sc[k]) >> p.block_shift];
+      } else {
+        in.q4[k] = 0u;
+        in.so[k] = 0;
+      }
+    }
+    in.row = MOMENT ? w.row_factor[r] : w.new_row[r];
+  };
+  const int64_t rstep = static_cast<int64_t>(gridDim.x) * (kThreads / kWave);
+  int64_t r = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + wave;
+  // The first row is loaded before the prologue sums the partials of the pass
+  // before (a chain of latencies of its own), except where the prologue may
+  // find that there is nothing to do.
+  const int64_t r_first = r < p.rows ? r : p.rows - 1;
+  RowIn cur;
+  const bool early = !(MOMENT && p.spec);
+  if (early) {
+    load_row(r_first, cur);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   float divisor = 1.0f, sqrt_mean = 0.0f;
   if (MOMENT) {
     divisor = divisor_of(w.usq_part, w.parts, p.count, p.clip, red);
@@ -606,54 +667,28 @@ __global__ __launch_bounds__(kThreads) void elem_row_kernel(const float* __restr
   } else {
     sqrt_mean = sqrt_mean_of(p, w, red);
   }
-  const bool with_m = MOMENT || p.spec;
+  if (!early) load_row(r_first, cur);
   const float rdiv = 1.0f / divisor;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int64_t chunk = blockIdx.y;
-  const int64_t c0 = chunk * kRowChunk;
-  const int ns = chunk_slots(p.cols, c0);
-  const int gsize = static_cast<int>(p.block_size >> 2);  // lanes per momentum block
-  // loads are unconditional (straight-line code keeps the compiler's waits
-  // per load): slots past the chunk's end re-read its last slot, and those
-  // results are dropped
-  int64_t sc[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) sc[k] = c0 + 4 * lane + 256 * (k < ns ? k : ns - 1);
   float4 cf[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) cf[k] = *reinterpret_cast<const float4*>(w.col_factor + sc[k]);
   double acc = 0.0, msq = 0.0;
-  const int64_t rstep = static_cast<int64_t>(gridDim.x) * (kThreads / kWave);
-  for (int64_t r = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + wave; r < p.rows; r += rstep) {
-    float rf;
-    if (MOMENT) {
-      rf = w.row_factor[r];
-    } else {
-      rf = row_factor_of(sqrt_mean, w.new_row[r]);
+  for (; r < p.rows; r += rstep) {
+    RowIn nxt;  // the last row re-reads itself (a cache hit) rather than branch
+    load_row(r + rstep < p.rows ? r + rstep : r, nxt);
+    __builtin_amdgcn_sched_barrier(0);  // in flight during this row's arithmetic
+    float rf = cur.row;
+    if (!MOMENT) {
+      rf = row_factor_of(sqrt_mean, cur.row);
       if (chunk == 0 && lane == 0) w.row_factor[r] = rf;
     }
     const int64_t rb = r * p.cols;
-    float4 v[4];
-    uint32_t q4[4];
-    float so[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      v[k] = *reinterpret_cast<const float4*>(g + rb + sc[k]);
-      if (with_m) {
-        q4[k] = *reinterpret_cast<const uint32_t*>(moment_q + rb + sc[k]);
-        so[k] = f16_to_f32(moment_scale[(rb + sc[k]) >> p.block_shift]);
-      } else {
-        q4[k] = 0u;
-        so[k] = 0.f;
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);  // every load issued before the arithmetic
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       if (k >= ns) break;
-      const float gv[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+      const float gv[4] = {cur.v[k].x, cur.v[k].y, cur.v[k].z, cur.v[k].w};
       const float cv[4] = {cf[k].x, cf[k].y, cf[k].z, cf[k].w};
+      const float s_old = f16_to_f32(cur.so[k]);
       float uu[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -669,8 +704,8 @@ __global__ __launch_bounds__(kThreads) void elem_row_kernel(const float* __restr
         float amax = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float prev = static_cast<float>(static_cast<int8_t>(q4[k] >> (8 * e)));
-          const float m = moment_of(uu[e], prev, so[k], p);
+          const float prev = static_cast<float>(static_cast<int8_t>(cur.q4[k] >> (8 * e)));
+          const float m = moment_of(uu[e], prev, s_old, p);
           amax = fmaxf(amax, fabsf(m));
           const float sq = m * m;
           msq += static_cast<double>(sq);
@@ -684,6 +719,7 @@ __global__ __launch_bounds__(kThreads) void elem_row_kernel(const float* __restr
         }
       }
     }
+    cur = nxt;
   }
   const int64_t slot = chunk * gridDim.x + blockIdx.x;
   if (!MOMENT) {
@@ -973,59 +1009,62 @@ __global__ __launch_bounds__(kThreads) void final_vec_kernel(const float* __rest
 // The same arithmetic as final_byte.
 constexpr int kFinalChunk = 512;
 
+struct FinalRowIn {
+  float4 ga, gb;
+  uint64_t q8, c8;
+  uint32_t old_byte;
+  float rf, s_old, rdec;
+  uint16_t s_new;
+};
+
+// This lane's byte of row r: loads are unconditional (straight-line code keeps
+// the compiler's waits per load); idle lanes read their row's last byte, rows
+// past the end the last row, and those results are dropped.
+__device__ __forceinline__ void load_final_row(const float* __restrict__ g, const int8_t* coord,
+                                               const uint8_t* packed, const int8_t* moment_q,
+                                               const uint16_t* moment_scale, const Params& p, const Work& w, int64_t r,
+                                               int64_t cc, FinalRowIn& in) {
+  const int64_t i0 = r * p.cols + cc;
+  in.ga = *reinterpret_cast<const float4*>(g + i0);
+  in.gb = *reinterpret_cast<const float4*>(g + i0 + 4);
+  in.q8 = *reinterpret_cast<const uint64_t*>(moment_q + i0);
+  in.c8 = *reinterpret_cast<const uint64_t*>(coord + i0);
+  in.old_byte = packed[r * (p.cols >> 3) + (cc >> 3)];
+  in.rf = w.row_factor[r];
+  const int64_t blk = i0 >> p.block_shift;  // block_size >= 8: one block for the byte
+  in.s_old = f16_to_f32(moment_scale[blk]);
+  in.s_new = w.s_new[blk];
+  in.rdec = w.s_rcp[blk];
+}
+
 template <bool DIV1>
 __device__ __forceinline__ int64_t final_row_loop(const float* __restrict__ g, int8_t* __restrict__ coord,
                                                   uint8_t* __restrict__ packed, int8_t* __restrict__ moment_q,
-                                                  const uint16_t* __restrict__ moment_scale, const Params& p,
-                                                  const Work& w, float divisor, float rdiv, float step_size,
-                                                  uint32_t combined, bool on) {
+                                                  uint16_t* moment_scale, const Params& p, const Work& w,
+                                                  const FinalScalars& f, FinalRowIn cur, int64_t r, int64_t c0) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * kFinalChunk + 8 * lane;
+  // first lane of its momentum block (block_size / 8 lanes of this wave)
+  const bool block_lead = (lane & ((1 << (p.block_shift - 3)) - 1)) == 0;
   const bool lane_on = c0 < p.cols;
-  const int64_t stride = p.cols >> 3;
+  const int64_t cc = lane_on ? c0 : p.cols - 8;
+  const float divisor = f.divisor, rdiv = f.rdiv, step_size = f.step_size;
+  const uint32_t combined = f.combined;
   float cv[8];
   {
-    const int64_t cl = lane_on ? c0 : p.cols - 8;
-    const float4 ca = *reinterpret_cast<const float4*>(w.col_factor + cl);
-    const float4 cb = *reinterpret_cast<const float4*>(w.col_factor + cl + 4);
+    const float4 ca = *reinterpret_cast<const float4*>(w.col_factor + cc);
+    const float4 cb = *reinterpret_cast<const float4*>(w.col_factor + cc + 4);
     cv[0] = ca.x; cv[1] = ca.y; cv[2] = ca.z; cv[3] = ca.w; cv[4] = cb.x; cv[5] = cb.y; cv[6] = cb.z; cv[7] = cb.w;
   }
   int64_t flips = 0;
   const int64_t rstep = static_cast<int64_t>(gridDim.x) * (kThreads / kWave);
-  // loads are unconditional (straight-line code keeps the compiler's waits
-  // per load): idle lanes read their row's last byte, rows past the end the
-  // last row, and those results are dropped
-  const int64_t cc = lane_on ? c0 : p.cols - 8;
-  struct RowIn {
-    float4 ga, gb;
-    uint64_t q8, c8;
-    uint32_t old_byte;
-    float rf, s_old, decode, rdec;
-  };
-  auto load_row = [&](int64_t r, RowIn& in) {
-    const int64_t i0 = r * p.cols + cc;
-    in.ga = *reinterpret_cast<const float4*>(g + i0);
-    in.gb = *reinterpret_cast<const float4*>(g + i0 + 4);
-    in.q8 = *reinterpret_cast<const uint64_t*>(moment_q + i0);
-    in.c8 = *reinterpret_cast<const uint64_t*>(coord + i0);
-    in.old_byte = packed[r * stride + (cc >> 3)];
-    in.rf = w.row_factor[r];
-    const int64_t blk = i0 >> p.block_shift;  // block_size >= 8: one block for the byte
-    in.s_old = f16_to_f32(moment_scale[blk]);
-    in.decode = fmaxf(f16_to_f32(w.s_new[blk]), 1e-12f);
-    in.rdec = w.s_rcp[blk];
-  };
-  int64_t r = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + wave;
-  RowIn cur;
-  load_row(r < p.rows ? r : 0, cur);
   for (; r < p.rows; r += rstep) {
     // the next row's loads in flight during this row's arithmetic; the last
     // row re-reads itself (a cache hit) rather than branch
-    RowIn nxt;
-    load_row(r + rstep < p.rows ? r + rstep : r, nxt);
+    FinalRowIn nxt;
+    load_final_row(g, coord, packed, moment_q, moment_scale, p, w, r + rstep < p.rows ? r + rstep : r, cc, nxt);
     __builtin_amdgcn_sched_barrier(0);
     const int64_t i0 = r * p.cols + cc;
+    const float decode = fmaxf(f16_to_f32(cur.s_new), 1e-12f);
     const uint32_t head = scramble_head(static_cast<uint32_t>(i0) ^ combined);
     const float gv[8] = {cur.ga.x, cur.ga.y, cur.ga.z, cur.ga.w, cur.gb.x, cur.gb.y, cur.gb.z, cur.gb.w};
     uint32_t byte = 0, cn_lo = 0, cn_hi = 0, qn_lo = 0, qn_hi = 0;
@@ -1043,7 +1082,7 @@ __device__ __forceinline__ int64_t final_row_loop(const float* __restrict__ g, i
       const float frac = target - lower;
       float rounded = lower + (uu < frac ? 1.0f : 0.0f);
       rounded = fminf(127.0f, fmaxf(-127.0f, rounded));
-      float q = rintf(div_by(m, cur.decode, cur.rdec));
+      float q = rintf(div_by(m, decode, cur.rdec));
       q = fminf(127.0f, fmaxf(-127.0f, q));
       const uint32_t cb8 = static_cast<uint32_t>(static_cast<uint8_t>(static_cast<int8_t>(rounded)));
       const uint32_t qb8 = static_cast<uint32_t>(static_cast<uint8_t>(static_cast<int8_t>(q)));
@@ -1057,10 +1096,14 @@ __device__ __forceinline__ int64_t final_row_loop(const float* __restrict__ g, i
       byte |= (rounded >= 0.0f ? 1u : 0u) << j;
     }
     if (lane_on) {
-      if (on) {
+      if (f.on) {
         *reinterpret_cast<uint64_t*>(coord + i0) = (static_cast<uint64_t>(cn_hi) << 32) | cn_lo;
         *reinterpret_cast<uint64_t*>(moment_q + i0) = (static_cast<uint64_t>(qn_hi) << 32) | qn_lo;
-        packed[r * stride + (cc >> 3)] = static_cast<uint8_t>(byte);
+        packed[r * (p.cols >> 3) + (cc >> 3)] = static_cast<uint8_t>(byte);
+        // the block lies in this wave's row chunk: its old scale was read by
+        // this wave alone, with the row (a prefetch of the same last row
+        // again is dropped)
+        if (block_lead) moment_scale[i0 >> p.block_shift] = cur.s_new;
       }
       flips += __popc(cur.old_byte ^ byte);
     }
@@ -1073,21 +1116,25 @@ __global__ __launch_bounds__(kThreads) void final_row_kernel(const float* __rest
                                                              int8_t* __restrict__ coord,
                                                              uint8_t* __restrict__ packed,
                                                              int8_t* __restrict__ moment_q,
-                                                             const uint16_t* __restrict__ moment_scale,
+                                                             uint16_t* moment_scale, int64_t* flips_out,
                                                              Params p, Work w) {
   __shared__ double red[kThreads / kWave];
   __shared__ int64_t ired[kThreads / kWave];
+  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * kFinalChunk + 8 * (threadIdx.x & (kWave - 1));
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave;
+  // the first row in flight while the prologue sums the momentum's partials
+  FinalRowIn first;
+  load_final_row(g, coord, packed, moment_q, moment_scale, p, w, r < p.rows ? r : p.rows - 1,
+                 c0 < p.cols ? c0 : p.cols - 8, first);
+  __builtin_amdgcn_sched_barrier(0);
   const FinalScalars f = final_prologue(p, w, red);
-  const float step_size = f.step_size, divisor = f.divisor, rdiv = f.rdiv;
-  const uint32_t combined = f.combined;
-  const bool on = f.on;
-  const int64_t flips =
-      divisor == 1.0f
-          ? final_row_loop<true>(g, coord, packed, moment_q, moment_scale, p, w, divisor, rdiv, step_size, combined, on)
-          : final_row_loop<false>(g, coord, packed, moment_q, moment_scale, p, w, divisor, rdiv, step_size, combined,
-                                  on);
+  const int64_t flips = f.divisor == 1.0f
+                            ? final_row_loop<true>(g, coord, packed, moment_q, moment_scale, p, w, f, first, r, c0)
+                            : final_row_loop<false>(g, coord, packed, moment_q, moment_scale, p, w, f, first, r, c0);
   const int64_t total = block_sum(flips, ired);
-  if (threadIdx.x == 0) w.flips_part[static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x] = on ? total : 0;
+  // whole numbers: the order of the additions does not show
+  if (threadIdx.x == 0 && f.on && total != 0 && flips_out)
+    atomicAdd(reinterpret_cast<unsigned long long*>(flips_out), static_cast<unsigned long long>(total));
 }
 
 __global__ __launch_bounds__(kThreads) void finish_kernel(uint16_t* __restrict__ moment_scale,
@@ -1955,20 +2002,34 @@ int launch_coordinate_update(const float* g, int8_t* coord, uint8_t* packed, int
   // row path: whole 256-column slots, momentum blocks inside one slot, and
   // at least one usq workgroup per chunk
   const bool row_path = p.vec && cols % 256 == 0 && block_size <= 256 && w.nchunks <= kUsqGroups;
-  const unsigned row_groups = static_cast<unsigned>(kUsqGroups / w.nchunks);
-  w.parts = row_path ? static_cast<int64_t>(row_groups) * w.nchunks : kUsqGroups;
+  // workgroups per chunk: four rows a wave, but one workgroup per CU at least
+  // and kUsqGroups in all at most.  Every pass starts by summing the partials
+  // of the one before, so a small surface in 1024 workgroups of a row a wave
+  // spends its time there (3072 x 768: 56 us in six launches, 35-36 in these five; 50257 x
+  // 768: 203 -> 174, 512 x 512: 45 -> 21)
+  const int64_t most = kUsqGroups / w.nchunks, least = most / 4 > 0 ? most / 4 : 1, four = (rows + 15) / 16;
+  const unsigned row_groups = static_cast<unsigned>(four < least ? least : (four < most ? four : most));
+  // off the row path: a workgroup per row, or four momentum blocks a workgroup
+  const int64_t quads = ceil_div(p.blocks, kThreads / kWave), units = rows > quads ? rows : quads;
+  const unsigned any_groups = static_cast<unsigned>(units < kUsqGroups ? units : kUsqGroups);
+  w.parts = row_path ? static_cast<int64_t>(row_groups) * w.nchunks : any_groups;
 
   int rc;
   if (row_path) {
     w.nstrips = row_groups;
     stats_row_kernel<<<dim3(row_groups, static_cast<unsigned>(w.nchunks)), kThreads, 0, stream>>>(g, row_v, p, w);
   } else {
+    // strips short enough for a workgroup per CU (300 x 1000 in strips of 64
+    // rows: five workgroups)
+    w.strip = kStrip;
+    while (w.strip > 4 && ceil_div(rows, w.strip) * w.nchunks < 256) w.strip /= 2;
+    w.nstrips = ceil_div(rows, w.strip);
     stats_kernel<<<dim3(static_cast<unsigned>(w.nchunks), static_cast<unsigned>(w.nstrips)), kThreads, 0, stream>>>(
         g, row_v, p, w);
   }
   if ((rc = static_cast<int>(hipGetLastError()))) return rc;
   const int col_groups = ceil_div(cols, 16);
-  colrow_kernel<<<col_groups + kRowsGroups, kThreads, 0, stream>>>(col_v, row_v, p, w, col_groups);
+  colrow_kernel<<<col_groups + kRowsGroups, kThreads, 0, stream>>>(col_v, row_v, p, w, col_groups, flips_out);
   if ((rc = static_cast<int>(hipGetLastError()))) return rc;
   if (row_path) {
     const dim3 grid(row_groups, static_cast<unsigned>(w.nchunks));
@@ -1976,9 +2037,9 @@ int launch_coordinate_update(const float* g, int8_t* coord, uint8_t* packed, int
     if ((rc = static_cast<int>(hipGetLastError()))) return rc;
     elem_row_kernel<true><<<grid, kThreads, 0, stream>>>(g, moment_q, moment_scale, p, w);
   } else {
-    usq_kernel<<<kUsqGroups, kThreads, 0, stream>>>(g, moment_q, moment_scale, p, w);
+    usq_kernel<<<any_groups, kThreads, 0, stream>>>(g, moment_q, moment_scale, p, w);
     if ((rc = static_cast<int>(hipGetLastError()))) return rc;
-    moment_kernel<<<kMomentGroups, kThreads, 0, stream>>>(g, moment_q, moment_scale, p, w);
+    moment_kernel<<<any_groups, kThreads, 0, stream>>>(g, moment_q, moment_scale, p, w);
   }
   if ((rc = static_cast<int>(hipGetLastError()))) return rc;
   const int64_t fchunks = (cols + kFinalChunk - 1) / kFinalChunk;
@@ -1986,17 +2047,23 @@ int launch_coordinate_update(const float* g, int8_t* coord, uint8_t* packed, int
   // as many workgroups as the device holds at once (one round, no tail),
   // at most kFinalGroups in all
   const int64_t fit = resident_final_groups();
-  const int64_t per_chunk = (fit > 0 ? (fit < kFinalGroups ? fit : kFinalGroups) : kFinalGroups) / fchunks;
+  int64_t per_chunk = (fit > 0 ? (fit < kFinalGroups ? fit : kFinalGroups) : kFinalGroups) / fchunks;
+  // (and, as above, four rows a wave, or a workgroup per CU: with up to 2048
+  // workgroups of a row a wave 3072 x 768 took 7 us longer)
+  const int64_t least_final = 256 / fchunks > 0 ? 256 / fchunks : 1, enough = four > least_final ? four : least_final;
+  if (final_rows && per_chunk > enough) per_chunk = enough;
   const unsigned final_groups = static_cast<unsigned>(per_chunk > 0 ? per_chunk : 1);
-  w.fparts = final_rows ? static_cast<int64_t>(final_groups) * fchunks : kFinalGroups;
+  const int64_t bytes = rows * ((cols + 7) / 8), threads = ceil_div(bytes, kThreads);
+  const unsigned byte_groups = static_cast<unsigned>(threads < kFinalGroups ? threads : kFinalGroups);
+  w.fparts = byte_groups;
   if (final_rows)
     final_row_kernel<<<dim3(final_groups, static_cast<unsigned>(fchunks)), kThreads, 0, stream>>>(
-        g, coord, packed, moment_q, moment_scale, p, w);
+        g, coord, packed, moment_q, moment_scale, flips_out, p, w);
   else if (p.vec)
-    final_vec_kernel<<<kFinalGroups, kThreads, 0, stream>>>(g, coord, packed, moment_q, moment_scale, p, w);
+    final_vec_kernel<<<byte_groups, kThreads, 0, stream>>>(g, coord, packed, moment_q, moment_scale, p, w);
   else
-    final_kernel<<<kFinalGroups, kThreads, 0, stream>>>(g, coord, packed, moment_q, moment_scale, p, w);
-  if ((rc = static_cast<int>(hipGetLastError()))) return rc;
+    final_kernel<<<byte_groups, kThreads, 0, stream>>>(g, coord, packed, moment_q, moment_scale, p, w);
+  if ((rc = static_cast<int>(hipGetLastError())) || final_rows) return rc;
   finish_kernel<<<ceil_div(p.blocks, kThreads) < 1024 ? ceil_div(p.blocks, kThreads) : 1024, kThreads, 0,
                   stream>>>(moment_scale, flips_out, p, w);
   return static_cast<int>(hipGetLastError());
