@@ -208,11 +208,9 @@ constexpr int B_STAGE = BN * BK / 8;  // bytes: 256 rows x 8 B of sign bits
 // Each wave covers all 256 rows and a quarter of the columns: every sign
 // fragment it expands feeds 8 MFMAs (the expansion VALU work, not the LDS
 // reads of the dense operand, is what limits a wave).
-constexpr int WAVES_N = 4;            // waves across N, the rest across M
-constexpr int WAVES_M = 4 / WAVES_N;
-constexpr int WMR = BM / WAVES_M;     // rows per wave
+constexpr int WAVES_N = 4;            // the workgroup's waves, across N
 constexpr int WNC = BN / WAVES_N;     // columns per wave
-constexpr int MBN = WMR / 32, NBN = WNC / 32;  // 32 x 32 blocks per wave
+constexpr int NBN = WNC / 32;         // 32 x 32 blocks per wave across N
 constexpr int EPL = 2 * WNC + 16;     // bytes per staged output row (+ pad)
 constexpr int EPR = WNC == 128 ? 32 : 16;  // staged output rows per piece
 typedef __attribute__((address_space(3))) void lds_t;
@@ -241,11 +239,12 @@ __device__ __forceinline__ void stage_barrier() {
 // loads go through VGPRs one step before their stage is written.
 constexpr int LDB_N = BK + 8;
 constexpr int BN_STAGE = (BN / 8) * LDB_N;  // bytes
-template <int BKIND>
+template <int BKIND, int TM>
 struct Loads {
-  // buffer loads per wave per K step: 8 A loads, plus 2 direct bit loads
-  // (and 1 scale load), or 3 register loads of bits along N
-  static constexpr int value = BKIND == B_BITS_ALONG_K ? 10 : 11;
+  // buffer loads per wave per K step: a load per 32 rows of A, plus 2 direct
+  // bit loads (and 1 scale load), or 3 register loads of bits along N
+  static constexpr int a = TM / 32;
+  static constexpr int value = a + (BKIND == B_BITS_ALONG_K ? 2 : 3);
 };
 
 // A given as rows of K (evidence: A = dy^T, dy stored [K][M]) is staged
@@ -261,25 +260,31 @@ typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 // One output tile; the LDS stages are the caller's (one __shared__ array per
 // stage, so that the compiler tracks each stage's direct loads separately
 // and waits only where this code says).
-template <int AKIND, int BKIND, int EPI, int DT>
+// TM: rows of the tile, 256, or 128 for A as rows of M and bits along K
+// (half_kernel below).
+template <int AKIND, int BKIND, int EPI, int DT, int TM = BM>
 __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0, uint8_t* A1, uint8_t* A2,
                                           uint8_t* A3, uint8_t* B0, uint8_t* B1, uint8_t* B2, uint8_t* B3,
                                           uint16_t* Sc) {
-  constexpr int NL = Loads<BKIND>::value;
+  static_assert(TM == BM || (AKIND == A_ROWS_M && BKIND != B_BITS_ALONG_N && EPI != EPI_PARTIAL), "half tiles");
+  constexpr int NL = Loads<BKIND, TM>::value, NLA = Loads<BKIND, TM>::a;
+  constexpr int WMR = TM, MBN = WMR / 32;  // rows and 32 x 32 blocks per wave across M
+  constexpr int wm = 0;                    // every wave covers all the tile's rows
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int wn = wave;
   const int l32 = lane & 31, kg = lane >> 5;
-  const int tiles_m = static_cast<int>((p.M + BM - 1) / BM);
+  const int tiles_m = static_cast<int>((p.M + TM - 1) / TM);
   const int tiles_n = static_cast<int>((p.N + BN - 1) / BN);
   int tm, tn;
   tile_of<AKIND == A_ROWS_K ? 1 : 2>(pid, tiles_m, tiles_n, tm, tn);
-  const int64_t m0 = static_cast<int64_t>(tm) * BM, n0 = static_cast<int64_t>(tn) * BN;
+  const int64_t m0 = static_cast<int64_t>(tm) * TM, n0 = static_cast<int64_t>(tn) * BN;
   const uint32_t one = one_pair<DT>();
   const int nk = static_cast<int>((p.K + BK - 1) / BK);  // K % BK != 0 only for A as rows of K
 
   // A (rows of M, K contiguous): the buffer starts at row m0, so rows past
-  // M read zero.  Wave w fills rows 64w .. 64w+63 with 8 loads of 8 rows;
+  // M read zero.  Wave w fills rows 64w .. 64w+63 with 8 loads of 8 rows (of
+  // a half tile, 32w .. 32w+31 with 4);
   // lane -> row 8j + lane/8 and LDS chunk lane%8, which holds global chunk
   // (lane%8) ^ swz(row); swz depends on j only through its parity.
   // A as rows of K: the buffer starts at column m0, so k-rows past K read
@@ -292,7 +297,7 @@ __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0,
     const int q8 = lane >> 3, pos = lane & 7;
 #pragma unroll
     for (int par = 0; par < 2; ++par)
-      a_voff[par] = static_cast<uint32_t>((64 * wave + q8) * p.lda * 2 + 16 * (pos ^ (4 * par + (q8 >> 1))));
+      a_voff[par] = static_cast<uint32_t>((8 * NLA * wave + q8) * p.lda * 2 + 16 * (pos ^ (4 * par + (q8 >> 1))));
     a_row8 = static_cast<uint32_t>(8 * p.lda * 2);
   } else {
     ra = rsrc(p.a + m0, (p.a_rows * p.lda - m0) * 2);
@@ -340,9 +345,9 @@ __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0,
     }
     const uint32_t k_off = live ? static_cast<uint32_t>(it) * a_kstep : 0x80000000u;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (part >= 0 && (j >> 1) != part) continue;
-      uint8_t* dst = AKIND == A_ROWS_M ? As + (64 * wave + 8 * j) * 128 : As + (8 * wave + j) * APK;
+    for (int j = 0; j < NLA; ++j) {
+      if (part >= 0 && j * 4 / NLA != part) continue;
+      uint8_t* dst = AKIND == A_ROWS_M ? As + (8 * NLA * wave + 8 * j) * 128 : As + (8 * wave + j) * APK;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_t*)dst, 16, a_voff[j & 1],
                                                static_cast<int>(j * a_row8 + k_off), 0, 0);
     }
@@ -394,7 +399,7 @@ __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0,
   // (lane = 16g + 4a... with t = (lane%16)/4, a = lane%4, g = lane/16);
   // as a destination it receives A[m = l32][k = 16s + 8kg + 4h + 0..3].
   const int tr_t = (lane & 15) >> 2, tr_a = lane & 3, tr_g = lane >> 4;
-  const int tr_base = APK * (4 * (tr_g >> 1) + (tr_t >> 1)) + 32 * (WMR / 8 * wm + 2 * (tr_g & 1) + (tr_a >> 1)) +
+  const int tr_base = APK * (4 * (tr_g >> 1) + (tr_t >> 1)) + 32 * (2 * (tr_g & 1) + (tr_a >> 1)) +
                       16 * (tr_t & 1) + 8 * (tr_a & 1);
   auto load_a = [&](const uint8_t* As, int s, bf16x8* dst) {
 #pragma unroll
@@ -469,10 +474,11 @@ __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0,
       dst[nb] = signs_across_k(*reinterpret_cast<const uint64_t*>(Bs + (c >> 3) * LDB_N + kk), c & 7, sc);
     }
   };
-  // MFMA chunk q (0..3) of a substep: blocks 4q .. 4q+3 in (mb, nb) order
+  // MFMA chunk q (0..3) of a substep: a quarter of the blocks in (mb, nb) order
   auto mfma_row = [&](int s, int q) {
+    constexpr int quarter = MBN * NBN / 4;
 #pragma unroll
-    for (int i = 4 * q; i < 4 * q + 4; ++i)
+    for (int i = quarter * q; i < quarter * (q + 1); ++i)
       acc[i / NBN][i % NBN] = mma_dt<DT>(a[s & 1][i / NBN], b[s & 1][i % NBN], acc[i / NBN][i % NBN]);
   };
 
@@ -765,6 +771,23 @@ struct StageSizes {
   __shared__ __attribute__((aligned(16))) uint8_t B2[BSZ];       \
   __shared__ __attribute__((aligned(16))) uint8_t B3[BSZ];       \
   __shared__ __attribute__((aligned(16))) uint16_t Sc[SSZ];
+
+// 128 x 256 outputs per workgroup, two workgroups per CU (accumulators in 128
+// registers, 72 KiB of LDS): the prologue and epilogue of one run beside the K
+// steps of the other, and products of few tiles or of a little more than whole
+// rounds fill the chip better.  Each expanded sign fragment feeds 4 MFMAs
+// instead of 8, so long K chains in whole rounds stay on 256-row tiles
+// (product_plan has the line).  The same operands in the same K order, so the
+// outputs are the same bits.  us, 256-row tiles (or their K split) -> these:
+// 8184 x 3072 over 768 46.9 -> 33.4, 8184 x 768 over 3072 54.2 -> 35.4, 1531 x
+// 4096 over 4096 62.0 -> 45.7, 2048 x 4096 over 4096 75.7 -> 51.7, 8192 x 4096
+// over 1024 62.2 -> 56.5; 16384 x 14336 over 4096 1242 -> 1292 (not taken).
+template <int BKIND, int EPI, int DT>
+__global__ __launch_bounds__(THREADS, 2) void half_kernel(Params p) {
+  using SZ = StageSizes<A_ROWS_M, BKIND>;
+  QSTE_WIDE_STAGES(A_STAGE / 2, SZ::b, SZ::s)
+  wide_tile<A_ROWS_M, BKIND, EPI, DT, BM / 2>(p, blockIdx.x, A0, A1, A2, A3, B0, B1, B2, B3, Sc);
+}
 
 template <int AKIND, int BKIND, int EPI, int DT>
 __global__ __launch_bounds__(THREADS, 1) void wide_kernel(Params p) {
@@ -1071,31 +1094,10 @@ static int launch_combine(const mfma::wide::Split& sp, const float* m_add, const
   return static_cast<int>(hipGetLastError());
 }
 
-int mfma_linear_forward(const void* x, int dtype, const uint8_t* packed, const float* scale,
-                        const float* bias, void* y, int64_t m, int64_t rows, int64_t cols,
-                        hipStream_t stream) {
-  if (!forward_ok(x, dtype, packed, m, rows, cols)) return 1;
-  mfma::Params p{};
-  p.a = static_cast<const uint16_t*>(x);
-  p.bits = packed;
-  p.out = y;
-  p.M = m; p.N = rows; p.K = cols;
-  p.lda = cols; p.pb = cols / 8;
-  p.a_rows = m; p.bit_rows = rows;
-  p.n_scale = scale; p.n_bias = bias;
-  if (dtype == QSTE_F16)
-    mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD, QSTE_F16>
-        <<<wide_grid(m, rows), mfma::wide::THREADS, 0, stream>>>(p);
-  else
-    mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD, QSTE_BF16>
-        <<<wide_grid(m, rows), mfma::wide::THREADS, 0, stream>>>(p);
-  return static_cast<int>(hipGetLastError());
-}
-
-// K ranges of a forward with `tiles` output tiles and nk K steps: a product
-// with fewer tiles than half the device's 256 CUs and a K chain of 12 steps or
-// more is cut into up to 16 ranges of at least 4 K steps (one round of
-// workgroups), else 1.
+// K ranges of a product with `tiles` output tiles and nk K steps: one with
+// fewer tiles than half the device's 256 CUs and a K chain of 12 steps or more
+// can be cut into up to 16 ranges of at least 4 K steps (one round of
+// workgroups).
 struct SplitK {
   int splits, ks_steps;
 };
@@ -1110,6 +1112,68 @@ static SplitK forward_split_plan(int tiles, int nk) {
   const int ks = (nk + s - 1) / s;
   return {(nk + ks - 1) / ks, ks};
 }
+
+// How a forward or input-gradient product of M x N outputs over nk K steps
+// runs: on 256-row tiles, on 128-row tiles, or on 256-row tiles in K ranges.
+// The estimates, in us, are fits to measured products (M, N and K from 256 to
+// 16384): a round of 256-row tiles takes 1.31 nk + 8; a round of 128-row
+// tiles, two to a CU, 1.38 nk + 5 and one to a CU 0.58 nk + 6.5; ranges add
+// the combine pass and its traffic.  They are within 10% of the measured
+// times where two of them come near each other.
+struct ProductPlan {
+  bool half;
+  SplitK split;
+  double us;
+};
+static ProductPlan product_plan(int64_t M, int64_t N, int nk, bool may_split) {
+  const int64_t tiles = wide_grid(M, N), halves = (M + 127) / 128 * ((N + 255) / 256);
+  ProductPlan best{false, {1, nk}, static_cast<double>((tiles + 255) / 256) * (1.31 * nk + 8.0)};
+  const int64_t rest = halves % 512;
+  const double half = static_cast<double>(halves / 512) * (1.38 * nk + 5.0) +
+                      (rest == 0 ? 0.0 : rest <= 256 ? 0.58 * nk + 6.5 : 1.38 * nk + 5.0);
+  if (half < best.us) best = ProductPlan{true, {1, nk}, half};
+  if (may_split) {
+    const SplitK sp = forward_split_plan(static_cast<int>(tiles), nk);
+    if (sp.splits > 1) {
+      const double bytes = static_cast<double>((sp.splits + 1) * tiles) * (mfma::wide::BM * mfma::wide::BN * 4);
+      const double us = 1.31 * sp.ks_steps + 7.0 + 3.0 + bytes / 5e6;
+      if (us < best.us) best = ProductPlan{false, sp, us};
+    }
+  }
+  return best;
+}
+
+template <int BKIND, int EPI, int DT>
+static int launch_half(const mfma::Params& p, hipStream_t stream) {
+  const int64_t grid = (p.M + 127) / 128 * ((p.N + 255) / 256);
+  mfma::wide::half_kernel<BKIND, EPI, DT><<<static_cast<unsigned>(grid), mfma::wide::THREADS, 0, stream>>>(p);
+  return static_cast<int>(hipGetLastError());
+}
+
+int mfma_linear_forward(const void* x, int dtype, const uint8_t* packed, const float* scale,
+                        const float* bias, void* y, int64_t m, int64_t rows, int64_t cols,
+                        hipStream_t stream) {
+  if (!forward_ok(x, dtype, packed, m, rows, cols)) return 1;
+  mfma::Params p{};
+  p.a = static_cast<const uint16_t*>(x);
+  p.bits = packed;
+  p.out = y;
+  p.M = m; p.N = rows; p.K = cols;
+  p.lda = cols; p.pb = cols / 8;
+  p.a_rows = m; p.bit_rows = rows;
+  p.n_scale = scale; p.n_bias = bias;
+  if (product_plan(m, rows, static_cast<int>(cols / mfma::wide::BK), false).half)
+    return dtype == QSTE_F16 ? launch_half<mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD, QSTE_F16>(p, stream)
+                             : launch_half<mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD, QSTE_BF16>(p, stream);
+  if (dtype == QSTE_F16)
+    mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD, QSTE_F16>
+        <<<wide_grid(m, rows), mfma::wide::THREADS, 0, stream>>>(p);
+  else
+    mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD, QSTE_BF16>
+        <<<wide_grid(m, rows), mfma::wide::THREADS, 0, stream>>>(p);
+  return static_cast<int>(hipGetLastError());
+}
+
 static size_t split_bytes(const SplitK& sp, int tiles) {
   return sp.splits > 1 ? static_cast<size_t>(sp.splits) * tiles * mfma::wide::BM * mfma::wide::BN * sizeof(float) : 0;
 }
@@ -1135,8 +1199,7 @@ static int launch_split(const mfma::Params& p, const SplitK& sp, float* partial,
 // rounding.  Workspace bytes, 0 where no split pays.
 size_t mfma_forward_split_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
   if (!mfma_dtype(dtype) || m <= 16 || rows <= 0 || cols <= 0 || cols % 64 != 0) return 0;
-  const int tiles = wide_grid(m, rows);
-  return split_bytes(forward_split_plan(tiles, static_cast<int>(cols / mfma::wide::BK)), tiles);
+  return split_bytes(product_plan(m, rows, static_cast<int>(cols / mfma::wide::BK), true).split, wide_grid(m, rows));
 }
 
 // Returns 1 when the call is not for this path (shape, or too little workspace).
@@ -1155,7 +1218,7 @@ int mfma_linear_forward_split(const void* x, int dtype, const uint8_t* packed, c
   p.a_rows = m; p.bit_rows = rows;
   p.out = y;
   p.n_scale = scale; p.n_bias = bias;
-  const SplitK sp = forward_split_plan(wide_grid(m, rows), static_cast<int>(cols / mfma::wide::BK));
+  const SplitK sp = product_plan(m, rows, static_cast<int>(cols / mfma::wide::BK), true).split;
   float* partial = static_cast<float*>(workspace);
   return dtype == QSTE_F16
              ? launch_split<mfma::B_BITS_ALONG_K, QSTE_F16, QSTE_F16>(p, sp, partial, stream)
@@ -1168,12 +1231,12 @@ int mfma_linear_forward_split(const void* x, int dtype, const uint8_t* packed, c
 // which weighs its time; a layer whose evidence and input gradient share one
 // launch is not cut, and the product called alone is cut as the layer's is,
 // so the two agree bit for bit.
-static SplitK dgrad_cut(int64_t m, int64_t rows, int64_t cols) {
-  return forward_split_plan(wide_grid(m, cols), static_cast<int>((rows + mfma::wide::BK - 1) / mfma::wide::BK));
+static ProductPlan dgrad_cut(int64_t m, int64_t rows, int64_t cols) {
+  return product_plan(m, cols, static_cast<int>((rows + mfma::wide::BK - 1) / mfma::wide::BK), true);
 }
 static SplitK dgrad_split(int64_t m, int64_t rows, int64_t cols) {
   if (mfma_evidence_plan(m, rows, cols, true).pair) return {1, 0};
-  return dgrad_cut(m, rows, cols);
+  return dgrad_cut(m, rows, cols).split;
 }
 int64_t mfma_dgrad_split_bytes(int64_t m, int64_t rows, int64_t cols) {
   if (m <= 0 || rows <= 0 || cols <= 0) return 0;
@@ -1222,6 +1285,9 @@ int mfma_linear_dgrad_t(const void* dy, int64_t ldy, int dtype, const uint8_t* w
     return dtype == QSTE_F16
                ? launch_split<mfma::B_BITS_ALONG_K_SCALED, QSTE_F16, QSTE_F16>(p, sp, partial, stream)
                : launch_split<mfma::B_BITS_ALONG_K_SCALED, QSTE_BF16, QSTE_BF16>(p, sp, partial, stream);
+  if (product_plan(m, cols, static_cast<int>(ldy / mfma::wide::BK), false).half)
+    return dtype == QSTE_F16 ? launch_half<mfma::B_BITS_ALONG_K_SCALED, mfma::EPI_PLAIN, QSTE_F16>(p, stream)
+                             : launch_half<mfma::B_BITS_ALONG_K_SCALED, mfma::EPI_PLAIN, QSTE_BF16>(p, stream);
   if (dtype == QSTE_F16)
     mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K_SCALED, mfma::EPI_PLAIN, QSTE_F16>
         <<<wide_grid(m, cols), mfma::wide::THREADS, 0, stream>>>(p);
@@ -1369,13 +1435,11 @@ static EvidencePlan compute_plan(int64_t samples, int64_t rows, int64_t cols, bo
   if (samples <= 0 || rows <= 0 || cols <= 0) return best;
   const int64_t dgrad[1][2] = {{td, nkd + kTileOverhead}};
   double dgrad_alone = td ? static_cast<double>(list_schedule(dgrad, 1)) : 0.0;
-  if (const int64_t splits = td ? dgrad_cut(samples, rows, cols).splits : 1; splits > 1) {
-    // as its own launch dX cuts K where its tiles are few
-    const int64_t ks = (nkd + splits - 1) / splits;
-    const int64_t ranges[1][2] = {{td * splits, ks + kTileOverhead}};
-    const double cut = static_cast<double>(list_schedule(ranges, 1)) +
-                       static_cast<double>((splits + 1) * td * kTileBytes) / kBytesPerStep + 2.0;
-    if (cut < dgrad_alone) dgrad_alone = cut;
+  if (td) {
+    // as its own launch dX may run on half tiles or in K ranges; its time in
+    // us, and a launch's, in K steps
+    const double own = (dgrad_cut(samples, rows, cols).us + 8.0) / 1.31;
+    if (own < dgrad_alone) dgrad_alone = own;
   }
   double best_cost = -1.0;
   for (int S = 1; S <= 8; S *= 2) {
@@ -1626,11 +1690,13 @@ static int64_t f32_chunk_rows(int64_t m, int64_t k) {
   return fit >= m ? m : fit / mfma::wide::BM * mfma::wide::BM;
 }
 
-static SplitK f32_split(int64_t m, int64_t n, int64_t k) {
-  return forward_split_plan(wide_grid(m, n), static_cast<int>(3 * up64(k) / mfma::wide::BK));
+static ProductPlan f32_plan(int64_t m, int64_t n, int64_t k) {
+  return product_plan(m, n, static_cast<int>(3 * up64(k) / mfma::wide::BK), true);
 }
 
-static size_t f32_partial(int64_t m, int64_t n, int64_t k) { return split_bytes(f32_split(m, n, k), wide_grid(m, n)); }
+static size_t f32_partial(int64_t m, int64_t n, int64_t k) {
+  return split_bytes(f32_plan(m, n, k).split, wide_grid(m, n));
+}
 
 // Workspace of an [m, n] product over k through the limbs (0: not for it):
 // the dense limbs of a chunk, the signs three times, and the split-K partials
@@ -1667,10 +1733,12 @@ static int f32_product(const float* dense, const float* col_mul, const uint8_t* 
     p.lda = 3 * kp; p.pb = 3 * kp / 8;
     p.a_rows = mi; p.bit_rows = n;
     p.n_scale = scale; p.n_bias = bias;
-    const SplitK sp = f32_split(mi, n, k);
+    const ProductPlan plan = f32_plan(mi, n, k);
     int rc;
-    if (sp.splits > 1) {
-      rc = launch_split<mfma::B_BITS_ALONG_K, QSTE_BF16, QSTE_F32>(p, sp, partial, stream);
+    if (plan.split.splits > 1) {
+      rc = launch_split<mfma::B_BITS_ALONG_K, QSTE_BF16, QSTE_F32>(p, plan.split, partial, stream);
+    } else if (plan.half) {
+      rc = launch_half<mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD_F32, QSTE_BF16>(p, stream);
     } else {
       mfma::wide::wide_kernel<mfma::A_ROWS_M, mfma::B_BITS_ALONG_K, mfma::EPI_FORWARD_F32, QSTE_BF16>
           <<<wide_grid(mi, n), mfma::wide::THREADS, 0, stream>>>(p);

@@ -558,8 +558,9 @@ struct Plan {
 // workgroup, forming fragments from x (0.087 us per chunk and tile of 16
 // rows: 192 VALU instructions) and x's reads from L2 (0.0085 us per chunk and
 // row) bound the kernel, not the weights; S ranges cut both S-fold, and cost
-// a second launch and the sums' round trip.  Measured, one range against the
-// best split: 8192 x 28672, M = 16: 19.9 / 17.9 us, M = 40: 40.6 / 31.9;
+// a second launch and the sums' round trip, a little more for more ranges.
+// Measured, one range against the best split: 8192 x 28672, M = 16: 19.9 / 18.1
+// us (two ranges; four 17.9), M = 40: 40.6 / 31.9;
 // 4096 x 14336, M = 24: 14.4 / 13.0, M = 16: 9.8 / 10.4 (not split); three
 // blocks and more (14336 x 4096, M = 40: 11.8 / 20.8) are never split.
 Plan plan_of(int64_t xr, int64_t rows, int64_t cols, bool may_split) {
@@ -572,7 +573,7 @@ Plan plan_of(int64_t xr, int64_t rows, int64_t cols, bool may_split) {
       const int64_t cps = (chunks + s - 1) / s, ns = (chunks + cps - 1) / cps;
       if ((blocks * ns + 255) / 256 > most) continue;  // a second round
       const double saved = static_cast<double>(chunks - cps) * (0.087 * tiles + 0.0085 * xr);
-      const double cost = 4.5 + static_cast<double>(ns * xr * rows) * 8.0 / 4e6;
+      const double cost = 4.5 + 1.3 * static_cast<double>(ns - 2) + static_cast<double>(ns * xr * rows) * 8.0 / 4e6;
       if (saved - cost > best) {
         best = saved - cost;
         splits = ns;
