@@ -2,6 +2,7 @@
 // workspace carving and kernel dispatch.  Nothing here allocates or
 // synchronizes; every launch goes on the caller's stream.
 #include "common.hpp"
+#include "prep.hpp"
 
 namespace qste {
 int launch_pack_coordinate(const int8_t*, uint8_t*, int64_t, int64_t, hipStream_t);
@@ -54,8 +55,8 @@ int mfma_backward_pair(const void*, int64_t, int, const uint8_t*, int64_t, const
 int launch_pad_rows(const void*, void*, int64_t, int64_t, int64_t, hipStream_t);
 int launch_colsums_pad(const void*, int, const float*, int64_t, int64_t, int64_t, uint16_t*, float*, float*, float*,
                        float*, hipStream_t);
-int launch_transpose_bits(const uint8_t*, uint8_t*, int64_t, int64_t, int64_t, int64_t, hipStream_t);
-int launch_f32_to_16(const float*, uint16_t*, int64_t, int64_t, int, hipStream_t);
+int launch_backward_prep(const void*, int, const float*, int64_t, int64_t, float*, float*, float*, float*,
+                         const TransposeJob&, const ScaleJob&, const TransposeJob&, const ScaleJob&, hipStream_t);
 size_t gemv_forward_workspace(int64_t, int64_t, int64_t, int);
 int gemv_linear_forward(const void*, int, const uint8_t*, const float*, const float*, void*, int64_t, int64_t,
                         int64_t, void*, size_t, hipStream_t);
@@ -459,6 +460,7 @@ int linear_backward_impl(const void* dy, int dtype, const uint8_t* packed_x, con
     const int64_t ldy = pad_dy ? up64(rows) : rows;
     const bool matrix = (ragged || (rows % 64 == 0 && cols % 64 == 0)) &&
                         mfma_backward_ok(dy_m, ldy, dtype, samples, rows, cols);
+    bool sums_with_prep = false;
     // the offset correction's column sums, unless the caller brings them
     // (with a bias gradient to form, dy is read for both anyway)
     if (matrix && pad_dy) {
@@ -468,6 +470,8 @@ int linear_backward_impl(const void* dy, int dtype, const uint8_t* packed_x, con
       if (offset_dot && !grad_bias) v = const_cast<float*>(offset_dot);  // only read from here on
     } else if (offset_dot && !grad_bias) {
       v = const_cast<float*>(offset_dot);
+    } else if (matrix) {
+      sums_with_prep = true;
     } else if ((rc = launch_colsums(dy, dtype, x_offset, samples, rows, v_part, grad_bias ? db_part : nullptr, v,
                                     grad_bias, s))) {
       return rc;
@@ -493,13 +497,16 @@ int linear_backward_impl(const void* dy, int dtype, const uint8_t* packed_x, con
         w_epi_pb = (cols + 127) / 128 * 16;
         if ((rc = launch_pad_rows(packed_w, base + l.w_pad, rows, pb, w_epi_pb, s))) return rc;
       }
-      if (dx) {
-        if ((rc = launch_transpose_bits(packed_w, w_t, rows, cols, pb, l.w_t_pitch, s))) return rc;
-        if ((rc = launch_f32_to_16(scale, s16, rows, up64(rows), dtype, s))) return rc;
-      }
+      const TransposeJob no_w{};
+      const ScaleJob no_ws{};
+      if ((rc = launch_backward_prep(
+               sums_with_prep ? dy : nullptr, dtype, x_offset, samples, rows, v_part, grad_bias ? db_part : nullptr, v,
+               grad_bias, transpose_job(packed_x, x_t, samples, cols, pb, l.x_t_pitch),
+               ScaleJob{x_scale, xs16, samples, up64(samples)},
+               dx ? transpose_job(packed_w, w_t, rows, cols, pb, l.w_t_pitch) : no_w,
+               dx ? ScaleJob{scale, s16, rows, up64(rows)} : no_ws, s)))
+        return rc;
       if (plan.pair) {
-        if ((rc = launch_transpose_bits(packed_x, x_t, samples, cols, pb, l.x_t_pitch, s))) return rc;
-        if ((rc = launch_f32_to_16(x_scale, xs16, samples, up64(samples), dtype, s))) return rc;
         rc = mfma_backward_pair(dy_m, ldy, dtype, x_t, l.x_t_pitch, xs16, evidence, w_t, l.w_t_pitch, s16, w_epi,
                                 w_epi_pb, dx, samples, rows, cols, v, scale, gs_part, plan, partial, s);
         if (rc == 0) return launch_sum_partials(gs_part, mfma_evidence_tiles(cols), rows, grad_scale, s);
@@ -511,8 +518,6 @@ int linear_backward_impl(const void* dy, int dtype, const uint8_t* packed_x, con
           if (rc) return rc;
         }
         dgrad_done = true;
-        if ((rc = launch_transpose_bits(packed_x, x_t, samples, cols, pb, l.x_t_pitch, s))) return rc;
-        if ((rc = launch_f32_to_16(x_scale, xs16, samples, up64(samples), dtype, s))) return rc;
         rc = mfma_evidence_t(dy_m, ldy, dtype, x_t, l.x_t_pitch, xs16, evidence, samples, rows, cols, v, scale, w_epi,
                              w_epi_pb, gs_part, &plan, partial, s);
         if (rc == 0) return launch_sum_partials(gs_part, mfma_evidence_tiles(cols), rows, grad_scale, s);

@@ -232,7 +232,7 @@ __global__ __launch_bounds__(kThreads) void backward_bf16x8_kernel(const uint4* 
 // input; each layer's backward forms v[c] = sum_t dY[t, c] * offset[t], the
 // offset correction of its evidence (functional.py:139-144), by reading its
 // dY again.  This pass writes dg and du and sums them as it goes, with the
-// chunking and order of colsum_partial_x8_kernel (reduce.hip): chunks of
+// chunking and order of colsum_partial_vec_kernel (reduce.hip): chunks of
 // kSumChunk samples, kSumWaves waves per chunk each summing a run of
 // consecutive samples with fmaf in sample order, the waves' sums added in
 // wave order, and the chunk partials [chunk][2][cols] summed in chunk order
