@@ -295,8 +295,11 @@ __device__ __forceinline__ float value_of(float x, float a) {
   } else if constexpr (KIND == QSTE_ACT_GELU_TANH) {
     const float beta = static_cast<float>(kSqrt2 * 1.12837916709551257390 * 0.5);
     const float kappa = static_cast<float>(kTanhCoefficient);
+    // torch's rounding: one fused multiply-add (equal to its values over all
+    // bf16 and fp16 inputs and 4M normal fp32 ones; with the product rounded
+    // first, 0.5% of the fp32 values differ by an ulp)
     const float cube = x * x * x;
-    const float inner = beta * (x + kappa * cube);
+    const float inner = beta * fmaf(kappa, cube, x);
     return 0.5f * x * (1.0f + tanhf(inner));
   } else if constexpr (KIND == QSTE_ACT_SILU) {
     return x / (1.0f + expf(-x));
@@ -474,7 +477,23 @@ __device__ __forceinline__ int32_t cvt_i32_nan0(float v) {
   return r;
 }
 
-// bf16 SiLU table entry: .x the derivative's bits, .y the value's bf16 bits.
+// bf16 SiLU and GELU take their value and derivative from an LDS table (4096
+// entries of 8 bytes, tab16_index's range) that each workgroup fills once and
+// then walks row blocks, so the exponentials, tanhs and divisions are paid per
+// table entry, not per element.  Pays from kTableElements on, with 16 waves
+// per CU (more of them fill more tables, fewer leave loads in flight too few).
+// us, per element (in a kernel of the same LDS) / table of 3072 / 4096 / 8192 waves: tanh-GELU 8184 x 3072 59.4 /
+// 33.8 / 32.7 / 37.0 (with torch's value pass before it 56.5), 16384 x 14336 585 /
+// 321 / 246 / 259 (506); GELU 1023 x 3072 11.6 / 11.7 / 13.4 / 13.2, 2046 x 3072
+// 18.8 / 14.9 / 16.7 / 22.1; SiLU 1023 x 3072 8.6 / 10.3 / 11.8 / 11.7, 16384 x 3072
+// 84.1 / 61.3 / 55.9 / 58.8.
+constexpr int64_t kTableElements = 4 << 20;
+constexpr int64_t kTableWaves = 4096;
+template <int DT, int KIND>
+constexpr bool kSmoothTable =
+    (KIND == QSTE_ACT_SILU || KIND == QSTE_ACT_GELU || KIND == QSTE_ACT_GELU_TANH) && DT == QSTE_BF16;
+
+// A table entry: .x the derivative's bits, .y the value's bf16 bits.
 using SmoothEntry = uint2;
 
 // The entry of any bf16 input (the table holds those of tab16_index's range).
@@ -527,7 +546,7 @@ __device__ __forceinline__ void table_chunk(const uint4& raw, const SmoothEntry*
 // mode: 0 -- compute y = f(x), store it (when y != NULL), derive from it
 //       1 -- y holds the forward output already (computed elsewhere); read it
 //       2 -- `provided` holds the fp32 derivative (x, y unused)
-// tab (bf16 SiLU in mode 0 with whole chunks, may be NULL): value and
+// tab (bf16 SiLU and GELU in mode 0 with whole chunks, may be NULL): value and
 // derivative of the tabulated bf16 inputs (tab16_index), filled by the caller.
 template <int DT, int G, int CH, int KIND, int BLOCK>
 __device__ __forceinline__ void smooth_row(const typename Elem<DT>::T* __restrict__ x,
@@ -541,7 +560,7 @@ __device__ __forceinline__ void smooth_row(const typename Elem<DT>::T* __restric
   // the specialised kinds run in one mode only (smooth_dispatch)
   const int mode = KIND == QSTE_ACT_SILU || KIND == QSTE_ACT_GELU
                        ? 0
-                       : (KIND == QSTE_ACT_GELU_TANH || KIND == QSTE_ACT_HARDSWISH ? 1 : run_mode);
+                       : (KIND == QSTE_ACT_HARDSWISH ? 1 : run_mode);
   constexpr int kRowsPerBlock = BLOCK / G;
   const int64_t row = block * kRowsPerBlock + threadIdx.x / G;
   const int t = threadIdx.x % G;
@@ -641,7 +660,7 @@ __device__ __forceinline__ void smooth_row(const typename Elem<DT>::T* __restric
         const int64_t q = t + static_cast<int64_t>(k) * G;
         if (live && q < nch) {
           bool done = false;
-          if constexpr (KIND == QSTE_ACT_SILU && DT == QSTE_BF16) {
+          if constexpr (kSmoothTable<DT, KIND>) {
             if (tab != nullptr) {
               uint32_t ybits[4];
               table_chunk<KIND>(raw[k], tab, a, cache[k], ybits);
@@ -708,28 +727,20 @@ __device__ __forceinline__ void smooth_row(const typename Elem<DT>::T* __restric
   if (t == 0) scale[row] = s;
 }
 
-// bf16 SiLU takes its value and derivative from an LDS table (4096 entries of
-// 8 bytes, tab16_index's range) that each workgroup fills once and then walks
-// row blocks, so the exponential and divisions are paid per table entry, not
-// per element.
-template <int DT, int KIND>
-constexpr bool kSmoothTable = KIND == QSTE_ACT_SILU && DT == QSTE_BF16;
-
-template <int DT, int G, int CH, int KIND, int BLOCK>
+template <int DT, int G, int CH, int KIND, int BLOCK, bool TABLE>
 __global__ __launch_bounds__(BLOCK) void smooth_rows_kernel(
     const typename Elem<DT>::T* __restrict__ x, typename Elem<DT>::T* __restrict__ y,
     const float* __restrict__ provided, int mode, SmoothParams p, void* __restrict__ payload,
     float* __restrict__ scale, int64_t rows, int64_t cols, int64_t blocks) {
   __shared__ float red[BLOCK / kWave];
-  if constexpr (kSmoothTable<DT, KIND>) {
+  if constexpr (TABLE) {
     __shared__ SmoothEntry tab[kTab16Entries];
     for (int j = threadIdx.x; j < kTab16Entries; j += BLOCK)
       tab[j] = smooth_entry<KIND>(tab16_bits(static_cast<uint32_t>(j)), p.a);
     __syncthreads();
     // every thread walks the same blocks, so the reductions' barriers match
     for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x)
-      smooth_row<DT, G, CH, KIND, BLOCK>(x, y, provided, mode, p.kind, p.a, payload, scale, rows, cols, red, b,
-                                         mode == 0 ? tab : nullptr);
+      smooth_row<DT, G, CH, KIND, BLOCK>(x, y, provided, 0, p.kind, p.a, payload, scale, rows, cols, red, b, tab);
   } else {
     smooth_row<DT, G, CH, KIND, BLOCK>(x, y, provided, mode, p.kind, p.a, payload, scale, rows, cols, red,
                                        blockIdx.x);
@@ -813,10 +824,15 @@ int smooth_launch(const void* x, void* y, const float* provided, int mode, Smoot
   using T = typename Elem<DT>::T;
   constexpr int kRows = BLOCK / G;
   const int64_t blocks = (rows + kRows - 1) / kRows;
-  // the tabulated kind: a few workgroups per CU, each filling its table once
-  const int64_t grid = kSmoothTable<DT, KIND> ? (blocks < 8192 / (BLOCK / kWave) ? blocks : 8192 / (BLOCK / kWave))
-                                              : blocks;
-  smooth_rows_kernel<DT, G, CH, KIND, BLOCK><<<static_cast<unsigned>(grid), BLOCK, 0, s>>>(
+  if constexpr (kSmoothTable<DT, KIND> && CH > 0) {
+    if (mode == 0 && cols % 8 == 0 && rows * cols >= kTableElements) {
+      const int64_t most = kTableWaves / (BLOCK / kWave);
+      smooth_rows_kernel<DT, G, CH, KIND, BLOCK, true><<<static_cast<unsigned>(blocks < most ? blocks : most), BLOCK, 0, s>>>(
+          static_cast<const T*>(x), static_cast<T*>(y), provided, mode, p, payload, scale, rows, cols, blocks);
+      return static_cast<int>(hipGetLastError());
+    }
+  }
+  smooth_rows_kernel<DT, G, CH, KIND, BLOCK, false><<<static_cast<unsigned>(blocks), BLOCK, 0, s>>>(
       static_cast<const T*>(x), static_cast<T*>(y), provided, mode, p, payload, scale, rows, cols, blocks);
   return static_cast<int>(hipGetLastError());
 }
@@ -841,9 +857,9 @@ int smooth_shapes(const void* x, void* y, const float* provided, int mode, Smoot
   }
 }
 
-// The MLP activations get kernels of their own: GELU and SiLU computing their
-// value, tanh-GELU and Hardswish deriving from torch's (which they cannot
-// reproduce bit for bit); every other case runs the run-time-kind kernel.
+// The MLP activations get kernels of their own: GELU, tanh-GELU and SiLU
+// computing their value, Hardswish (and tanh-GELU given its value) deriving from
+// torch's; every other case runs the run-time-kind kernel.
 template <int DT>
 int smooth_dispatch(const void* x, void* y, const float* provided, int mode, SmoothParams p, void* payload,
                     float* scale, int64_t rows, int64_t cols, hipStream_t s) {
@@ -851,7 +867,7 @@ int smooth_dispatch(const void* x, void* y, const float* provided, int mode, Smo
     return smooth_shapes<DT, QSTE_ACT_SILU>(x, y, provided, mode, p, payload, scale, rows, cols, s);
   if (mode == 0 && p.kind == QSTE_ACT_GELU)
     return smooth_shapes<DT, QSTE_ACT_GELU>(x, y, provided, mode, p, payload, scale, rows, cols, s);
-  if (mode == 1 && p.kind == QSTE_ACT_GELU_TANH)
+  if (mode != 2 && p.kind == QSTE_ACT_GELU_TANH)
     return smooth_shapes<DT, QSTE_ACT_GELU_TANH>(x, y, provided, mode, p, payload, scale, rows, cols, s);
   if (mode == 1 && p.kind == QSTE_ACT_HARDSWISH)
     return smooth_shapes<DT, QSTE_ACT_HARDSWISH>(x, y, provided, mode, p, payload, scale, rows, cols, s);

@@ -352,12 +352,12 @@ _SMOOTH: dict[str, object] = {
 
 # (kind, dtype) pairs whose kernel value equals torch's on the GPU (checked by
 # tests/test_gpu_activations.py); the rest take torch's value and the kernel
-# derives from it.  torch evaluates tanh-GELU and Hardswish in fp32 with a
-# different operation order (1-ulp differences in fp32 on ~0.4% / ~27% of
-# inputs), which a bf16/fp16 rounding hides only most of the time, so both
-# take torch's value in every dtype.
+# derives from it.  torch evaluates Hardswish in fp32 with a different
+# operation order (1-ulp differences in fp32 on ~27% of inputs), which a
+# bf16/fp16 rounding hides only most of the time, so it takes torch's value in
+# every dtype.
 _KERNEL_VALUE: set[tuple[str, torch.dtype]] = {
-    (k, d) for k in ("gelu", "silu", "tanh", "sigmoid", "elu", "celu", "selu", "softplus", "mish")
+    (k, d) for k in ("gelu", "gelu_tanh", "silu", "tanh", "sigmoid", "elu", "celu", "selu", "softplus", "mish")
     for d in _KERNEL_DTYPES
 }
 
@@ -393,6 +393,8 @@ class _SmoothFn(Function):
         if flat.dtype in _KERNEL_DTYPES and (kernel_kind, flat.dtype) in _KERNEL_VALUE:
             out, payload, scale = kernels.smooth_activation(flat, kernel_kind, kernel_param)
             output = out.view(shape)
+            if kernel_kind == "gelu_tanh" and not inputs.is_contiguous():
+                output = torch.empty_like(inputs).copy_(output)  # torch's layout of it
         else:
             output = forward(inputs, param)
             x32 = flat if flat.dtype in _KERNEL_DTYPES else flat.float()
