@@ -417,6 +417,15 @@ int qste_row_scale(const void* log_scale, int dtype, void* scale, void* exp_valu
 int qste_row_scale_backward(const void* exp_value, const void* grad, int dtype, void* grad_log_scale, int64_t n,
                             float lo, float hi, void* stream);
 
+/* The end of an optimizer step over `count` surfaces: log_scale[i], fp32 [n[i]],
+ * is clamped to [lo, hi] in place (a NaN stays NaN) and, when nflips > 0,
+ * *total = the sum of the nflips <= count counters flips[i].  The three arrays are host
+ * memory, read before the call returns; what they point at and total are
+ * device memory.  Replaces the clamp per surface and the sum of the flips in
+ * QSTEOptimizer.step (src/qste/optim.py:162-198). */
+int qste_step_finish(float* const* log_scale, const int64_t* n, int count, const int64_t* const* flips, int nflips,
+                     float lo, float hi, int64_t* total, void* stream);
+
 /* ---- binary embedding (src/qste/modules.py:68-100) ---------------------- */
 
 /* out [count, cols] (out_dtype) = sign(packed[ids[n]]) * scale[ids[n]];

@@ -67,6 +67,8 @@ int launch_row_scale(const void*, int, void*, void*, int64_t, float, float, hipS
 size_t swiglu_backward_sums_workspace(int64_t, int64_t);
 int launch_swiglu_backward_sums(const void*, const void*, const void*, int, void*, void*, const float*, const float*,
                                 int64_t, int64_t, float*, float*, hipStream_t, int64_t);
+int launch_step_finish(float* const*, const int64_t*, int, const int64_t* const*, int, float, float, int64_t*,
+                       hipStream_t);
 int launch_row_scale_backward(const void*, const void*, int, void*, int64_t, float, float, hipStream_t);
 // fp32 products through bf16 limbs (gemm_mfma.hip): 0 bytes / return 1 when
 // the shape is not for them
@@ -681,6 +683,20 @@ int qste_row_scale(const void* log_scale, int dtype, void* scale, void* exp_valu
   if (n == 0) return 0;
   if (!log_scale || !scale || !exp_value) return QSTE_E_NULL;
   return launch_row_scale(log_scale, dtype, scale, exp_value, n, lo, hi, as_stream(stream));
+}
+
+int qste_step_finish(float* const* log_scale, const int64_t* n, int count, const int64_t* const* flips, int nflips,
+                     float lo, float hi, int64_t* total, void* stream) {
+  if (count < 0 || nflips < 0 || nflips > count) return QSTE_E_SHAPE;
+  if (count == 0) return 0;
+  if (!log_scale || !n || (nflips > 0 && (!flips || !total))) return QSTE_E_NULL;
+  for (int i = 0; i < count; ++i) {
+    if (n[i] < 0) return QSTE_E_SHAPE;
+    if (n[i] > 0 && !log_scale[i]) return QSTE_E_NULL;
+  }
+  for (int i = 0; i < nflips; ++i)
+    if (!flips[i]) return QSTE_E_NULL;
+  return launch_step_finish(log_scale, n, count, flips, nflips, lo, hi, total, as_stream(stream));
 }
 
 int qste_row_scale_backward(const void* exp_value, const void* grad, int dtype, void* grad_log_scale, int64_t n,

@@ -13,6 +13,8 @@ workspaces the C entry points ask for; the library itself never allocates.
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 from torch import Tensor
 
@@ -187,8 +189,6 @@ def stream_read(src: Tensor, groups: int | None = None) -> None:
 def device_info(device=None) -> dict:
     """What the runtime reports for ``device``: compute units, maximum shader
     clock and memory clock (MHz), LDS bytes per compute unit."""
-
-    import ctypes
 
     device = torch.device(device or "cuda")
     out = (ctypes.c_int64 * 4)()
@@ -816,6 +816,30 @@ def row_scale_backward(exp_value: Tensor, grad: Tensor, lo: float, hi: float) ->
                                                float(hi), _stream(device))
     _lib.check(code, "row_scale_backward")
     return out
+
+
+def step_finish(log_scales: list[Tensor], lo: float, hi: float, flips: list[Tensor]) -> Tensor | None:
+    """``clamp_(lo, hi)`` of every log-scale and the sum of the flip counters
+    (device int64 scalars), one launch; None, with nothing done, unless all
+    are plain tensors of one GPU (log-scales fp32 and contiguous)."""
+
+    device = log_scales[0].device
+    if device.type != "cuda" or len(flips) > len(log_scales):
+        return None
+    for t in log_scales:
+        if type(t) is not Tensor or t.dtype != torch.float32 or t.device != device or not t.is_contiguous():
+            return None
+    for t in flips:
+        if type(t) is not Tensor or t.dtype != torch.int64 or t.device != device or t.numel() != 1:
+            return None
+    count = len(log_scales)
+    total = torch.empty((), dtype=torch.int64, device=device)
+    pointers, lengths = ctypes.c_void_p * count, ctypes.c_int64 * count
+    code = _lib.load().qste_step_finish(
+        pointers(*[t.data_ptr() for t in log_scales]), lengths(*[t.numel() for t in log_scales]), count,
+        pointers(*[t.data_ptr() for t in flips]), len(flips), float(lo), float(hi), _ptr(total), _stream(device))
+    _lib.check(code, "step_finish")
+    return total
 
 
 # ---------------------------------------------------------------------------

@@ -76,6 +76,7 @@ SIGNATURES = {
     "qste_swiglu_backward_sums": (_int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _sz, _vp]),
     "qste_swiglu_backward_sums_into": (_int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _sz, _vp]),
     "qste_row_scale": (_int, [_vp, _int, _vp, _vp, _i64, _flt, _flt, _vp]),
+    "qste_step_finish": (_int, [_vp, _vp, _int, _vp, _int, _flt, _flt, _vp, _vp]),
     "qste_row_scale_backward": (_int, [_vp, _vp, _int, _vp, _i64, _flt, _flt, _vp]),
     "qste_packed_embedding": (_int, [_vp, _i64, _vp, _vp, _vp, _int, _i64, _i64, _vp]),
     "qste_embedding_backward_workspace_bytes": (_sz, [_i64, _i64]),

@@ -225,11 +225,16 @@ class QSTEOptimizer:
             pending = slot.surface.flush_evidence(keep_buffer=self.deferred)
             if pending is not None:
                 self._apply(slot.surface, pending)
-            slot.surface.log_scale.data.clamp_(lo, hi)
+        log_scales = [slot.surface.log_scale.data for slot in self._slots.values()]
         counts = [slot.flips for slot in self._slots.values() if slot.applied]
+        total = kernels.step_finish(log_scales, lo, hi, counts)
+        if total is None:
+            for log_scale in log_scales:
+                log_scale.clamp_(lo, hi)
         flips = 0
         if counts:
-            total = torch.stack(counts).sum()
+            if total is None:
+                total = torch.stack(counts).sum()
             if total.is_cuda and self._host_count is None:
                 self._host_count = torch.empty((), dtype=torch.int64, pin_memory=True)
             flips = _read_count(total, self._host_count)
