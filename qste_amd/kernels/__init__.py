@@ -235,7 +235,7 @@ def profile(device=None) -> str:
             f"hbm={props.total_memory / 2**30:.0f}GiB  lds={info['lds_per_cu'] / 1024:.0f}KiB/CU  "
             f"library=libqste_hip v{version}  "
             "(products: bf16/fp16 MFMA 256x256 tiles, fp32 as three bf16 limbs; up to 64 rows (21 in fp32): weight "
-            "bits as sparse-MFMA indexes; coordinate step: one launch for columns % 2048 == 0, else six)")
+            "bits as sparse-MFMA indexes; coordinate step: one launch for columns % 2048 == 0, else five or six)")
 
 
 # ---------------------------------------------------------------------------
