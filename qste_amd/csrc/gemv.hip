@@ -421,7 +421,10 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
     }
   }
 
-  // partial sums of the 8 waves, added in wave order
+  // partial sums of the 8 waves, added in wave order, in the LDS the x rows
+  // were staged in: two chunks in LDS leave loads past the last chunk in
+  // flight (they land as zeros), and the barrier alone does not wait for them
+  if constexpr (C::XBUF > 1) wait_vm<0>();
   if (tid < 16 * NBW) {
     epi[0][tid] = out_scale;
     epi[1][tid] = out_bias;

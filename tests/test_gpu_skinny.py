@@ -96,6 +96,24 @@ def test_fp32_rows(rows, cols, m):
         _check(torch.from_numpy(got[:m - 1]), x[:m - 1], packed, scale, bias, cols)
 
 
+# few rows with two chunks of x in LDS at a time: a wave's third chunk (past
+# 8192 columns) reuses a buffer, the last chunk is cut short, and the sums of
+# one and two blocks land where x rows were staged
+@pytest.mark.parametrize("rows,cols,m,dtype", [(4097, 14464, 1, torch.bfloat16), (8192, 16512, 4, torch.float16),
+                                               (1000, 9088, 2, torch.bfloat16), (40, 28672, 3, torch.float16),
+                                               (5000, 12416, 1, torch.float32)])
+def test_few_rows_over_many_chunks(rows, cols, m, dtype):
+    from qste_amd import kernels
+
+    print(f"skinny {rows}x{cols} m={m} {dtype}", flush=True)
+    packed, x, scale, bias = _problem(rows, cols, m, dtype, rows + cols + m)
+    pick = np.unique(np.concatenate([np.arange(0, rows, max(1, rows // 97)), np.arange(max(0, rows - 40), rows)]))
+    got = kernels.packed_linear_affine(torch.from_numpy(x).to(DEV, dtype), torch.from_numpy(packed).to(DEV),
+                                       torch.from_numpy(scale).to(DEV), torch.from_numpy(bias).to(DEV), cols)
+    assert torch.isfinite(got).all()
+    _check(got[:, torch.from_numpy(pick).to(DEV)], x, np.ascontiguousarray(packed[pick]), scale[pick], bias[pick], cols)
+
+
 @pytest.mark.parametrize("rows,cols,m", [(8192, 28672, 16), (1000, 8192, 64), (4096, 14336, 24)])
 def test_split_plans_are_deterministic(rows, cols, m):
     """Shapes whose plan splits K: two calls agree bit for bit, and with the
