@@ -57,6 +57,7 @@ int launch_colsums_pad(const void*, int, const float*, int64_t, int64_t, int64_t
                        float*, hipStream_t);
 int launch_backward_prep(const void*, int, const float*, int64_t, int64_t, float*, float*, float*, float*,
                          const TransposeJob&, const ScaleJob&, const TransposeJob&, const ScaleJob&, hipStream_t);
+bool gemv_takes(int64_t, int64_t, int64_t, int);
 size_t gemv_forward_workspace(int64_t, int64_t, int64_t, int);
 int gemv_linear_forward(const void*, int, const uint8_t*, const float*, const float*, void*, int64_t, int64_t,
                         int64_t, void*, size_t, hipStream_t);
@@ -294,7 +295,7 @@ int64_t padded_forward_cols(int64_t m, int64_t rows, int64_t cols, int dtype) {
 size_t elem_bytes(int dtype) { return dtype == QSTE_F32 ? 4 : 2; }
 
 size_t plain_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
-  if (const size_t skinny = gemv_forward_workspace(m, rows, cols, dtype)) return skinny;
+  if (gemv_takes(m, rows, cols, dtype)) return gemv_forward_workspace(m, rows, cols, dtype);
   return dtype == QSTE_F32 ? f32_forward_workspace(m, rows, cols) : mfma_forward_split_workspace(m, rows, cols, dtype);
 }
 

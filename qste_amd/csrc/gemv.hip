@@ -550,6 +550,9 @@ void launch_xr(int nbw, const Args& p, bool resident, hipStream_t stream) {
 // Rows of x a launch takes: four tiles of 16, or 21 rows of three limbs.
 constexpr int64_t kRows16 = 64, kRows32 = 21;
 
+// Blocks of weights a plan that splits K has at most (two per CU).
+constexpr int64_t kSplitBlocks = 2 * 256;
+
 struct Plan {
   int nbw, splits, chunks_per_split;
 };
@@ -570,7 +573,7 @@ Plan plan_of(int64_t xr, int64_t rows, int64_t cols, bool may_split) {
   const int64_t blocks = (rows + 15) / 16, chunks = (cols + CHUNK_K - 1) / CHUNK_K;
   const int64_t most = most_blocks(static_cast<int>(xr)), tiles = (xr + 15) / 16;
   int64_t splits = 1, per = chunks;
-  if (may_split && blocks <= 2 * 256) {
+  if (may_split && blocks <= kSplitBlocks) {
     double best = 0.0;
     for (int64_t s = 2; s <= 4 && 2 * s <= chunks; s *= 2) {
       const int64_t cps = (chunks + s - 1) / s, ns = (chunks + cps - 1) / cps;
@@ -621,16 +624,19 @@ size_t up256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 int launch_limbs(const float*, int64_t, int64_t, uint16_t*, hipStream_t);
 
+// Whether a product of these sizes is for this path.
+bool gemv_takes(int64_t m, int64_t rows, int64_t cols, int dtype) { return gemv::x_rows(dtype, m, rows, cols) > 0; }
+
 // Workspace of a product on this path: fp32 x's limbs, and the range sums of
-// the plan (past 16 rows of two ranges at least, so that the size does not
-// depend on where the plan's line lies); 0 where none is needed or the
-// product is not for this path.
+// the plan (past 16 rows two ranges wherever the blocks are few enough for any
+// plan to split, so that the size does not depend on where the plan's line
+// lies); 0 where none is needed or the product is not for this path.
 size_t gemv_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
   const int64_t xr = gemv::x_rows(dtype, m, rows, cols);
   if (xr == 0) return 0;
   const gemv::Plan plan = gemv::plan_of(xr, rows, cols, true);
   int64_t ranges = plan.splits > 1 ? plan.splits : 0;
-  if (m > 16 && ranges < 2) ranges = 2;
+  if (m > 16 && ranges < 2 && (rows + 15) / 16 <= gemv::kSplitBlocks) ranges = 2;
   return (dtype == QSTE_F32 ? gemv::up256(static_cast<size_t>(xr * cols) * 2) : 0) +
          static_cast<size_t>(ranges * xr * rows) * sizeof(float);
 }

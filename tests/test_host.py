@@ -112,6 +112,20 @@ def test_error_codes_and_workspace_queries_need_no_gpu():
                                       64, 1, 0, None, None, None, None, 0, None) == -3
 
 
+def test_skinny_forward_asks_for_no_space_it_cannot_use():
+    """Up to 64 rows only a layer of at most 512 blocks of 16 weight rows can
+    have its K cut into ranges; a wider one asks for no range sums."""
+
+    from qste_amd.kernels import _lib
+
+    query = _lib.load().qste_packed_linear_affine_workspace_bytes
+    for rows in (8208, 14336, 28672, 50257):
+        for m in (1, 16, 17, 40, 64):
+            assert query(m, rows, 4096, 2) == 0, (rows, m)
+        assert query(21, rows, 4096, 0) == 63 * 4096 * 2  # the limbs of x alone
+    assert 0 < query(64, 8192, 4096, 2) <= 4 * 64 * 8192 * 4
+
+
 def test_fp32_limb_workspaces_are_capped_and_shared():
     """The fp32 products' bf16 limbs (6 bytes per dense value) are held to
     512 MiB: forward and input gradient in chunks of output rows, an
