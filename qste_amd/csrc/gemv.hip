@@ -165,10 +165,14 @@ __device__ __forceinline__ void finish4(const Args& p, int64_t m, int64_t n, f32
 
 // XR rows of x are staged (>= p.xr: 4 or a multiple of 16; rows past p.xr
 // are left as they are, their outputs are never stored), NBW blocks of 16
-// weight rows per workgroup.  RESIDENT: a chunk's fragments are all formed
-// first and the blocks streamed past them.
-template <int XR, int NBW, bool RESIDENT>
+// weight rows per workgroup.
+template <int XR, int NBW>
 struct Cfg {
+  // A chunk's fragments of one tile of x are all formed first and the blocks
+  // streamed past them: pays from three blocks on (28672 x 8192, M = 1: 10.3
+  // against 12.7 us; 4096 x 4096, one block: 3.9 both ways; 4096 x 14336: 7.7
+  // against 7.2)
+  static constexpr bool RESIDENT = XR <= 16 && NBW >= 3;
   static constexpr int MT = (XR + 15) / 16;                     // MFMA columns / 16
   static constexpr int STAGES = XR <= 16 ? 1 : 4;               // x stages per chunk
   static constexpr int JS = 4 / STAGES;
@@ -184,13 +188,12 @@ struct Cfg {
   static constexpr int bytes = WAVES * x_bytes > red_bytes ? WAVES * x_bytes : red_bytes;
   // weight loads in flight: a chunk's, or two where blocks are streamed (the
   // CUs' streams stay interleaved; 4 in flight: 4-6% slower at M = 1)
-  static constexpr int D = !RESIDENT ? NBW : (NBW < 2 ? NBW : 2);
+  static constexpr int D = RESIDENT ? 2 : NBW;
 };
 
-template <int DT, int XR, int NBW, bool RESIDENT>
+template <int DT, int XR, int NBW>
 __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
-  using C = Cfg<XR, NBW, RESIDENT>;
-  static_assert(!RESIDENT || XR <= 16, "fragments of one tile fit the registers");
+  using C = Cfg<XR, NBW>;
   constexpr int MT = C::MT, JS = C::JS, D = C::D;
   __shared__ __attribute__((aligned(16))) uint8_t smem[C::bytes];
   __shared__ float epi[2][16 * NBW];
@@ -297,7 +300,7 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
     out_scale = p.scale[n0 + tid];
     out_bias = p.bias ? p.bias[n0 + tid] : 0.0f;
   }
-  if constexpr (RESIDENT) {
+  if constexpr (C::RESIDENT) {
     for (; c < c_last; c += WAVES) {
       wait_vm<D>();  // all but the newest loads, the weights in flight: x is in LDS
       u32x8 f[4][2][2];
@@ -323,12 +326,10 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
 #pragma unroll
       for (int b = 0; b < NBW; ++b) {
         const u32x4 w = W[b];
-        auto next = [&] {  // the load D blocks ahead
-          if (b + D < NBW) W[b + D] = issue_w1(c, b + D);
-          else W[b + D - NBW] = issue_w1(c + WAVES, b + D - NBW);
-          __builtin_amdgcn_sched_barrier(0);
-        };
-        if (D < NBW) next();
+        // the load D blocks ahead
+        if (b + D < NBW) W[b + D] = issue_w1(c, b + D);
+        else W[b + D - NBW] = issue_w1(c + WAVES, b + D - NBW);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t e = even_index(w[j]), o = odd_index(w[j]);
@@ -338,7 +339,6 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
           acc[b][0] = Op<DT>::template mma<1>(ones, f[j][1][1], acc[b][0], o);
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (D == NBW) next();
       }
     }
   } else {
@@ -515,15 +515,9 @@ __global__ __launch_bounds__(256) void combine_kernel(Args p) {
 }
 
 template <int DT, int XR, int NBW>
-void launch(const Args& p, bool resident, hipStream_t stream) {
+void launch(const Args& p, hipStream_t stream) {
   const int groups = static_cast<int>((p.N + 16 * NBW - 1) / (16 * NBW));
-  if constexpr (XR <= 16) {
-    if (resident) {
-      skinny_kernel<DT, XR, NBW, true><<<groups * p.splits, THREADS, 0, stream>>>(p);
-      return;
-    }
-  }
-  skinny_kernel<DT, XR, NBW, false><<<groups * p.splits, THREADS, 0, stream>>>(p);
+  skinny_kernel<DT, XR, NBW><<<groups * p.splits, THREADS, 0, stream>>>(p);
 }
 
 // Weight blocks per workgroup at most: what the waves' accumulators and their
@@ -531,20 +525,20 @@ void launch(const Args& p, bool resident, hipStream_t stream) {
 constexpr int most_blocks(int xr) { return xr <= 32 ? 8 : (xr <= 48 ? 6 : 4); }
 
 template <int DT, int XR, int NBW = 1>
-void launch_nbw(int nbw, const Args& p, bool resident, hipStream_t stream) {
+void launch_nbw(int nbw, const Args& p, hipStream_t stream) {
   if constexpr (NBW < most_blocks(XR)) {
-    if (nbw > NBW) return launch_nbw<DT, XR, NBW + 1>(nbw, p, resident, stream);
+    if (nbw > NBW) return launch_nbw<DT, XR, NBW + 1>(nbw, p, stream);
   }
-  launch<DT, XR, NBW>(p, resident, stream);
+  launch<DT, XR, NBW>(p, stream);
 }
 
 template <int DT>
-void launch_xr(int nbw, const Args& p, bool resident, hipStream_t stream) {
-  if (p.xr <= 4) launch_nbw<DT, 4>(nbw, p, resident, stream);
-  else if (p.xr <= 16) launch_nbw<DT, 16>(nbw, p, resident, stream);
-  else if (p.xr <= 32) launch_nbw<DT, 32>(nbw, p, resident, stream);
-  else if (p.xr <= 48) launch_nbw<DT, 48>(nbw, p, resident, stream);
-  else launch_nbw<DT, 64>(nbw, p, resident, stream);
+void launch_xr(int nbw, const Args& p, hipStream_t stream) {
+  if (p.xr <= 4) launch_nbw<DT, 4>(nbw, p, stream);
+  else if (p.xr <= 16) launch_nbw<DT, 16>(nbw, p, stream);
+  else if (p.xr <= 32) launch_nbw<DT, 32>(nbw, p, stream);
+  else if (p.xr <= 48) launch_nbw<DT, 48>(nbw, p, stream);
+  else launch_nbw<DT, 64>(nbw, p, stream);
 }
 
 // Rows of x a launch takes: four tiles of 16, or 21 rows of three limbs.
@@ -605,10 +599,7 @@ int64_t x_rows(int dtype, int64_t m, int64_t rows, int64_t cols) {
 
 template <int DT>
 int run(const Args& p, const Plan& plan, bool fp32, hipStream_t stream) {
-  // streaming blocks past resident fragments pays from three blocks on
-  // (28672 x 8192, M = 1: 10.3 against 12.7 us; 4096 x 4096, one block: 3.9
-  // both ways; 4096 x 14336: 7.7 against 7.2)
-  launch_xr<DT>(plan.nbw, p, plan.nbw >= 3, stream);
+  launch_xr<DT>(plan.nbw, p, stream);
   int rc = static_cast<int>(hipGetLastError());
   if (rc || p.splits == 1) return rc;
   const int64_t items = p.xr / p.limbs * ((p.N + 3) / 4);
