@@ -165,16 +165,19 @@ __device__ __forceinline__ void finish4(const Args& p, int64_t m, int64_t n, f32
 
 // XR rows of x are staged (>= p.xr: 4 or a multiple of 16; rows past p.xr
 // are left as they are, their outputs are never stored), NBW blocks of 16
-// weight rows per workgroup.
-template <int XR, int NBW>
+// weight rows per workgroup.  STAGED: x arrives in four stages a chunk, as it
+// has to past 16 rows; up to 16 rows that is for fp32, whose rows then share
+// one order of sums whatever their number.
+template <int XR, int NBW, bool STAGED>
 struct Cfg {
+  static_assert(STAGED || XR <= 16, "whole chunks of more rows do not fit");
   // A chunk's fragments of one tile of x are all formed first and the blocks
   // streamed past them: pays from three blocks on (28672 x 8192, M = 1: 10.3
   // against 12.7 us; 4096 x 4096, one block: 3.9 both ways; 4096 x 14336: 7.7
   // against 7.2)
-  static constexpr bool RESIDENT = XR <= 16 && NBW >= 3;
+  static constexpr bool RESIDENT = !STAGED && NBW >= 3;
   static constexpr int MT = (XR + 15) / 16;                     // MFMA columns / 16
-  static constexpr int STAGES = XR <= 16 ? 1 : 4;               // x stages per chunk
+  static constexpr int STAGES = STAGED ? 4 : 1;                 // x stages per chunk
   static constexpr int JS = 4 / STAGES;
   // one stage: whole chunks of a row (1 KB and a pad: the 16 rows of a
   // fragment read cover all banks), or 256 bytes of a row (16-byte piece i of
@@ -191,9 +194,9 @@ struct Cfg {
   static constexpr int D = RESIDENT ? 2 : NBW;
 };
 
-template <int DT, int XR, int NBW>
+template <int DT, int XR, int NBW, bool STAGED>
 __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
-  using C = Cfg<XR, NBW>;
+  using C = Cfg<XR, NBW, STAGED>;
   constexpr int MT = C::MT, JS = C::JS, D = C::D;
   __shared__ __attribute__((aligned(16))) uint8_t smem[C::bytes];
   __shared__ float epi[2][16 * NBW];
@@ -480,13 +483,13 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
   }
 }
 
-// splits > 1: the range sums added in range order (and each row's limbs,
-// smallest first), then scale, bias and one rounding; four outputs a thread.
-template <int OUT>
+// splits > 1 (16-bit x): the range sums added in range order, then scale, bias
+// and one rounding; four outputs a thread.
+template <int DT>
 __global__ __launch_bounds__(256) void combine_kernel(Args p) {
-  const int64_t quads = (p.N + 3) / 4, rows = p.xr / p.limbs;
+  const int64_t quads = (p.N + 3) / 4;
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= rows * quads) return;
+  if (i >= p.xr * quads) return;
   const int64_t m = i / quads, n = 4 * (i - m * quads);
   const bool full = (p.N & 3) == 0;
   float sc[4], bi[4];
@@ -496,49 +499,43 @@ __global__ __launch_bounds__(256) void combine_kernel(Args p) {
     bi[j] = n + j < p.N && p.bias ? p.bias[n + j] : 0.0f;
   }
   f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int l = p.limbs - 1; l >= 0; --l) {
-    f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s = 0; s < p.splits; ++s) {
-      const float* d = p.partial + (static_cast<int64_t>(s) * p.xr + m * p.limbs + l) * p.N + n;
-      if (full) {
-        t += *reinterpret_cast<const f32x4*>(d);
-      } else {
+  for (int s = 0; s < p.splits; ++s) {
+    const float* d = p.partial + (static_cast<int64_t>(s) * p.xr + m) * p.N + n;
+    if (full) {
+      v += *reinterpret_cast<const f32x4*>(d);
+    } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (n + j < p.N) t[j] += d[j];
-      }
+      for (int j = 0; j < 4; ++j)
+        if (n + j < p.N) v[j] += d[j];
     }
-    v = v + t;
   }
-  const bool vec = full && (reinterpret_cast<uintptr_t>(p.y) & (OUT == QSTE_F32 ? 15 : 7)) == 0;
-  finish4<OUT>(p, m, n, v, sc, bi, vec);
-}
-
-template <int DT, int XR, int NBW>
-void launch(const Args& p, hipStream_t stream) {
-  const int groups = static_cast<int>((p.N + 16 * NBW - 1) / (16 * NBW));
-  skinny_kernel<DT, XR, NBW><<<groups * p.splits, THREADS, 0, stream>>>(p);
+  const bool vec = full && (reinterpret_cast<uintptr_t>(p.y) & 7) == 0;
+  finish4<DT>(p, m, n, v, sc, bi, vec);
 }
 
 // Weight blocks per workgroup at most: what the waves' accumulators and their
 // image in LDS at the end have room for.
 constexpr int most_blocks(int xr) { return xr <= 32 ? 8 : (xr <= 48 ? 6 : 4); }
 
-template <int DT, int XR, int NBW = 1>
+template <int DT, int XR, bool STAGED, int NBW = 1>
 void launch_nbw(int nbw, const Args& p, hipStream_t stream) {
   if constexpr (NBW < most_blocks(XR)) {
-    if (nbw > NBW) return launch_nbw<DT, XR, NBW + 1>(nbw, p, stream);
+    if (nbw > NBW) return launch_nbw<DT, XR, STAGED, NBW + 1>(nbw, p, stream);
   }
-  launch<DT, XR, NBW>(p, stream);
+  const int groups = static_cast<int>((p.N + 16 * NBW - 1) / (16 * NBW));
+  skinny_kernel<DT, XR, NBW, STAGED><<<groups * p.splits, THREADS, 0, stream>>>(p);
 }
 
 template <int DT>
 void launch_xr(int nbw, const Args& p, hipStream_t stream) {
-  if (p.xr <= 4) launch_nbw<DT, 4>(nbw, p, stream);
-  else if (p.xr <= 16) launch_nbw<DT, 16>(nbw, p, stream);
-  else if (p.xr <= 32) launch_nbw<DT, 32>(nbw, p, stream);
-  else if (p.xr <= 48) launch_nbw<DT, 48>(nbw, p, stream);
-  else launch_nbw<DT, 64>(nbw, p, stream);
+  if constexpr (DT == QSTE_BF16) {
+    if (p.limbs == 3 && p.xr <= 16) return launch_nbw<DT, 16, true>(nbw, p, stream);
+  }
+  if (p.xr <= 4) launch_nbw<DT, 4, false>(nbw, p, stream);
+  else if (p.xr <= 16) launch_nbw<DT, 16, false>(nbw, p, stream);
+  else if (p.xr <= 32) launch_nbw<DT, 32, true>(nbw, p, stream);
+  else if (p.xr <= 48) launch_nbw<DT, 48, true>(nbw, p, stream);
+  else launch_nbw<DT, 64, true>(nbw, p, stream);
 }
 
 // Rows of x a launch takes: four tiles of 16, or 21 rows of three limbs.
@@ -559,21 +556,25 @@ struct Plan {
 // rows: 192 VALU instructions) and x's reads from L2 (0.0085 us per chunk and
 // row) bound the kernel, not the weights; S ranges cut both S-fold, and cost
 // a second launch and the sums' round trip, a little more for more ranges.
-// Measured, one range against the best split: 8192 x 28672, M = 16: 19.9 / 18.1
-// us (two ranges; four 17.9), M = 40: 40.6 / 31.9;
-// 4096 x 14336, M = 24: 14.4 / 13.0, M = 16: 9.8 / 10.4 (not split); three
+// Measured, one range against the best split: 8192 x 28672, M = 40: 40.6 / 31.9
+// us; 4096 x 14336, M = 24: 14.4 / 13.0; three
 // blocks and more (14336 x 4096, M = 40: 11.8 / 20.8) are never split.
+//
+// A row's sums are in an order of its own K alone, not of how many other rows
+// the call brings: up to 16 rows are never cut (8192 x 28672, M = 16: 14.4 cut in
+// two, 15.2 whole), nor are fp32 rows, and past 16 the line is drawn for the
+// instance's last row (32, 48, 64), so only those steps change a row's bits.
 Plan plan_of(int64_t xr, int64_t rows, int64_t cols, bool may_split) {
   const int64_t blocks = (rows + 15) / 16, chunks = (cols + CHUNK_K - 1) / CHUNK_K;
   const int64_t most = most_blocks(static_cast<int>(xr)), tiles = (xr + 15) / 16;
   int64_t splits = 1, per = chunks;
-  if (may_split && blocks <= kSplitBlocks) {
+  if (may_split && xr > 16 && blocks <= kSplitBlocks) {
     double best = 0.0;
     for (int64_t s = 2; s <= 4 && 2 * s <= chunks; s *= 2) {
       const int64_t cps = (chunks + s - 1) / s, ns = (chunks + cps - 1) / cps;
       if ((blocks * ns + 255) / 256 > most) continue;  // a second round
-      const double saved = static_cast<double>(chunks - cps) * (0.087 * tiles + 0.0085 * xr);
-      const double cost = 4.5 + 1.3 * static_cast<double>(ns - 2) + static_cast<double>(ns * xr * rows) * 8.0 / 4e6;
+      const double saved = static_cast<double>(chunks - cps) * tiles * (0.087 + 16 * 0.0085);
+      const double cost = 4.5 + 1.3 * static_cast<double>(ns - 2) + static_cast<double>(ns * 16 * tiles * rows) * 8.0 / 4e6;
       if (saved - cost > best) {
         best = saved - cost;
         splits = ns;
@@ -598,14 +599,12 @@ int64_t x_rows(int dtype, int64_t m, int64_t rows, int64_t cols) {
 }
 
 template <int DT>
-int run(const Args& p, const Plan& plan, bool fp32, hipStream_t stream) {
+int run(const Args& p, const Plan& plan, hipStream_t stream) {
   launch_xr<DT>(plan.nbw, p, stream);
   int rc = static_cast<int>(hipGetLastError());
   if (rc || p.splits == 1) return rc;
-  const int64_t items = p.xr / p.limbs * ((p.N + 3) / 4);
-  const int grid = static_cast<int>((items + 255) / 256);
-  if (fp32) combine_kernel<QSTE_F32><<<grid, 256, 0, stream>>>(p);
-  else combine_kernel<DT><<<grid, 256, 0, stream>>>(p);
+  const int64_t items = p.xr * ((p.N + 3) / 4);
+  combine_kernel<DT><<<static_cast<int>((items + 255) / 256), 256, 0, stream>>>(p);
   return static_cast<int>(hipGetLastError());
 }
 
@@ -625,10 +624,11 @@ bool gemv_takes(int64_t m, int64_t rows, int64_t cols, int dtype) { return gemv:
 size_t gemv_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
   const int64_t xr = gemv::x_rows(dtype, m, rows, cols);
   if (xr == 0) return 0;
-  const gemv::Plan plan = gemv::plan_of(xr, rows, cols, true);
+  const bool fp32 = dtype == QSTE_F32;
+  const gemv::Plan plan = gemv::plan_of(xr, rows, cols, !fp32);
   int64_t ranges = plan.splits > 1 ? plan.splits : 0;
-  if (m > 16 && ranges < 2 && (rows + 15) / 16 <= gemv::kSplitBlocks) ranges = 2;
-  return (dtype == QSTE_F32 ? gemv::up256(static_cast<size_t>(xr * cols) * 2) : 0) +
+  if (!fp32 && m > 16 && ranges < 2 && (rows + 15) / 16 <= gemv::kSplitBlocks) ranges = 2;
+  return (fp32 ? gemv::up256(static_cast<size_t>(xr * cols) * 2) : 0) +
          static_cast<size_t>(ranges * xr * rows) * sizeof(float);
 }
 
@@ -645,7 +645,7 @@ int gemv_linear_forward(const void* x, int dtype, const uint8_t* packed, const f
   const bool room = workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
                     workspace_bytes >= gemv_forward_workspace(m, rows, cols, dtype);
   if (fp32 && !room) return 1;
-  const gemv::Plan plan = gemv::plan_of(xr, rows, cols, room);
+  const gemv::Plan plan = gemv::plan_of(xr, rows, cols, room && !fp32);
   gemv::Args p{};
   p.x = static_cast<const uint16_t*>(x);
   p.bits = packed;
@@ -667,8 +667,7 @@ int gemv_linear_forward(const void* x, int dtype, const uint8_t* packed, const f
     ws += gemv::up256(static_cast<size_t>(p.xr * cols) * 2);
   }
   p.partial = reinterpret_cast<float*>(ws);
-  return dtype == QSTE_F16 ? gemv::run<QSTE_F16>(p, plan, false, stream)
-                           : gemv::run<QSTE_BF16>(p, plan, fp32, stream);
+  return dtype == QSTE_F16 ? gemv::run<QSTE_F16>(p, plan, stream) : gemv::run<QSTE_BF16>(p, plan, stream);
 }
 
 }  // namespace qste

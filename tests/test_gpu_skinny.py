@@ -114,6 +114,27 @@ def test_few_rows_over_many_chunks(rows, cols, m, dtype):
     _check(got[:, torch.from_numpy(pick).to(DEV)], x, np.ascontiguousarray(packed[pick]), scale[pick], bias[pick], cols)
 
 
+@pytest.mark.parametrize("rows,cols,dtype,steps", [
+    (8192, 28672, torch.bfloat16, (1, 4, 5, 16)), (300, 8192, torch.float16, (1, 2, 16)),
+    (14336, 4096, torch.bfloat16, (1, 3, 11, 16)), (4096, 14336, torch.float16, (17, 24, 32)),
+    (1000, 8192, torch.bfloat16, (33, 40, 48)), (8192, 16384, torch.bfloat16, (49, 64)),
+    (2048, 2048, torch.float32, (1, 5, 6, 11, 21)), (1000, 8192, torch.float32, (1, 2, 16, 17, 21))])
+def test_a_rows_bits_do_not_depend_on_the_batch(rows, cols, dtype, steps):
+    """The first row of a call is bit for bit the same however many rows come
+    with it (up to 16, and inside each of the larger instances; in fp32 up to
+    21): K is cut, and its chunks are added, by the layer's sizes alone."""
+
+    from qste_amd import kernels
+
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    tp = torch.randint(0, 256, (rows, cols // 8), generator=g, device=DEV, dtype=torch.uint8)
+    ts = torch.rand(rows, generator=g, device=DEV) * 0.02 + 0.01
+    tx = torch.randn(steps[-1], cols, generator=g, device=DEV).to(dtype)
+    ys = [kernels.packed_linear_affine(tx[:m].contiguous(), tp, ts, None, cols) for m in steps]
+    for m, y in zip(steps, ys):
+        assert torch.equal(y, ys[-1][:m]), m
+
+
 @pytest.mark.parametrize("rows,cols,m", [(8192, 28672, 16), (1000, 8192, 64), (4096, 14336, 24)])
 def test_split_plans_are_deterministic(rows, cols, m):
     """Shapes whose plan splits K: two calls agree bit for bit, and with the
