@@ -57,7 +57,8 @@ int launch_colsums_pad(const void*, int, const float*, int64_t, int64_t, int64_t
                        float*, hipStream_t);
 int launch_backward_prep(const void*, int, const float*, int64_t, int64_t, float*, float*, float*, float*,
                          const TransposeJob&, const ScaleJob&, const TransposeJob&, const ScaleJob&, hipStream_t);
-bool gemv_takes(int64_t, int64_t, int64_t, int);
+double gemv_forward_us(int64_t, int64_t, int64_t, int);
+double mfma_forward_us(int64_t, int64_t, int64_t, bool);
 size_t gemv_forward_workspace(int64_t, int64_t, int64_t, int);
 int gemv_linear_forward(const void*, int, const uint8_t*, const float*, const float*, void*, int64_t, int64_t,
                         int64_t, void*, size_t, hipStream_t);
@@ -172,9 +173,66 @@ BackwardLayout backward_layout(int64_t samples, int64_t rows, int64_t cols, Layo
   return l;
 }
 
+size_t elem_bytes(int dtype) { return dtype == QSTE_F32 ? 4 : 2; }
+
+// How a forward runs.
+struct ForwardRoute {
+  bool skinny;     // on the skinny kernel (up to 64 rows, 21 of fp32)
+  int64_t padded;  // on copies of x and the signs of this many columns, 0: as they are
+};
+
+// The columns that the copies of a ragged layer have: rows of whole 16-byte
+// words of signs, zeros behind the data (a zero x times either sign adds
+// nothing).
+int64_t padded_cols(int64_t cols) { return (cols + 127) / 128 * 128; }
+
+// Time of those copies in us: their two launches, and the signs' traffic
+// (4096 x 832: 5.3, 50257 x 4160: 18).
+double padding_us(int64_t rows, int64_t cols) {
+  return 5.3 + static_cast<double>(rows * ((cols + 7) / 8 + padded_cols(cols) / 8)) / 4e6;
+}
+
+// Up to 64 rows the skinny kernel reads x once per workgroup and spends its time
+// on the outputs where K is short, so a wide layer of short K is faster on the
+// tiles, and so are widths that the tiles take as they are and the skinny
+// kernel on copies only.  The estimates decide, for the same number of rows
+// throughout an instance of the kernel.  Measured in us, skinny kernel / tiles:
+// 50257 x 768, 16 rows 11 / 12, 32 rows 18 / 13, 64 rows 40 / 14; 50257 x 4096, 32
+// rows 25 / 41, 64 rows 56 / 43; 4096 x 768, 64 rows 8 / 12; 4096 x 320 on copies,
+// 16 rows 8.8 / 7.7, 4096 x 1600 9.2 / 18.8.  fp32 rows have the scalar kernel
+// instead of the tiles (about 0.125 us a column, or 25 TFLOP/s): 50257 x 128, 21
+// rows 41 / 21, 50257 x 256 41 / 36, 2048 x 256 7 / 36.
+//
+// Past 64 rows a ragged 16-bit layer goes to the tiles on copies once its K pays
+// for them: the scalar kernel's time is its K chain, about 2.3 us per 16
+// columns, and the copies and the product take 24-29 us (128 x 300 x 300: 45 -> 24,
+// 2048 x 1000 x 3000: 503 -> 46, but 1000 x 130 x 130: 24 / 26).
+ForwardRoute forward_route(int64_t m, int64_t rows, int64_t cols, int dtype) {
+  if (m <= 0 || rows <= 0 || cols <= 64) return {false, 0};
+  const int64_t wide = padded_cols(cols);
+  const double skinny = gemv_forward_us(m, rows, wide, dtype);
+  const int64_t copies = cols % 128 != 0 ? wide : 0;
+  const double ragged = copies ? padding_us(rows, cols) : 0.0;
+  if (dtype == QSTE_F32) {
+    // past 21 rows the limb copies pad by themselves
+    if (skinny < 0.0) return {false, 0};
+    const double chain = 0.125 * static_cast<double>(cols), rate = 42.0 * static_cast<double>(rows) * cols / 50e6;
+    const bool take = skinny + ragged < (chain > rate ? chain : rate) + 4.0;
+    return {take, take ? copies : 0};
+  }
+  const bool whole = cols % 64 == 0;  // the tiles take it as it is
+  if (skinny < 0.0) return {false, whole || cols <= 160 ? 0 : wide};
+  const double tiles = mfma_forward_us(m <= 16 ? 16 : (m + 15) / 16 * 16, rows, whole ? cols : wide, m > 16) +
+                       (whole ? 0.0 : ragged);
+  if (skinny + ragged < tiles) return {true, copies};
+  return {false, whole ? 0 : wide};
+}
+
 int forward_dispatch(const void* x, int dtype, const uint8_t* packed, const float* scale,
                      const float* bias, void* y, int64_t m, int64_t rows, int64_t cols, hipStream_t s) {
-  int rc = gemv_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, nullptr, 0, s);
+  int rc = forward_route(m, rows, cols, dtype).skinny
+               ? gemv_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, nullptr, 0, s)
+               : 1;
   if (rc != 1) return rc;
   rc = mfma_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, s);
   if (rc != 1) return rc;
@@ -273,36 +331,15 @@ int qste_packed_linear_affine(const void* x, int dtype, const uint8_t* packed, c
 
 namespace {
 
-// A forward whose columns no matrix path takes (a multiple of 64; of 128 up to
-// 64 rows, 21 of fp32) runs it on copies of x and the signs that are padded
-// with zeros (a zero x times either sign adds nothing).  The scalar kernel's
-// time is its K chain, about 2.3 us per 16 columns; the copies and the product
-// take 9-13 us up to 64 rows (64 x 300 x 130: 23.5 -> 12.3, 32 x 65 x 65: 14.2
-// -> 9.4) and 24-29 us on 256-row tiles (128 x 300 x 300: 45 -> 24, 2048 x 1000
-// x 3000: 503 -> 46, but 1000 x 130 x 130: 24 / 26): hence the two lines.
-int64_t padded_forward_cols(int64_t m, int64_t rows, int64_t cols, int dtype) {
-  if (m <= 0 || rows <= 0) return 0;
-  if (dtype == QSTE_F32) {
-    // past 21 rows the limb copies pad by themselves
-    if (m > 21 || cols <= 64 || cols % 128 == 0) return 0;
-  } else {
-    if (cols <= (m <= 64 ? 64 : 160) || cols % (m <= 64 ? 128 : 64) == 0) return 0;
-  }
-  // the copies are rows of whole 16-byte words of signs
-  return (cols + 127) / 128 * 128;
-}
-
-size_t elem_bytes(int dtype) { return dtype == QSTE_F32 ? 4 : 2; }
-
 size_t plain_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) {
-  if (gemv_takes(m, rows, cols, dtype)) return gemv_forward_workspace(m, rows, cols, dtype);
+  if (forward_route(m, rows, cols, dtype).skinny) return gemv_forward_workspace(m, rows, cols, dtype);
   return dtype == QSTE_F32 ? f32_forward_workspace(m, rows, cols) : mfma_forward_split_workspace(m, rows, cols, dtype);
 }
 
 }  // namespace
 
 size_t qste_packed_linear_affine_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int dtype) {
-  if (const int64_t pc = padded_forward_cols(m, rows, cols, dtype))
+  if (const int64_t pc = forward_route(m, rows, cols, dtype).padded)
     return align_up(static_cast<size_t>(m * pc) * elem_bytes(dtype)) + align_up(static_cast<size_t>(rows * pc / 8)) +
            plain_forward_workspace(m, rows, pc, dtype);
   return plain_forward_workspace(m, rows, cols, dtype);
@@ -315,7 +352,8 @@ int qste_packed_linear_affine_ws(const void* x, int dtype, const uint8_t* packed
   if (m < 0 || rows < 0 || cols < 0) return QSTE_E_SHAPE;
   if (m * rows == 0) return 0;
   if (!y || !scale || (cols > 0 && (!x || !packed))) return QSTE_E_NULL;
-  const int64_t pc = padded_forward_cols(m, rows, cols, dtype);
+  const ForwardRoute route = forward_route(m, rows, cols, dtype);
+  const int64_t pc = route.padded;
   if (pc && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
       workspace_bytes >= qste_packed_linear_affine_workspace_bytes(m, rows, cols, dtype)) {
     hipStream_t s = as_stream(stream);
@@ -328,7 +366,7 @@ int qste_packed_linear_affine_ws(const void* x, int dtype, const uint8_t* packed
     return qste_packed_linear_affine_ws(xp, dtype, reinterpret_cast<uint8_t*>(wp), scale, bias, y, m, rows, pc,
                                         wp + wb, workspace_bytes - xb - wb, stream);
   }
-  if (cols > 0) {
+  if (route.skinny) {
     const int rc = gemv_linear_forward(x, dtype, packed, scale, bias, y, m, rows, cols, workspace, workspace_bytes,
                                        as_stream(stream));
     if (rc != 1) return rc;

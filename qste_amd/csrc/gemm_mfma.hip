@@ -1174,6 +1174,11 @@ int mfma_linear_forward(const void* x, int dtype, const uint8_t* packed, const f
   return static_cast<int>(hipGetLastError());
 }
 
+// Time of a 16-bit forward on the tiles in us (K rounded up to whole steps).
+double mfma_forward_us(int64_t m, int64_t rows, int64_t cols, bool may_split) {
+  return product_plan(m, rows, static_cast<int>((cols + mfma::wide::BK - 1) / mfma::wide::BK), may_split).us;
+}
+
 static size_t split_bytes(const SplitK& sp, int tiles) {
   return sp.splits > 1 ? static_cast<size_t>(sp.splits) * tiles * mfma::wide::BM * mfma::wide::BN * sizeof(float) : 0;
 }

@@ -561,8 +561,8 @@ struct Plan {
 // blocks and more (14336 x 4096, M = 40: 11.8 / 20.8) are never split.
 //
 // A row's sums are in an order of its own K alone, not of how many other rows
-// the call brings: up to 16 rows are never cut (8192 x 28672, M = 16: 14.4 cut in
-// two, 15.2 whole), nor are fp32 rows, and past 16 the line is drawn for the
+// the call brings: up to 16 rows are never cut (8192 x 28672, M = 16: 14.5 us cut in
+// two, 16.1 whole), nor are fp32 rows, and past 16 the line is drawn for the
 // instance's last row (32, 48, 64), so only those steps change a row's bits.
 Plan plan_of(int64_t xr, int64_t rows, int64_t cols, bool may_split) {
   const int64_t blocks = (rows + 15) / 16, chunks = (cols + CHUNK_K - 1) / CHUNK_K;
@@ -585,6 +585,25 @@ Plan plan_of(int64_t xr, int64_t rows, int64_t cols, bool may_split) {
   const int64_t work = blocks * splits, rounds = (work + 256 * most - 1) / (256 * most);
   int64_t nbw = (work + 256 * rounds - 1) / (256 * rounds);
   return Plan{static_cast<int>(nbw < 1 ? 1 : nbw), static_cast<int>(splits), static_cast<int>(per)};
+}
+
+// Time of a call in us with xr rows of x, fitted to 1000 measured products (300
+// to 128256 rows of weights over 128 to 28672 columns): 90% of the times are
+// within 13% of it.  A round of workgroups takes a fixed time, the sums and
+// outputs of its blocks (first two terms), and per chunk x's reads, the MFMAs
+// and a wave's chain.
+double estimate(int64_t xr, const Plan& plan, int64_t rows, bool staged) {
+  struct Rates {
+    double call, round, block, read, mma, chain;
+  };
+  const Rates t = staged ? Rates{1.6, 0.87, 0.317, 0.0055, 0.0255, 1.42} : Rates{1.4, 1.16, 0.172, 0.0064, 0.007, 0.84};
+  const double tiles = static_cast<double>((xr + 15) / 16), per = static_cast<double>(plan.chunks_per_split);
+  const int64_t groups = (rows + 16 * plan.nbw - 1) / (16 * plan.nbw) * plan.splits;
+  const double combine = plan.splits > 1 ? 3.0 + static_cast<double>(plan.splits * xr * rows) * 8.0 / 3.3e6 : 0.0;
+  return t.call + combine +
+         static_cast<double>((groups + 255) / 256) *
+             (t.round + plan.nbw * tiles * (t.block + t.mma * per) + t.read * per * static_cast<double>(xr) +
+              t.chain * static_cast<double>((plan.chunks_per_split + WAVES - 1) / WAVES));
 }
 
 // Rows of 16-bit x that m rows make (three limbs for an fp32 row), 0 when
@@ -614,8 +633,17 @@ size_t up256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 int launch_limbs(const float*, int64_t, int64_t, uint16_t*, hipStream_t);
 
-// Whether a product of these sizes is for this path.
-bool gemv_takes(int64_t m, int64_t rows, int64_t cols, int dtype) { return gemv::x_rows(dtype, m, rows, cols) > 0; }
+// Time of a product on this path in us, negative when its sizes are not for it.
+// It is the time of the instance's last row (16, 32, 48 or 64; 21 in fp32): a
+// choice made by it does not change with the rows a call brings along.
+double gemv_forward_us(int64_t m, int64_t rows, int64_t cols, int dtype) {
+  const int64_t xr = gemv::x_rows(dtype, m, rows, cols);
+  if (xr == 0) return -1.0;
+  const bool fp32 = dtype == QSTE_F32;
+  const int64_t top = fp32 ? 3 * gemv::kRows32 : (xr + 15) / 16 * 16;
+  // (fp32: the limbs of x are a launch of their own)
+  return gemv::estimate(top, gemv::plan_of(top, rows, cols, !fp32), rows, fp32 || top > 16) + (fp32 ? 2.7 : 0.0);
+}
 
 // Workspace of a product on this path: fp32 x's limbs, and the range sums of
 // the plan (past 16 rows two ranges wherever the blocks are few enough for any

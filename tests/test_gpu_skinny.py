@@ -135,6 +135,42 @@ def test_a_rows_bits_do_not_depend_on_the_batch(rows, cols, dtype, steps):
         assert torch.equal(y, ys[-1][:m]), m
 
 
+@pytest.mark.parametrize("rows,cols,m,dtype", [(50257, 768, 64, torch.float16), (32000, 256, 48, torch.float16),
+                                               (16384, 320, 33, torch.bfloat16), (50257, 832, 64, torch.float16)])
+def test_wide_layers_of_short_k_run_on_the_tiles(rows, cols, m, dtype):
+    """An output head at up to 64 rows over few columns is faster on the tiles:
+    it has the bits of the call with more rows than the skinny kernel takes."""
+
+    from qste_amd import kernels
+
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    tp = torch.randint(0, 256, (rows, cols // 8), generator=g, device=DEV, dtype=torch.uint8)
+    ts = torch.rand(rows, generator=g, device=DEV) * 0.02 + 0.01
+    tx = torch.randn(65, cols, generator=g, device=DEV).to(dtype)
+    y = kernels.packed_linear_affine(tx[:m].contiguous(), tp, ts, None, cols)
+    assert torch.equal(y, kernels.packed_linear_affine(tx, tp, ts, None, cols)[:m])
+
+
+@pytest.mark.parametrize("rows,cols,m,scalar", [(50257, 128, 21, True), (50257, 65, 2, True), (50257, 768, 21, False),
+                                                (2048, 256, 1, False)])
+def test_fp32_rows_of_short_k_stay_scalar(rows, cols, m, scalar):
+    """fp32 rows over few columns of a wide layer have the scalar kernel's bits
+    (those of the call without a workspace), longer K the skinny kernel's."""
+
+    from qste_amd import kernels
+
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    tp = torch.randint(0, 256, (rows, (cols + 7) // 8), generator=g, device=DEV, dtype=torch.uint8)
+    ts = torch.rand(rows, generator=g, device=DEV) * 0.02 + 0.01
+    tx = torch.randn(m, cols, generator=g, device=DEV)
+    y, plain = kernels.packed_linear_affine(tx, tp, ts, None, cols), torch.empty(m, rows, device=DEV)
+    assert kernels._lib.load().qste_packed_linear_affine(
+        tx.data_ptr(), 0, tp.data_ptr(), ts.data_ptr(), None, plain.data_ptr(), m, rows, cols,
+        torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(y, plain) == scalar
+    assert torch.allclose(y, plain, rtol=1e-4, atol=1e-5)
+
+
 @pytest.mark.parametrize("rows,cols,m", [(8192, 28672, 16), (1000, 8192, 64), (4096, 14336, 24)])
 def test_split_plans_are_deterministic(rows, cols, m):
     """Shapes whose plan splits K: two calls agree bit for bit, and with the
