@@ -98,18 +98,32 @@ inline size_t align_up(size_t v) { return (v + 255) & ~static_cast<size_t>(255);
 
 inline int64_t up64(int64_t v) { return (v + 63) / 64 * 64; }
 
-// A 16-bit layer whose rows or columns are no multiple of 64 runs its backward
+// A 16-bit layer whose rows or columns are no multiple of 64 can run its backward
 // on the matrix cores too, from zero-padded copies (of dy where rows are
-// ragged, of the weight signs where columns are), once the products are worth
-// the copies' launches.  Measured, scalar kernels / matrix cores, in us: 64
-// samples of 300 x 300 (2^22.5 multiply-adds) 78 / 74, 64 of 300 x 130
-// (2^21.3) 75 / about the same, 256 of 300 x 300 120 / 78, 512 of 1000 x 1000
-// 245 / 80, 2048 of 1000 x 3000 698 / 110.
+// ragged, of the weight signs where columns are).  The estimates, in us, are
+// fitted to 394 measured layers (1 to 8192 samples, 64 to 8192 rows, 64 to 4096
+// columns, with and without an input gradient) and choose within 14% of the
+// faster one: the scalar kernels take a serial chain (samples for the
+// evidence, rows for the input gradient) or their rate, the matrix cores the
+// copies' and the operands' launches.  Scalar / matrix cores: 64 samples of
+// 300 x 300 (the least work tried) 78 / 74, 512 of 1000 x 1000 245 / 80, 2048 of
+// 1000 x 3000 698 / 110; without an input gradient 16 of 156 x 3136 16 / 46, 100 of
+// 184 x 264 30 / 59, 408 of 384 x 450 66 / 49.
 constexpr int64_t kRaggedWork = int64_t{1} << 22;
-bool ragged_backward(int dtype, int64_t samples, int64_t rows, int64_t cols) {
-  return (dtype == QSTE_BF16 || dtype == QSTE_F16) && (rows % 64 != 0 || cols % 64 != 0) && samples > 0 && rows > 0 &&
-         cols > 0 && static_cast<double>(samples) * rows * cols >= static_cast<double>(kRaggedWork) &&
-         static_cast<double>(samples) * up64(rows) * 2 < 4294967296.0;
+bool ragged_backward(int dtype, int64_t samples, int64_t rows, int64_t cols, bool with_dx) {
+  if ((dtype != QSTE_BF16 && dtype != QSTE_F16) || (rows % 64 == 0 && cols % 64 == 0) || samples <= 0 || rows <= 0 ||
+      cols <= 0)
+    return false;
+  const double work = static_cast<double>(samples) * rows * cols, dy = static_cast<double>(samples) * rows * 4.0;
+  if (work < static_cast<double>(kRaggedWork) || static_cast<double>(samples) * up64(rows) * 2 >= 4294967296.0)
+    return false;
+  const double chain_e = 0.143 * samples, rate_e = 2.0 * work / 35e6, chain_d = 0.157 * rows, rate_d = 2.0 * work / 43e6;
+  const double scalar = 17.0 + (chain_e > rate_e ? chain_e : rate_e) +
+                        (with_dx ? 2.1 + (chain_d > rate_d ? chain_d : rate_d) : 0.0);
+  const double matrix = 36.0 + 0.0017 * samples + 2.0 * work / 385e6 + dy / 7.4e6 +
+                        static_cast<double>(rows) * cols * 4.0 / 17e6 + (rows % 64 ? 19.0 : 0.0) +
+                        (cols % 64 ? 5.4 : 0.0) + (with_dx ? 3.2 + 0.0036 * rows : 0.0);
+  return matrix < scalar;
 }
 
 struct BackwardLayout {
@@ -125,7 +139,10 @@ enum LayoutKind { LAYOUT_PLAIN, LAYOUT_LIMBS, LAYOUT_RAGGED };
 
 LayoutKind layout_kind(int dtype, int64_t samples, int64_t rows, int64_t cols) {
   if (dtype == QSTE_F32) return LAYOUT_LIMBS;
-  return ragged_backward(dtype, samples, rows, cols) ? LAYOUT_RAGGED : LAYOUT_PLAIN;
+  // (with or without an input gradient: the workspace is sized before that is known)
+  return ragged_backward(dtype, samples, rows, cols, true) || ragged_backward(dtype, samples, rows, cols, false)
+             ? LAYOUT_RAGGED
+             : LAYOUT_PLAIN;
 }
 
 BackwardLayout backward_layout(int64_t samples, int64_t rows, int64_t cols, LayoutKind kind = LAYOUT_PLAIN) {
@@ -483,6 +500,7 @@ int linear_backward_impl(const void* dy, int dtype, const uint8_t* packed_x, con
   // theirs through padded copies when the workspace has room for them
   // (qste_linear_backward_workspace_bytes_dtype), the SIMT kernels otherwise
   LayoutKind kind = layout_kind(dtype, samples, rows, cols);
+  if (kind == LAYOUT_RAGGED && !ragged_backward(dtype, samples, rows, cols, dx != nullptr)) kind = LAYOUT_PLAIN;
   BackwardLayout l = backward_layout(samples, rows, cols, kind);
   if (workspace_bytes < l.total) l = backward_layout(samples, rows, cols, kind = LAYOUT_PLAIN);
   if (!workspace || workspace_bytes < l.total) return QSTE_E_WORKSPACE;

@@ -110,6 +110,30 @@ def test_backward(rows, cols, m, dt, need_input, with_bias):
                                     dt)) <= 1e-3
 
 
+@pytest.mark.parametrize("rows,cols,m", [(1112, 3264, 128), (777, 768, 64), (1910, 320, 48)])
+def test_few_samples_without_an_input_gradient_stay_on_the_general_kernels(rows, cols, m):
+    """The evidence alone is a short chain there: it has the bits of the call
+    without room for the copies, which the call with an input gradient has not."""
+
+    from qste_amd import kernels
+
+    lib = kernels._lib.load()
+    packed, x, dy, scale, _ = problem(rows, cols, m, "bf16", rows + cols + m)
+    xbits, off, xs = oracle.pack_affine_rows(x)
+    tdy, txb, to, txs, tp, ts = t(dy, torch.bfloat16), t(xbits), t(off), t(xs), t(packed), t(scale)
+    alone, both = (kernels.linear_backward(tdy, txb, to, txs, tp, ts, cols, need_bias=False, need_input=n)[1]
+                   for n in (False, True))
+    copies = (m * (-(-rows // 64) * 64) * 2 if rows % 64 else 0) + (rows * (-(-cols // 128) * 16) if cols % 64 else 0)
+    small = lib.qste_linear_backward_workspace_bytes_dtype(m, rows, cols, 2) - copies // 2
+    work, general, gs = torch.empty(small, dtype=torch.uint8, device=DEV), torch.empty_like(alone), torch.empty_like(ts)
+    assert lib.qste_linear_backward(
+        tdy.data_ptr(), 2, txb.data_ptr(), to.data_ptr(), txs.data_ptr(), tp.data_ptr(), ts.data_ptr(), None,
+        general.data_ptr(), gs.data_ptr(), None, m, rows, cols, work.data_ptr(), small,
+        torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(alone, general)
+    assert not torch.equal(both, general)
+
+
 @pytest.mark.parametrize("rows,cols,m", [(300, 65, 5), (300, 100, 64), (1000, 777, 65), (129, 4161, 1), (65, 130, 300),
                                          (4097, 1000, 33), (256, 192, 16), (1000, 8001, 70), (50257, 767, 20)])
 @pytest.mark.parametrize("dt", ["bf16", "f16"])

@@ -126,6 +126,17 @@ def test_skinny_forward_asks_for_no_space_it_cannot_use():
     assert 0 < query(64, 8192, 4096, 2) <= 4 * 64 * 8192 * 4
 
 
+def test_small_ragged_backwards_ask_for_no_copies():
+    """A ragged 16-bit layer whose scalar chains are short (few samples and
+    rows) asks for what an fp32 one too small for limbs does: no padded copies."""
+
+    from qste_amd.kernels import _lib
+
+    query = _lib.load().qste_linear_backward_workspace_bytes_dtype
+    for samples, rows, cols in ((16, 156, 3136), (100, 184, 264), (16, 106, 2880)):
+        assert query(samples, rows, cols, 2) == query(samples, rows, cols, 1) == query(samples, rows, cols, 0)
+
+
 def test_fp32_limb_workspaces_are_capped_and_shared():
     """The fp32 products' bf16 limbs (6 bytes per dense value) are held to
     512 MiB: forward and input gradient in chunks of output rows, an
