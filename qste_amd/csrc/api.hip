@@ -227,6 +227,10 @@ double padding_us(int64_t rows, int64_t cols) {
 ForwardRoute forward_route(int64_t m, int64_t rows, int64_t cols, int dtype) {
   if (m <= 0 || rows <= 0 || cols <= 64) return {false, 0};
   const int64_t wide = padded_cols(cols);
+  // copies that the matrix kernels' 32-bit offsets cannot reach are not made
+  const bool reach = static_cast<double>(m) * wide * elem_bytes(dtype) < 4294967296.0 &&
+                     static_cast<double>(rows) * wide / 8 < 4294967296.0;
+  if (cols % 128 != 0 && !reach) return {false, 0};
   const double skinny = gemv_forward_us(m, rows, wide, dtype);
   const int64_t copies = cols % 128 != 0 ? wide : 0;
   const double ragged = copies ? padding_us(rows, cols) : 0.0;

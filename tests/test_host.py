@@ -126,6 +126,19 @@ def test_skinny_forward_asks_for_no_space_it_cannot_use():
     assert 0 < query(64, 8192, 4096, 2) <= 4 * 64 * 8192 * 4
 
 
+def test_no_padded_copies_past_the_matrix_kernels_reach():
+    """A ragged forward whose padded copy of x (or of the signs) would pass 4 GiB
+    runs on the general kernel from x itself, as it would from the copy: no
+    workspace."""
+
+    from qste_amd.kernels import _lib
+
+    query = _lib.load().qste_packed_linear_affine_workspace_bytes
+    assert query(1 << 20, 256, 1000, 2) >= (1 << 20) * 1024 * 2
+    for m, rows, cols in ((1 << 21, 256, 1000), (1 << 24, 8, 777), (100, 1 << 20, 40001), (40, 1 << 20, 40001)):
+        assert query(m, rows, cols, 2) == 0, (m, rows, cols)
+
+
 def test_small_ragged_backwards_ask_for_no_copies():
     """A ragged 16-bit layer whose scalar chains are short (few samples and
     rows) asks for what an fp32 one too small for limbs does: no padded copies."""
