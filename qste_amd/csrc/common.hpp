@@ -210,6 +210,13 @@ __device__ __forceinline__ float div_by(float x, float d, float r) {
   return e == e ? fmaf(e, r, q0) : q0;
 }
 
+// The bf16 limbs of fp32 operands (gemm_mfma.hip) hold them times
+// 2^limb_shift(top), `top` being the largest exponent of a row of outputs, or
+// kLimbNone when it has no finite nonzero operand; a product's accumulators
+// stay below 2^kLimbTop times the number of its terms.
+constexpr int kLimbTop = 96, kLimbNone = -(1 << 20);
+__host__ __device__ constexpr int limb_shift(int top) { return top == kLimbNone ? 0 : kLimbTop - top; }
+
 inline int ceil_div(int64_t a, int64_t b) { return static_cast<int>((a + b - 1) / b); }
 
 // Wave priority `x mod 4` (s_setprio takes an immediate).  The hardware

@@ -44,8 +44,9 @@ enum { B_BITS_ALONG_K = 0, B_BITS_ALONG_N = 1, B_BITS_ALONG_K_SCALED = 2 };
 // EPI_PARTIAL: the bare fp32 accumulators of one K range of a split-K
 // evidence, finished by evidence_combine_kernel.  EPI_FORWARD_F32: the
 // forward's scale and bias, stored as fp32 (the fp32 products, whose dense
-// operand arrives as three bf16 limbs along K).
-enum { EPI_FORWARD = 0, EPI_PLAIN = 1, EPI_EVIDENCE = 2, EPI_PARTIAL = 3, EPI_FORWARD_F32 = 4 };
+// operand arrives as three bf16 limbs along K).  EPI_EVIDENCE_F32: the
+// evidence of such an operand.  Both undo the limbs' power of two per row.
+enum { EPI_FORWARD = 0, EPI_PLAIN = 1, EPI_EVIDENCE = 2, EPI_PARTIAL = 3, EPI_FORWARD_F32 = 4, EPI_EVIDENCE_F32 = 5 };
 
 struct Params {
   const uint16_t* a;     // bf16 dense operand (x or dy)
@@ -66,6 +67,7 @@ struct Params {
   const uint8_t* w_bits; // evidence: sign_w for the scale gradient
   int64_t w_pb;          // evidence: bytes per row of w_bits
   float* gs_partial;     // evidence: [WAVES_N * tiles_n][M]
+  const int* m_top;      // limbs: the largest exponent of row m's operands (limb_shift)
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, int64_t bytes) {
@@ -584,38 +586,51 @@ __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0,
 
   if (EPI == EPI_FORWARD_F32) {
     // y = acc * scale[n] + bias[n] in fp32, stored as computed (32 lanes x 4
-    // bytes per row per store)
+    // bytes per row per store); the rows' powers of two go to LDS first (read
+    // between the stores they would wait for each)
     float* y = static_cast<float*>(p.out);
+    int* xst = reinterpret_cast<int*>(A0);  // [TM]
+    if (tid < TM) xst[tid] = m0 + tid < p.M ? -limb_shift(p.m_top[m0 + tid]) : 0;
+    stage_barrier<0>();
     float sc[NBN], bi[NBN];
 #pragma unroll
     for (int nb = 0; nb < NBN; ++nb) {
       const int64_t col = n0 + WNC * wn + 32 * nb + l32;
       sc[nb] = (col < p.N && p.n_scale) ? p.n_scale[col] : 1.0f;
       bi[nb] = (col < p.N && p.n_bias) ? p.n_bias[col] : 0.0f;
+      // waited for here: at their uses between the stores the waits would be
+      // for those as well (7304 x 4032 over 1280: 230 -> 186 us)
+      asm volatile("" : "+v"(sc[nb]), "+v"(bi[nb]));
     }
 #pragma unroll
-    for (int mb = 0; mb < MBN; ++mb)
+    for (int mb = 0; mb < MBN; ++mb) {
+      int back[16];  // of the lane's rows of the block, four at a time
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<int4*>(back + 4 * i) = *reinterpret_cast<const int4*>(xst + 32 * mb + 8 * i + 4 * kg);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int64_t row = m0 + WMR * wm + 32 * mb + 8 * (r >> 2) + 4 * kg + (r & 3);
 #pragma unroll
         for (int nb = 0; nb < NBN; ++nb) {
           const int64_t col = n0 + WNC * wn + 32 * nb + l32;
-          float v = acc[mb][nb][r] * sc[nb];
+          float v = ldexpf(acc[mb][nb][r], back[r]) * sc[nb];
           v = v + bi[nb];
           if (row < p.M && col < p.N) y[row * p.N + col] = v;
         }
       }
+    }
     return;
   }
 
-  if (EPI == EPI_EVIDENCE) {
+  if (EPI == EPI_EVIDENCE || EPI == EPI_EVIDENCE_F32) {
     // E0 = acc + v[m]; E = E0 * s[m] (fp32, 32 lanes x 4 bytes per row per
     // store); row partials of E0 * sign_w over this wave's columns.
     // The tile's sign_w bits (256 rows x 32 bytes), v and s go to LDS first.
     uint8_t* wst = A0;                                  // [256][32] bytes
     float* vst = reinterpret_cast<float*>(A0 + 8192);   // [256]
     float* sst = vst + BM;                              // [256]
+    int* xst = reinterpret_cast<int*>(sst + BM);        // [256]
     {
       const int64_t row = m0 + tid;
       const __amdgpu_buffer_rsrc_t rw = rsrc(p.w_bits, p.w_bits ? p.M * p.w_pb : 0);
@@ -627,6 +642,7 @@ __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0,
       }
       vst[tid] = (p.m_add && row < p.M) ? p.m_add[row] : 0.0f;
       sst[tid] = (p.m_scale && row < p.M) ? p.m_scale[row] : 1.0f;
+      if (EPI == EPI_EVIDENCE_F32) xst[tid] = row < p.M ? -limb_shift(p.m_top[row]) : 0;
     }
     stage_barrier<0>();
     float* ev = static_cast<float*>(p.out);
@@ -645,7 +661,7 @@ __device__ __forceinline__ void wide_tile(const Params& p, int pid, uint8_t* A0,
 #pragma unroll
         for (int nb = 0; nb < NBN; ++nb) {
           const int64_t col = n0 + WNC * wn + 32 * nb + l32;
-          const float e0 = acc[mb][nb][r] + add;
+          const float e0 = (EPI == EPI_EVIDENCE_F32 ? ldexpf(acc[mb][nb][r], xst[lrow]) : acc[mb][nb][r]) + add;
           // columns past N hold zero bits and contribute -e0: skip them
           if (col < p.N) acc_part += ((wd[nb] >> l32) & 1u) ? e0 : -e0;
           if (row < p.M && col < p.N) ev[row * p.N + col] = e0 * mul;
@@ -965,6 +981,7 @@ template <int OUT>
 __global__ __launch_bounds__(THREADS) void forward_combine_kernel(const float* __restrict__ partial, int tiles,
                                                                   int splits, const float* __restrict__ n_scale,
                                                                   const float* __restrict__ n_bias,
+                                                                  const int* __restrict__ m_top,
                                                                   void* __restrict__ out, int64_t M, int64_t N) {
   const int tiles_m = static_cast<int>((M + BM - 1) / BM), tiles_n = static_cast<int>((N + BN - 1) / BN);
   const int i = static_cast<int>(blockIdx.y);
@@ -982,6 +999,11 @@ __global__ __launch_bounds__(THREADS) void forward_combine_kernel(const float* _
   }
   const int64_t col0 = static_cast<int64_t>(tn) * BN + lcol;
   float v[4] = {acc.x, acc.y, acc.z, acc.w};
+  if constexpr (OUT == QSTE_F32) {
+    const int back = -limb_shift(m_top[row]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = ldexpf(v[q], back);
+  }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int64_t col = col0 + q;
@@ -1194,7 +1216,7 @@ static int launch_split(const mfma::Params& p, const SplitK& sp, float* partial,
   if (rc) return rc;
   const dim3 grid(mfma::wide::BM / (mfma::wide::THREADS / kWave), static_cast<unsigned>(tiles));
   mfma::wide::forward_combine_kernel<OUT><<<grid, mfma::wide::THREADS, 0, stream>>>(
-      partial, tiles, sp.splits, p.n_scale, p.n_bias, p.out, p.M, p.N);
+      partial, tiles, sp.splits, p.n_scale, p.n_bias, p.m_top, p.out, p.M, p.N);
   return static_cast<int>(hipGetLastError());
 }
 
@@ -1556,73 +1578,203 @@ int mfma_backward_pair(const void* dy, int64_t ldy, int dtype, const uint8_t* x_
 // fp32 products on the bf16 MFMA path.  An fp32 value v splits exactly into
 // three bf16 limbs: hi = bf16(v), mid = bf16(v - hi), lo = bf16(v - hi - mid)
 // (each difference is exact in fp32; v - hi has at most 16 significant
-// bits and v - hi - mid at most 8, so lo holds it exactly; only values whose
-// last limb falls below bf16's subnormals lose it).  A limb times +-1 is
+// bits and v - hi - mid at most 8, so lo holds it exactly).  A limb times +-1 is
 // exact, so a product over K becomes the same bf16 MFMA product over 3K --
 // the dense operand's three limbs along K against the signs repeated three
 // times -- with every product exact and the sums in the MFMA's fp32
-// accumulators.  Per-k scales (the row scale of dX, the sample scale of
-// the evidence) are multiplied into the fp32 operand first, one fp32
-// rounding each, where the reference's fp32 GEMM rounds the product inside
-// its fused multiply-add.
+// accumulators.
+//
+// Per-k scales (the row scale of dX, the sample scale of the evidence) are
+// multiplied into the operand first.  The scalar kernels do not round that
+// product (it is part of a fused multiply-add); here lo takes what rounding it
+// to fp32 leaves over: the limbs hold the product to 2^-26 of it and better.
+//
+// bf16's range ends where fp32's does, so lo would lose bits of values below
+// 2^-110 and hold none of those below 2^-126.  The limbs of a row of outputs
+// are therefore those of the operands times a power of two that brings the
+// row's largest to 2^kLimbTop (limb_shift), undone in the epilogue: exact in
+// both places, and all 24 bits are kept down to 2^-206 of the largest.  The
+// largest exponent of a row is found in the pass that writes its limbs (rows
+// contiguous: a second read, from the cache), or in a pass before it (evidence,
+// rows of outputs being columns of dy).
 // ---------------------------------------------------------------------------
 
 namespace limbs {
 
+// Exponent of v (times m), as frexp counts; kLimbNone for zero, infinities, NaN.
+__device__ __forceinline__ int exponent_of(float v, float m) {
+  const bool counts = __builtin_isfinite(v) && v != 0.0f && __builtin_isfinite(m) && m != 0.0f;
+  return counts ? __builtin_amdgcn_frexp_expf(v) + __builtin_amdgcn_frexp_expf(m) : kLimbNone;
+}
+
+// The limbs of v * 2^shift, or with MUL of v * m * 2^shift.  An infinity or NaN
+// is carried by hi alone, so the products see what fp32's do.
+template <bool MUL>
+__device__ __forceinline__ void limbs_of(float v, float m, int shift, uint16_t h[3]) {
+  float f, rest = 0.0f;
+  if constexpr (MUL) {
+    const float a = __builtin_amdgcn_frexp_mantf(v), b = __builtin_amdgcn_frexp_mantf(m);
+    const int e = __builtin_amdgcn_frexp_expf(v) + __builtin_amdgcn_frexp_expf(m) + shift;
+    const float p = a * b;
+    f = ldexpf(p, e);
+    rest = ldexpf(fmaf(a, b, -p), e);
+  } else {
+    f = ldexpf(v, shift);
+  }
+  h[0] = f32_to_bf16(f);
+  float r1 = f - bf16_to_f32(h[0]);
+  const bool finite = __builtin_isfinite(f);  // shifted operands do not overflow
+  r1 = finite ? r1 : 0.0f;
+  rest = finite ? rest : 0.0f;
+  h[1] = f32_to_bf16(r1);
+  h[2] = f32_to_bf16((r1 - bf16_to_f32(h[1])) + rest);
+}
+
+struct Quad {
+  float v[4];
+};
+
+// x[c .. c + 3] of a row, zeros from `cols` on
+__device__ __forceinline__ Quad load_quad(const float* row, int64_t c, int64_t cols, bool vec) {
+  Quad q{{0.0f, 0.0f, 0.0f, 0.0f}};
+  if (vec && c < cols) {
+    const float4 f = *reinterpret_cast<const float4*>(row + c);
+    q.v[0] = f.x, q.v[1] = f.y, q.v[2] = f.z, q.v[3] = f.w;
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (c + k < cols) q.v[k] = row[c + k];
+  }
+  return q;
+}
+
+__device__ __forceinline__ void store_limbs(uint16_t* o, int64_t plane, const uint16_t h[4][3]) {
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+    *reinterpret_cast<uint2*>(o + p * plane) = make_uint2(h[0][p] | (static_cast<uint32_t>(h[1][p]) << 16),
+                                                          h[2][p] | (static_cast<uint32_t>(h[3][p]) << 16));
+}
+
 // out[plane * p + r * ld + c] for the three limbs p of x[r, c] (times
-// row_mul[r] or col_mul[c] when given), c < `padded` (a multiple of 4, as ld
-// and plane are), zero from `cols` on; four columns a thread.
-__global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ x, int64_t rows, int64_t cols,
-                                                    const float* __restrict__ row_mul,
-                                                    const float* __restrict__ col_mul, uint16_t* __restrict__ out,
-                                                    int64_t ld, int64_t plane, int64_t padded) {
+// col_mul[c] when given), c < `padded` (a multiple of 4, as ld and plane are),
+// zero from `cols` on; top[r] = the largest exponent of the row.  G threads a
+// row, which hold up to 16 G columns of it in registers between the two passes
+// (read again past that).
+constexpr int kHeld = 4;  // quads a thread holds
+template <int G, bool MUL>
+__global__ __launch_bounds__(G < 256 ? 256 : G) void split_rows_kernel(const float* __restrict__ x, int64_t rows,
+                                                                       int64_t cols, const float* __restrict__ col_mul,
+                                                                       uint16_t* __restrict__ out, int64_t ld,
+                                                                       int64_t plane, int64_t padded,
+                                                                       int* __restrict__ top) {
+  constexpr int kThreads = G < 256 ? 256 : G;
+  __shared__ int wave_top[kThreads / kWave];
+  const int64_t r = blockIdx.x * static_cast<int64_t>(kThreads / G) + threadIdx.x / G;
+  const int t = threadIdx.x % G;
+  const bool live = r < rows;  // the same in all of a row's threads
+  const bool vec = (cols & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  const float* row = x + (live ? r : 0) * cols;
+  auto mul = [&](int64_t c) { return MUL && c < cols ? col_mul[c] : 1.0f; };
+  // the largest exponent, or without MUL the bits of the largest finite |x|
+  auto largest = [&](const Quad& q, int64_t c) {
+    int e = MUL ? kLimbNone : 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if constexpr (MUL) {
+        e = max(e, exponent_of(q.v[k], mul(c + k)));
+      } else {
+        const int bits = static_cast<int>(__float_as_uint(q.v[k]) & 0x7FFFFFFFu);
+        e = max(e, bits < 0x7F800000 ? bits : 0);
+      }
+    }
+    return e;
+  };
+  Quad held[kHeld];
+#pragma unroll
+  for (int u = 0; u < kHeld; ++u) held[u] = load_quad(row, 4 * (t + u * G), cols, vec);
+  int e = MUL ? kLimbNone : 0;
+#pragma unroll
+  for (int u = 0; u < kHeld; ++u) e = max(e, largest(held[u], 4 * (t + u * G)));
+  for (int64_t c = 4 * (t + kHeld * G); c < cols; c += 4 * G) e = max(e, largest(load_quad(row, c, cols, vec), c));
+#pragma unroll
+  for (int o = kWave / 2; o >= 1; o >>= 1) e = max(e, __shfl_xor(e, o, kWave));
+  if constexpr (G > kWave) {
+    if (threadIdx.x % kWave == 0) wave_top[threadIdx.x / kWave] = e;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kThreads / kWave; ++w) e = max(e, wave_top[w]);
+  }
+  if (!live) return;
+  if constexpr (!MUL) e = e == 0 ? kLimbNone : __builtin_amdgcn_frexp_expf(__uint_as_float(static_cast<uint32_t>(e)));
+  if (t == 0) top[r] = e;
+  const int shift = limb_shift(e);
+  auto put = [&](const Quad& q, int64_t c) {
+    uint16_t h[4][3];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) limbs_of<MUL>(q.v[k], mul(c + k), shift, h[k]);
+    store_limbs(out + r * ld + c, plane, h);
+  };
+#pragma unroll
+  for (int u = 0; u < kHeld; ++u)
+    if (4 * (t + u * G) < padded) put(held[u], 4 * (t + u * G));
+  for (int64_t c = 4 * (t + kHeld * G); c < padded; c += 4 * G) put(load_quad(row, c, cols, vec), c);
+}
+
+// The same with rows of outputs along the columns of x [rows, cols]: row_mul[r]
+// is multiplied in, top[c] (set to kLimbNone before) takes column c's largest
+// exponent.  A workgroup takes 64 columns of kTopRows rows, a wave a row.
+constexpr int kTopRows = 64;
+__global__ __launch_bounds__(256) void column_top_kernel(const float* __restrict__ x, int64_t rows, int64_t cols,
+                                                         const float* __restrict__ row_mul, int* __restrict__ top) {
+  const int64_t c = blockIdx.x * static_cast<int64_t>(kWave) + threadIdx.x % kWave;
+  if (c >= cols) return;
+  const int64_t r0 = blockIdx.y * static_cast<int64_t>(kTopRows);
+  const int64_t r1 = r0 + kTopRows < rows ? r0 + kTopRows : rows;
+  // all of a lane's rows in flight; past the end the last row again
+  constexpr int kPer = kTopRows / (256 / kWave);
+  float v[kPer], m[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int64_t r = min(r0 + threadIdx.x / kWave + u * (256 / kWave), r1 - 1);
+    v[u] = x[r * cols + c];
+    m[u] = row_mul ? row_mul[r] : 1.0f;
+  }
+  int e = kLimbNone;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) e = max(e, exponent_of(v[u], m[u]));
+  if (e != kLimbNone) atomicMax(top + c, e);  // whole numbers: the order does not show
+}
+
+__global__ __launch_bounds__(256) void split_columns_kernel(const float* __restrict__ x, int64_t rows, int64_t cols,
+                                                            const float* __restrict__ row_mul,
+                                                            const int* __restrict__ top, uint16_t* __restrict__ out,
+                                                            int64_t ld, int64_t plane, int64_t padded) {
   const int64_t per = padded / 4, n = rows * per;
   const bool vec = (cols & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int64_t r = i / per, c = 4 * (i - r * per);
-    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (vec && c < cols) {
-      const float4 q = *reinterpret_cast<const float4*>(x + r * cols + c);
-      v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
-    } else {
+    const Quad q = load_quad(x + r * cols, c, cols, vec);
+    const float mul = row_mul ? row_mul[r] : 1.0f;
+    int e[4];  // (`top` has `padded` entries: the columns past the data are zero)
+    *reinterpret_cast<int4*>(e) = *reinterpret_cast<const int4*>(top + c);
+    uint16_t h[4][3];
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (c + k < cols) v[k] = x[r * cols + c + k];
-    }
-    uint16_t h[3][4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      float f = v[k];
-      if (row_mul) f = f * row_mul[r];
-      if (col_mul && c + k < cols) f = f * col_mul[c + k];
-      uint16_t hi = f32_to_bf16(f);
-      const bool finite = __builtin_isfinite(f);
-      // a finite value that rounds past bf16's largest finite one keeps its
-      // top 16 bits instead (truncation: the residual is exact as well); an
-      // infinite or NaN value is carried by hi alone, its other limbs zero,
-      // so the products see the same inf or NaN the fp32 operand holds
-      if (finite && (hi & 0x7F80u) == 0x7F80u) hi = static_cast<uint16_t>(__float_as_uint(f) >> 16);
-      const float r1 = finite ? f - bf16_to_f32(hi) : 0.0f;
-      const uint16_t mid = f32_to_bf16(r1);
-      h[0][k] = hi;
-      h[1][k] = mid;
-      h[2][k] = f32_to_bf16(r1 - bf16_to_f32(mid));
-    }
-    uint16_t* o = out + r * ld + c;
-#pragma unroll
-    for (int p = 0; p < 3; ++p)
-      *reinterpret_cast<uint2*>(o + p * plane) = make_uint2(h[p][0] | (static_cast<uint32_t>(h[p][1]) << 16),
-                                                            h[p][2] | (static_cast<uint32_t>(h[p][3]) << 16));
+    for (int k = 0; k < 4; ++k) limbs_of<true>(q.v[k], mul, limb_shift(e[k]), h[k]);
+    store_limbs(out + r * ld + c, plane, h);
   }
 }
 
 // out[plane * p + r * out_ld + j] = in[r * in_ld + j] for p = 0, 1, 2 and
 // j < bytes, zero for j < `padded` (a multiple of 8, as out_ld and plane are):
 // the packed signs repeated for each limb; in may be plane 0 of out itself
-// (bytes == padded then), which is left as it is
+// (bytes == padded then), which is left as it is.  top[0 .. tops) = kLimbNone.
 __global__ __launch_bounds__(256) void repeat_kernel(const uint8_t* in, int64_t rows, int64_t bytes, int64_t in_ld,
-                                                     uint8_t* out, int64_t out_ld, int64_t plane, int64_t padded) {
+                                                     uint8_t* out, int64_t out_ld, int64_t plane, int64_t padded,
+                                                     int* top = nullptr, int64_t tops = 0) {
+  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < tops;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    top[i] = kLimbNone;
   struct __attribute__((packed)) Unaligned8 {
     uint64_t w;
   };
@@ -1655,12 +1807,26 @@ inline size_t up256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 }  // namespace limbs
 
-// The limbs of x [rows, cols] as rows of their own: out [3 rows, cols], row
-// 3r + i limb i (hi, mid, lo) of row r.
-int launch_limbs(const float* x, int64_t rows, int64_t cols, uint16_t* out, hipStream_t stream) {
-  limbs::split_kernel<<<limbs::grid_for(rows * cols / 4), 256, 0, stream>>>(x, rows, cols, nullptr, nullptr, out,
-                                                                            3 * cols, cols, cols);
+// Threads a row: enough to hold it, more where the rows are too few for the chip
+// (a thread's elements are a serial chain: one row of 768 on one wave 4.4 us, on
+// four 2.9).
+static int launch_split_rows(const float* x, int64_t rows, int64_t cols, const float* col_mul, uint16_t* out,
+                             int64_t ld, int64_t plane, int64_t padded, int* top, hipStream_t stream) {
+#define QSTE_SPLIT_ROWS(G)                                                                             \
+  (col_mul ? limbs::split_rows_kernel<G, true> : limbs::split_rows_kernel<G, false>)                   \
+      <<<static_cast<unsigned>(G < 256 ? (rows + 3) / 4 : rows), G < 256 ? 256 : G, 0, stream>>>(       \
+          x, rows, cols, col_mul, out, ld, plane, padded, top)
+  if (cols <= 256 || (cols <= 16 * 64 && rows >= 1024)) QSTE_SPLIT_ROWS(64);
+  else if (cols <= 16 * 256 || rows >= 1024) QSTE_SPLIT_ROWS(256);
+  else QSTE_SPLIT_ROWS(1024);
+#undef QSTE_SPLIT_ROWS
   return static_cast<int>(hipGetLastError());
+}
+
+// The limbs of x [rows, cols] as rows of their own: out [3 rows, cols], row
+// 3r + i limb i (hi, mid, lo) of row r, times 2^limb_shift(top[r]).
+int launch_limbs(const float* x, int64_t rows, int64_t cols, uint16_t* out, int* top, hipStream_t stream) {
+  return launch_split_rows(x, rows, cols, nullptr, out, 3 * cols, cols, cols, top, stream);
 }
 
 int launch_transpose_bits(const uint8_t*, uint8_t*, int64_t, int64_t, int64_t, int64_t, hipStream_t);
@@ -1704,8 +1870,8 @@ static size_t f32_partial(int64_t m, int64_t n, int64_t k) {
 }
 
 // Workspace of an [m, n] product over k through the limbs (0: not for it):
-// the dense limbs of a chunk, the signs three times, and the split-K partials
-// of a full chunk or of the last, shorter one.
+// the dense limbs of a chunk and its rows' exponents, the signs three times, and
+// the split-K partials of a full chunk or of the last, shorter one.
 static size_t f32_product_workspace(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || !f32_limbs_worth(m, n, k)) return 0;
   const int64_t mc = f32_chunk_rows(m, k);
@@ -1715,7 +1881,7 @@ static size_t f32_product_workspace(int64_t m, int64_t n, int64_t k) {
     const size_t tail = f32_partial(m % mc, n, k);
     if (tail > partial) partial = tail;
   }
-  return limbs::up256(static_cast<size_t>(mc) * 3 * up64(k) * 2) +
+  return limbs::up256(static_cast<size_t>(mc) * 3 * up64(k) * 2) + limbs::up256(static_cast<size_t>(mc) * sizeof(int)) +
          limbs::up256(static_cast<size_t>(n) * 3 * up64(k) / 8) + partial;
 }
 
@@ -1723,13 +1889,13 @@ static size_t f32_product_workspace(int64_t m, int64_t n, int64_t k) {
 // of rows of the dense operand; the signs (bits along k, [n][3 up64(k) / 8],
 // planes of up64(k) / 8) are at `b` already.
 static int f32_product(const float* dense, const float* col_mul, const uint8_t* b, const float* scale,
-                       const float* bias, float* out, int64_t m, int64_t n, int64_t k, uint16_t* a, float* partial,
-                       hipStream_t stream) {
+                       const float* bias, float* out, int64_t m, int64_t n, int64_t k, uint16_t* a, int* top,
+                       float* partial, hipStream_t stream) {
   const int64_t kp = up64(k), mc = f32_chunk_rows(m, k);
   for (int64_t i0 = 0; i0 < m; i0 += mc) {
     const int64_t mi = m - i0 < mc ? m - i0 : mc;
-    limbs::split_kernel<<<limbs::grid_for(mi * kp / 4), 256, 0, stream>>>(dense + i0 * k, mi, k, nullptr, col_mul, a,
-                                                                          3 * kp, kp, kp);
+    int rc = launch_split_rows(dense + i0 * k, mi, k, col_mul, a, 3 * kp, kp, kp, top, stream);
+    if (rc) return rc;
     mfma::Params p{};
     p.a = a;
     p.bits = b;
@@ -1738,8 +1904,8 @@ static int f32_product(const float* dense, const float* col_mul, const uint8_t* 
     p.lda = 3 * kp; p.pb = 3 * kp / 8;
     p.a_rows = mi; p.bit_rows = n;
     p.n_scale = scale; p.n_bias = bias;
+    p.m_top = top;
     const ProductPlan plan = f32_plan(mi, n, k);
-    int rc;
     if (plan.split.splits > 1) {
       rc = launch_split<mfma::B_BITS_ALONG_K, QSTE_BF16, QSTE_F32>(p, plan.split, partial, stream);
     } else if (plan.half) {
@@ -1766,10 +1932,11 @@ int mfma_f32_forward(const float* x, const uint8_t* packed, const float* scale, 
   const int64_t kp = up64(cols), kb = kp / 8, mc = f32_chunk_rows(m, cols), pb = (cols + 7) / 8;
   if (!fits32(mc * 3 * kp * 2) || !fits32(rows * 3 * kb)) return 1;
   uint16_t* a = static_cast<uint16_t*>(workspace);
-  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(mc) * 3 * kp * 2);
+  int* top = reinterpret_cast<int*>(static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(mc) * 3 * kp * 2));
+  uint8_t* b = reinterpret_cast<uint8_t*>(top) + limbs::up256(static_cast<size_t>(mc) * sizeof(int));
   float* partial = reinterpret_cast<float*>(b + limbs::up256(static_cast<size_t>(rows) * 3 * kb));
   limbs::repeat_kernel<<<limbs::grid_for(rows * kb / 8), 256, 0, stream>>>(packed, rows, pb, pb, b, 3 * kb, kb, kb);
-  return f32_product(x, nullptr, b, scale, bias, y, m, rows, cols, a, partial, stream);
+  return f32_product(x, nullptr, b, scale, bias, y, m, rows, cols, a, top, partial, stream);
 }
 
 size_t f32_dgrad_workspace(int64_t m, int64_t rows, int64_t cols) { return f32_product_workspace(m, cols, rows); }
@@ -1783,14 +1950,15 @@ int mfma_f32_dgrad(const float* dy, const uint8_t* packed, const float* row_scal
   const int64_t kp = up64(rows), kb = kp / 8, mc = f32_chunk_rows(m, rows);
   if (!fits32(mc * 3 * kp * 2) || !fits32(cols * 3 * kb)) return 1;
   uint16_t* a = static_cast<uint16_t*>(workspace);
-  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(mc) * 3 * kp * 2);
+  int* top = reinterpret_cast<int*>(static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(mc) * 3 * kp * 2));
+  uint8_t* b = reinterpret_cast<uint8_t*>(top) + limbs::up256(static_cast<size_t>(mc) * sizeof(int));
   float* partial = reinterpret_cast<float*>(b + limbs::up256(static_cast<size_t>(cols) * 3 * kb));
   // the transposed signs into plane 0 of each row of b (zero past `rows`),
   // then repeated into planes 1 and 2
   const int rc = launch_transpose_bits(packed, b, rows, cols, (cols + 7) / 8, 3 * kb, stream);
   if (rc) return rc;
   limbs::repeat_kernel<<<limbs::grid_for(cols * kb / 8), 256, 0, stream>>>(b, cols, kb, 3 * kb, b, 3 * kb, kb, kb);
-  return f32_product(dy, row_scale, b, nullptr, nullptr, dx, m, cols, rows, a, partial, stream);
+  return f32_product(dy, row_scale, b, nullptr, nullptr, dx, m, cols, rows, a, top, partial, stream);
 }
 
 // Whether the evidence takes the limbs; its K is the samples.  From 128 rows
@@ -1811,7 +1979,8 @@ size_t f32_evidence_workspace(int64_t samples, int64_t rows, int64_t cols) {
   // pass, so a product whose limbs exceed the budget is not split up
   const size_t a = static_cast<size_t>(3 * samples) * up64(rows) * 2;
   if (a > kLimbBudget) return 0;
-  return limbs::up256(a) + limbs::up256(static_cast<size_t>(3 * samples) * (up64(cols) / 8)) +
+  return limbs::up256(a) + limbs::up256(static_cast<size_t>(up64(rows)) * sizeof(int)) +
+         limbs::up256(static_cast<size_t>(3 * samples) * (up64(cols) / 8)) +
          (cols % 64 ? limbs::up256(static_cast<size_t>(rows) * ((cols + 127) / 128 * 16)) : 0);
 }
 
@@ -1829,14 +1998,19 @@ int mfma_f32_evidence(const float* dy, const uint8_t* packed_x, const float* x_s
   const int64_t k3 = 3 * samples, rp = up64(rows), cb = up64(cols) / 8, pb = (cols + 7) / 8;
   if (!fits32(k3 * rp * 2) || !fits32(k3 * cb)) return 1;
   uint16_t* a = static_cast<uint16_t*>(workspace);
-  uint8_t* b = static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(k3) * rp * 2);
-  limbs::split_kernel<<<limbs::grid_for(samples * rp / 4), 256, 0, stream>>>(dy, samples, rows, x_scale, nullptr, a,
-                                                                             rp, samples * rp, rp);
+  int* top = reinterpret_cast<int*>(static_cast<uint8_t*>(workspace) + limbs::up256(static_cast<size_t>(k3) * rp * 2));
+  uint8_t* b = reinterpret_cast<uint8_t*>(top) + limbs::up256(static_cast<size_t>(rp) * sizeof(int));
   limbs::repeat_kernel<<<limbs::grid_for(samples * cb / 8), 256, 0, stream>>>(packed_x, samples, pb, pb, b, cb,
-                                                                             samples * cb, cb);
+                                                                             samples * cb, cb, top, rp);
+  limbs::column_top_kernel<<<dim3(static_cast<unsigned>((rows + kWave - 1) / kWave),
+                                  static_cast<unsigned>((samples + limbs::kTopRows - 1) / limbs::kTopRows)),
+                             256, 0, stream>>>(dy, samples, rows, x_scale, top);
+  limbs::split_columns_kernel<<<limbs::grid_for(samples * rp / 4), 256, 0, stream>>>(dy, samples, rows, x_scale, top, a,
+                                                                                     rp, samples * rp, rp);
   mfma::Params p = evidence_params(a, b, nullptr, ev, k3, rows, cols, m_add, m_scale, w_bits, gs_partial);
   p.lda = rp;
   p.pb = cb;
+  p.m_top = top;
   if (cols % 64 != 0 && w_bits) {  // the epilogue reads the signs of W in whole dwords
     uint8_t* wp = b + limbs::up256(static_cast<size_t>(k3) * cb);
     p.w_pb = (cols + 127) / 128 * 16;
@@ -1844,7 +2018,7 @@ int mfma_f32_evidence(const float* dy, const uint8_t* packed_x, const float* x_s
     if (rc) return rc;
     p.w_bits = wp;
   }
-  mfma::wide::wide_kernel<mfma::A_ROWS_K, mfma::B_BITS_ALONG_N, mfma::EPI_EVIDENCE, QSTE_BF16>
+  mfma::wide::wide_kernel<mfma::A_ROWS_K, mfma::B_BITS_ALONG_N, mfma::EPI_EVIDENCE_F32, QSTE_BF16>
       <<<wide_grid(rows, cols), mfma::wide::THREADS, 0, stream>>>(p);
   return static_cast<int>(hipGetLastError());
 }

@@ -120,6 +120,7 @@ struct Args {
   const float* bias;    // may be null
   void* y;              // [xr / limbs, N] (16-bit, or fp32 with limbs)
   float* partial;       // splits > 1: [splits][xr][N]
+  const int* top;       // fp32: the largest exponent of each row of x (its limbs carry a power of two)
   int xr;               // rows of x
   int limbs;            // 1, or 3 (y in fp32, row m = rows 3m .. 3m + 2 of x)
   int splits;
@@ -200,6 +201,8 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
   constexpr int MT = C::MT, JS = C::JS, D = C::D;
   __shared__ __attribute__((aligned(16))) uint8_t smem[C::bytes];
   __shared__ float epi[2][16 * NBW];
+  constexpr bool kLimbs = DT == QSTE_BF16 && STAGED;  // what fp32 rows run on
+  __shared__ int back[kLimbs ? XR / 3 : 1];           // fp32: the power of two to undo, per row of y
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, q = lane >> 4;
@@ -297,12 +300,14 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
     if constexpr (C::XBUF > 1) issue_x(c + WAVES, 0, 1);
     __builtin_amdgcn_sched_barrier(0);
   }
-  // the epilogue's row scale and bias, fetched while the first loads fly
+  // the epilogue's row scale, bias and powers of two, fetched while the first loads fly
   float out_scale = 0.0f, out_bias = 0.0f;
   if (tid < 16 * NBW && n0 + tid < p.N) {
     out_scale = p.scale[n0 + tid];
     out_bias = p.bias ? p.bias[n0 + tid] : 0.0f;
   }
+  int out_top = 0;
+  if (kLimbs && p.limbs == 3 && tid < p.xr / 3) out_top = p.top[tid];
   if constexpr (C::RESIDENT) {
     for (; c < c_last; c += WAVES) {
       wait_vm<D>();  // all but the newest loads, the weights in flight: x is in LDS
@@ -432,6 +437,7 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
     epi[0][tid] = out_scale;
     epi[1][tid] = out_bias;
   }
+  if (kLimbs && p.limbs == 3 && tid < p.xr / 3) back[tid] = -limb_shift(out_top);
   __syncthreads();
   f32x4* red = reinterpret_cast<f32x4*>(smem);  // [WAVES][NBW * MT][64]
 #pragma unroll
@@ -474,12 +480,16 @@ __global__ __launch_bounds__(THREADS, 1) void skinny_kernel(Args p) {
     if (n >= p.N) continue;
     const float* sc = &epi[0][16 * b + 4 * g];
     const float* bi = &epi[1][16 * b + 4 * g];
-    if (p.limbs == 3) {
-      const f32x4 v = (total(b, 3 * m + 2, g) + total(b, 3 * m + 1, g)) + total(b, 3 * m, g);
-      finish4<QSTE_F32>(p, m, n, v, sc, bi, vec);
-    } else {
-      finish4<DT>(p, m, n, total(b, m, g), sc, bi, vec);
+    if constexpr (kLimbs) {
+      if (p.limbs == 3) {
+        f32x4 v = (total(b, 3 * m + 2, g) + total(b, 3 * m + 1, g)) + total(b, 3 * m, g);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = ldexpf(v[j], back[m]);
+        finish4<QSTE_F32>(p, m, n, v, sc, bi, vec);
+        continue;
+      }
     }
+    finish4<DT>(p, m, n, total(b, m, g), sc, bi, vec);
   }
 }
 
@@ -631,7 +641,7 @@ size_t up256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 }  // namespace gemv
 
-int launch_limbs(const float*, int64_t, int64_t, uint16_t*, hipStream_t);
+int launch_limbs(const float*, int64_t, int64_t, uint16_t*, int*, hipStream_t);
 
 // Time of a product on this path in us, negative when its sizes are not for it.
 // It is the time of the instance's last row (16, 32, 48 or 64; 21 in fp32): a
@@ -645,7 +655,7 @@ double gemv_forward_us(int64_t m, int64_t rows, int64_t cols, int dtype) {
   return gemv::estimate(top, gemv::plan_of(top, rows, cols, !fp32), rows, fp32 || top > 16) + (fp32 ? 2.7 : 0.0);
 }
 
-// Workspace of a product on this path: fp32 x's limbs, and the range sums of
+// Workspace of a product on this path: fp32 x's limbs and their exponents, or the range sums of
 // the plan (past 16 rows two ranges wherever the blocks are few enough for any
 // plan to split, so that the size does not depend on where the plan's line
 // lies); 0 where none is needed or the product is not for this path.
@@ -656,7 +666,7 @@ size_t gemv_forward_workspace(int64_t m, int64_t rows, int64_t cols, int dtype) 
   const gemv::Plan plan = gemv::plan_of(xr, rows, cols, !fp32);
   int64_t ranges = plan.splits > 1 ? plan.splits : 0;
   if (!fp32 && m > 16 && ranges < 2 && (rows + 15) / 16 <= gemv::kSplitBlocks) ranges = 2;
-  return (fp32 ? gemv::up256(static_cast<size_t>(xr * cols) * 2) : 0) +
+  return (fp32 ? gemv::up256(static_cast<size_t>(xr * cols) * 2) + gemv::up256(static_cast<size_t>(m) * sizeof(int)) : 0) +
          static_cast<size_t>(ranges * xr * rows) * sizeof(float);
 }
 
@@ -689,10 +699,11 @@ int gemv_linear_forward(const void* x, int dtype, const uint8_t* packed, const f
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   if (fp32) {
     uint16_t* xl = reinterpret_cast<uint16_t*>(ws);
-    const int rc = launch_limbs(static_cast<const float*>(x), m, cols, xl, stream);
+    int* top = reinterpret_cast<int*>(ws + gemv::up256(static_cast<size_t>(p.xr * cols) * 2));
+    const int rc = launch_limbs(static_cast<const float*>(x), m, cols, xl, top, stream);
     if (rc) return rc;
     p.x = xl;
-    ws += gemv::up256(static_cast<size_t>(p.xr * cols) * 2);
+    p.top = top;
   }
   p.partial = reinterpret_cast<float*>(ws);
   return dtype == QSTE_F16 ? gemv::run<QSTE_F16>(p, plan, stream) : gemv::run<QSTE_BF16>(p, plan, stream);

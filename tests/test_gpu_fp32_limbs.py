@@ -259,3 +259,87 @@ def test_products_over_row_chunks():
     torch.cuda.synchronize()
     want = oracle.linear_dgrad_f64(xs, packed_t.cpu().numpy(), n, row_scale.cpu().numpy())
     assert _rel(dx[torch.from_numpy(sel).to(DEV)].cpu().numpy(), want) <= 2e-6
+
+
+def _spread(n, seed):
+    """Powers of two from fp32's smallest normal to 2^80, one per output row."""
+
+    return np.ldexp(np.float32(1.0), np.random.default_rng(seed).permutation(np.linspace(-126, 80, n).astype(int)))
+
+
+def _within(got, want, mag, scale_rounding=2.0 ** -149):
+    """The bar of ``_bounded`` row by row (fp32's grid ends at 2^-149)."""
+
+    got, want = np.asarray(got, np.float64), np.asarray(want, np.float64)
+    err = np.abs(got - want)
+    assert np.all(err <= 2.0 ** -20 * mag + 4 * scale_rounding), np.max(err / (mag + scale_rounding))
+
+
+@pytest.mark.parametrize("m,rows,cols", [(1, 300, 1024), (5, 640, 2048), (21, 333, 640), (24, 300, 2048),
+                                         (300, 257, 1000), (256, 512, 2048)])
+def test_forward_keeps_24_bits_at_any_magnitude(m, rows, cols):
+    """Each row of x at a power of two of its own: its outputs are as exact,
+    against its own terms, as a row's near one (bf16's third limb alone would
+    leave 2^-8 of a row at 2^-126).  The output row scale is 2^40, so that
+    outputs stay inside fp32's range."""
+
+    from qste_amd import kernels
+
+    x, packed, _, _ = _problem(m, rows, cols, m + cols)
+    big = _spread(m, m) if m > 1 else np.array([2.0 ** -125], np.float32)
+    xs = (x.cpu().numpy().clip(-4, 4) * big[:, None]).astype(np.float32)
+    scale = torch.full((rows,), 2.0 ** 20, device=DEV)
+    y = kernels.packed_linear_affine(torch.from_numpy(xs).to(DEV), packed, scale, None, cols)
+    want = oracle.linear_fwd_f64(xs, packed.cpu().numpy(), scale.cpu().numpy(), None, cols)
+    _within(y.cpu().numpy(), want, np.abs(xs.astype(np.float64)).sum(1)[:, None] * 2.0 ** 20)
+
+
+@pytest.mark.parametrize("m,rows,cols", [(256, 1024, 512), (64, 1000, 333), (300, 2048, 257)])
+def test_backward_keeps_24_bits_at_any_magnitude(m, rows, cols):
+    """dX with a power of two per row of dy, the evidence with one per column."""
+
+    from qste_amd import kernels
+
+    g = torch.Generator(device=DEV).manual_seed(m + rows)
+    dy = torch.randn(m, rows, generator=g, device=DEV).clamp_(-4, 4).cpu().numpy()
+    coord = torch.randint(-127, 128, (rows, cols), generator=g, device=DEV, dtype=torch.int32).to(torch.int8)
+    packed = kernels.pack_coordinate(coord)
+    scale = torch.rand(rows, generator=g, device=DEV) * 0.5 + 0.5
+    d = (dy * _spread(m, 3)[:, None]).astype(np.float32)
+    dx = kernels.packed_transpose(torch.from_numpy(d).to(DEV), packed, cols, row_scale=scale)
+    sc = scale.cpu().numpy()
+    want = oracle.linear_dgrad_f64(d, packed.cpu().numpy(), cols, sc)
+    _within(dx.cpu().numpy(), want, (np.abs(d.astype(np.float64)) @ sc.astype(np.float64))[:, None])
+
+    d = (dy * _spread(rows, 4)[None, :]).astype(np.float32)
+    px = kernels.pack_coordinate(torch.randint(-127, 128, (m, cols), generator=g, device=DEV,
+                                               dtype=torch.int32).to(torch.int8))
+    xs = torch.rand(m, generator=g, device=DEV) + 0.5
+    ev = kernels.evidence_from_packed(torch.from_numpy(d).to(DEV), px, cols, row_scale=xs)
+    want = oracle.evidence_f64(d, px.cpu().numpy(), cols, xs.cpu().numpy())
+    mag = (np.abs(d.astype(np.float64)) * xs.cpu().numpy()[:, None].astype(np.float64)).sum(0)[:, None]
+    _within(ev.cpu().numpy(), want, mag)
+
+
+def test_scaled_operands_are_not_rounded_to_24_bits():
+    """dX where two scaled terms nearly cancel: what is left is as exact as a
+    fused multiply-add leaves it.  The three limbs of a product hold it to half
+    of the third one's last place: 8 bits each below the product's leading
+    power of two make that 2^-26 of the product, for two terms 2^-25 (dy * scale
+    rounded to fp32 first leaves up to 2^-24 of each)."""
+
+    from qste_amd import kernels
+
+    m, rows, cols = 256, 512, 384
+    rng = np.random.default_rng(5)
+    scale = (rng.random(rows) * 0.5 + 0.5).astype(np.float32)
+    dy = np.zeros((m, rows), np.float32)
+    i, j = rng.integers(0, 256, m), rng.integers(256, 512, m)
+    dy[np.arange(m), i] = (rng.random(m) + 1.0).astype(np.float32)
+    dy[np.arange(m), j] = -(dy[np.arange(m), i].astype(np.float64) * scale[i] / scale[j]).astype(np.float32)
+    packed = np.full((rows, cols // 8), 0xFF, np.uint8)
+    dx = kernels.packed_transpose(torch.from_numpy(dy).to(DEV), torch.from_numpy(packed).to(DEV), cols,
+                                  row_scale=torch.from_numpy(scale).to(DEV)).cpu().numpy()
+    want = (dy.astype(np.float64) * scale.astype(np.float64)).sum(1)
+    term = np.abs(dy[np.arange(m), i] * scale[i])
+    assert np.max(np.abs(dx - want[:, None]) / term[:, None]) <= 2.0 ** -25

@@ -122,7 +122,7 @@ def test_skinny_forward_asks_for_no_space_it_cannot_use():
     for rows in (8208, 14336, 28672, 50257):
         for m in (1, 16, 17, 40, 64):
             assert query(m, rows, 4096, 2) == 0, (rows, m)
-        assert query(21, rows, 4096, 0) == 63 * 4096 * 2  # the limbs of x alone
+        assert query(21, rows, 4096, 0) <= 63 * 4096 * 2 + 256  # the limbs of x alone, and what they are scaled by
     assert 0 < query(64, 8192, 4096, 2) <= 4 * 64 * 8192 * 4
 
 
