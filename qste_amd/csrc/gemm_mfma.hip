@@ -1861,24 +1861,34 @@ static int64_t f32_chunk_rows(int64_t m, int64_t k) {
   return fit >= m ? m : fit / mfma::wide::BM * mfma::wide::BM;
 }
 
-static ProductPlan f32_plan(int64_t m, int64_t n, int64_t k) {
-  return product_plan(m, n, static_cast<int>(3 * up64(k) / mfma::wide::BK), true);
+// The plan of an [m, n] product over k.  The error of a sum grows with the
+// accumulations of its chain, so a forward whose tiles are few enough for K
+// ranges takes them even where one chain on 128-row tiles would be faster:
+// 2048 x 2048 over 640, against 64 bits, 3.2e-7 in one chain, 1.0e-7 in four
+// ranges.  (`ranges`: a forward.  dX has its ranges where they are faster.)
+static ProductPlan f32_plan(int64_t m, int64_t n, int64_t k, bool ranges) {
+  const int nk = static_cast<int>(3 * up64(k) / mfma::wide::BK);
+  if (ranges) {
+    const SplitK sp = forward_split_plan(wide_grid(m, n), nk);
+    if (sp.splits > 1) return ProductPlan{false, sp, 0.0};
+  }
+  return product_plan(m, n, nk, true);
 }
 
-static size_t f32_partial(int64_t m, int64_t n, int64_t k) {
-  return split_bytes(f32_plan(m, n, k).split, wide_grid(m, n));
+static size_t f32_partial(int64_t m, int64_t n, int64_t k, bool ranges) {
+  return split_bytes(f32_plan(m, n, k, ranges).split, wide_grid(m, n));
 }
 
 // Workspace of an [m, n] product over k through the limbs (0: not for it):
 // the dense limbs of a chunk and its rows' exponents, the signs three times, and
 // the split-K partials of a full chunk or of the last, shorter one.
-static size_t f32_product_workspace(int64_t m, int64_t n, int64_t k) {
+static size_t f32_product_workspace(int64_t m, int64_t n, int64_t k, bool ranges) {
   if (m <= 0 || n <= 0 || k <= 0 || !f32_limbs_worth(m, n, k)) return 0;
   const int64_t mc = f32_chunk_rows(m, k);
   if (mc == 0) return 0;
-  size_t partial = f32_partial(mc, n, k);
+  size_t partial = f32_partial(mc, n, k, ranges);
   if (m % mc) {
-    const size_t tail = f32_partial(m % mc, n, k);
+    const size_t tail = f32_partial(m % mc, n, k, ranges);
     if (tail > partial) partial = tail;
   }
   return limbs::up256(static_cast<size_t>(mc) * 3 * up64(k) * 2) + limbs::up256(static_cast<size_t>(mc) * sizeof(int)) +
@@ -1890,7 +1900,7 @@ static size_t f32_product_workspace(int64_t m, int64_t n, int64_t k) {
 // planes of up64(k) / 8) are at `b` already.
 static int f32_product(const float* dense, const float* col_mul, const uint8_t* b, const float* scale,
                        const float* bias, float* out, int64_t m, int64_t n, int64_t k, uint16_t* a, int* top,
-                       float* partial, hipStream_t stream) {
+                       float* partial, bool ranges, hipStream_t stream) {
   const int64_t kp = up64(k), mc = f32_chunk_rows(m, k);
   for (int64_t i0 = 0; i0 < m; i0 += mc) {
     const int64_t mi = m - i0 < mc ? m - i0 : mc;
@@ -1905,7 +1915,7 @@ static int f32_product(const float* dense, const float* col_mul, const uint8_t* 
     p.a_rows = mi; p.bit_rows = n;
     p.n_scale = scale; p.n_bias = bias;
     p.m_top = top;
-    const ProductPlan plan = f32_plan(mi, n, k);
+    const ProductPlan plan = f32_plan(mi, n, k, ranges);
     if (plan.split.splits > 1) {
       rc = launch_split<mfma::B_BITS_ALONG_K, QSTE_BF16, QSTE_F32>(p, plan.split, partial, stream);
     } else if (plan.half) {
@@ -1920,7 +1930,7 @@ static int f32_product(const float* dense, const float* col_mul, const uint8_t* 
   return 0;
 }
 
-size_t f32_forward_workspace(int64_t m, int64_t rows, int64_t cols) { return f32_product_workspace(m, rows, cols); }
+size_t f32_forward_workspace(int64_t m, int64_t rows, int64_t cols) { return f32_product_workspace(m, rows, cols, true); }
 
 // y [m, rows] fp32 = (x @ sign^T) * scale + bias through the limbs.  Returns 1
 // when the call is not for this path (shape, or too little workspace).
@@ -1936,10 +1946,10 @@ int mfma_f32_forward(const float* x, const uint8_t* packed, const float* scale, 
   uint8_t* b = reinterpret_cast<uint8_t*>(top) + limbs::up256(static_cast<size_t>(mc) * sizeof(int));
   float* partial = reinterpret_cast<float*>(b + limbs::up256(static_cast<size_t>(rows) * 3 * kb));
   limbs::repeat_kernel<<<limbs::grid_for(rows * kb / 8), 256, 0, stream>>>(packed, rows, pb, pb, b, 3 * kb, kb, kb);
-  return f32_product(x, nullptr, b, scale, bias, y, m, rows, cols, a, top, partial, stream);
+  return f32_product(x, nullptr, b, scale, bias, y, m, rows, cols, a, top, partial, true, stream);
 }
 
-size_t f32_dgrad_workspace(int64_t m, int64_t rows, int64_t cols) { return f32_product_workspace(m, cols, rows); }
+size_t f32_dgrad_workspace(int64_t m, int64_t rows, int64_t cols) { return f32_product_workspace(m, cols, rows, false); }
 
 // dx [m, cols] fp32 = dy @ (row_scale * sign) through the limbs: dy scaled
 // by the row scale along K, the signs transposed (bits along K).
@@ -1958,7 +1968,7 @@ int mfma_f32_dgrad(const float* dy, const uint8_t* packed, const float* row_scal
   const int rc = launch_transpose_bits(packed, b, rows, cols, (cols + 7) / 8, 3 * kb, stream);
   if (rc) return rc;
   limbs::repeat_kernel<<<limbs::grid_for(cols * kb / 8), 256, 0, stream>>>(b, cols, kb, 3 * kb, b, 3 * kb, kb, kb);
-  return f32_product(dy, row_scale, b, nullptr, nullptr, dx, m, cols, rows, a, top, partial, stream);
+  return f32_product(dy, row_scale, b, nullptr, nullptr, dx, m, cols, rows, a, top, partial, false, stream);
 }
 
 // Whether the evidence takes the limbs; its K is the samples.  From 128 rows

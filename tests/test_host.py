@@ -126,6 +126,18 @@ def test_skinny_forward_asks_for_no_space_it_cannot_use():
     assert 0 < query(64, 8192, 4096, 2) <= 4 * 64 * 8192 * 4
 
 
+def test_fp32_forwards_of_few_tiles_keep_their_k_ranges():
+    """An fp32 forward of at most 128 tiles over 12 K steps or more sums its K in
+    ranges (a shorter chain is the more exact one): room for their partial sums."""
+
+    from qste_amd.kernels import _lib
+
+    query, tile = _lib.load().qste_packed_linear_affine_workspace_bytes, 256 * 256 * 4
+    for m, rows, cols, tiles, ranges in ((2048, 2048, 640, 64, 4), (1476, 4792, 5120, 114, 2), (394, 5248, 448, 42, 5),
+                                         (1546, 1664, 384, 49, 4)):
+        assert query(m, rows, cols, 0) >= tiles * ranges * tile, (m, rows, cols)
+
+
 def test_no_padded_copies_past_the_matrix_kernels_reach():
     """A ragged forward whose padded copy of x (or of the signs) would pass 4 GiB
     runs on the general kernel from x itself, as it would from the copy: no
