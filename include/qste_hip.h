@@ -170,6 +170,18 @@ size_t qste_linear_backward_workspace_bytes(int64_t samples, int64_t rows, int64
  * qste_linear_backward runs both products on the MFMA path; given only
  * qste_linear_backward_workspace_bytes() it runs them in fp32 SIMT code. */
 size_t qste_linear_backward_workspace_bytes_dtype(int64_t samples, int64_t rows, int64_t cols, int dtype);
+/* How qste_linear_backward runs a layer whose operands are aligned and whose
+ * workspace has the size of the query for its dtype (no GPU needed): the
+ * general kernels, fp32 limbs, evidence and dx in one launch, or evidence on
+ * 256-row tiles and dx (if wanted) on 256-row tiles, on 128-row tiles or over
+ * ranges of K.  No counterpart in the reference. */
+#define QSTE_ROUTE_GENERAL 0
+#define QSTE_ROUTE_LIMBS 1
+#define QSTE_ROUTE_PAIR 2
+#define QSTE_ROUTE_TILES 3
+#define QSTE_ROUTE_HALF_TILES 4
+#define QSTE_ROUTE_RANGES 5
+int qste_linear_backward_route(int64_t samples, int64_t rows, int64_t cols, int dtype, int with_dx);
 int qste_linear_backward(const void* dy, int dtype, const uint8_t* packed_x,
                          const float* x_offset, const float* x_scale,
                          const uint8_t* packed_w, const float* scale, void* dx,

@@ -41,6 +41,7 @@ int mfma_linear_dgrad(const void*, int, const uint8_t*, const float*, void*, int
 int mfma_linear_dgrad_t(const void*, int64_t, int, const uint8_t*, int64_t, const uint16_t*, void*, int64_t, int64_t,
                         int64_t, float*, hipStream_t);
 int64_t mfma_dgrad_split_bytes(int64_t, int64_t, int64_t);
+bool mfma_dgrad_half(int64_t, int64_t, int64_t);
 int mfma_evidence(const void*, int, const uint8_t*, const float*, float*, int64_t, int64_t, int64_t,
                   const float*, const float*, const uint8_t*, float*, const EvidencePlan*, float*, hipStream_t);
 int mfma_evidence_t(const void*, int64_t, int, const uint8_t*, int64_t, const uint16_t*, float*, int64_t, int64_t,
@@ -485,6 +486,23 @@ size_t qste_linear_backward_workspace_bytes(int64_t samples, int64_t rows, int64
 size_t qste_linear_backward_workspace_bytes_dtype(int64_t samples, int64_t rows, int64_t cols, int dtype) {
   if (samples < 0 || rows < 0 || cols < 0) return 0;
   return backward_layout(samples, rows, cols, layout_kind(dtype, samples, rows, cols)).total;
+}
+
+int qste_linear_backward_route(int64_t samples, int64_t rows, int64_t cols, int dtype, int with_dx) {
+  if (!dtype_ok(dtype)) return QSTE_E_DTYPE;
+  if (samples < 0 || rows <= 0 || cols <= 0) return QSTE_E_SHAPE;
+  const bool dx = with_dx != 0;
+  if (dtype == QSTE_F32)
+    return backward_layout(samples, rows, cols, LAYOUT_LIMBS).limb_bytes > 0 ? QSTE_ROUTE_LIMBS : QSTE_ROUTE_GENERAL;
+  const bool ragged = ragged_backward(dtype, samples, rows, cols, dx);
+  if (samples == 0 || !(ragged || (rows % 64 == 0 && cols % 64 == 0)) ||
+      !mfma_backward_ok(nullptr, ragged ? up64(rows) : rows, dtype, samples, rows, cols))
+    return QSTE_ROUTE_GENERAL;
+  if (mfma_evidence_plan(samples, rows, cols, dx).pair) return QSTE_ROUTE_PAIR;
+  if (!dx) return QSTE_ROUTE_TILES;
+  return mfma_dgrad_split_bytes(samples, rows, cols) > 0 ? QSTE_ROUTE_RANGES
+         : mfma_dgrad_half(samples, rows, cols)          ? QSTE_ROUTE_HALF_TILES
+                                                         : QSTE_ROUTE_TILES;
 }
 
 namespace {

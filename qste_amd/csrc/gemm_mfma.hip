@@ -1270,6 +1270,11 @@ int64_t mfma_dgrad_split_bytes(int64_t m, int64_t rows, int64_t cols) {
   return static_cast<int64_t>(split_bytes(dgrad_split(m, rows, cols), wide_grid(m, cols)));
 }
 
+// Whether dX as a launch of its own runs on 128-row tiles (from transposed signs).
+bool mfma_dgrad_half(int64_t m, int64_t rows, int64_t cols) {
+  return dgrad_split(m, rows, cols).splits == 1 && dgrad_cut(m, rows, cols).half;
+}
+
 // `partial`: mfma_dgrad_split_bytes of space, or null (unsplit)
 int mfma_linear_dgrad(const void* dy, int dtype, const uint8_t* packed, const float* row_scale, void* dx,
                       int64_t m, int64_t rows, int64_t cols, float* partial, hipStream_t stream) {

@@ -41,6 +41,7 @@ SIGNATURES = {
     "qste_packed_row_inner": (_int, [_vp, _vp, _vp, _i64, _i64, _vp]),
     "qste_linear_backward_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "qste_linear_backward_workspace_bytes_dtype": (_sz, [_i64, _i64, _i64, _int]),
+    "qste_linear_backward_route": (_int, [_i64, _i64, _i64, _int, _int]),
     "qste_evidence_from_packed_workspace_bytes_dtype": (_sz, [_i64, _i64, _i64, _int]),
     "qste_packed_linear_affine_workspace_bytes": (_sz, [_i64, _i64, _i64, _int]),
     "qste_packed_linear_affine_ws": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp]),

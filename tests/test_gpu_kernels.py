@@ -524,8 +524,8 @@ def test_mfma_products_ragged(rows, cols, m, dt):
 # one launch or alone); (4160, 4096, 2048): 272 tiles, ragged M, the first
 # 256 whole and the last 16 split in two.
 # (3072, 768, 8184) and (768, 3072, 8184): config 3's MLP layers (GPT-2 small,
-# 8 x 1023 tokens), whose backward runs the pair kernel with every evidence
-# tile split over a ragged K.
+# 8 x 1023 tokens), every evidence tile split over a ragged K; the first one's
+# backward runs the pair kernel, the second's dX is a launch of 128-row tiles.
 SPLIT_SHAPES = [(256, 256, 16384), (512, 320, 3000), (1024, 4096, 8192), (4096, 1024, 8192),
                 (4160, 4096, 2048), (3072, 768, 8184), (768, 3072, 8184)]
 

@@ -11,8 +11,11 @@ outputs one rounding to the dtype.
 Sizes sit where the kernel's layout can go wrong: row counts at the edges of
 its 4-, 16-, 32-, 48- and 64-row instances, K inside a 512-column chunk and
 over several chunks of a wave, N inside a block of 16 and of a workgroup,
-output rows whose start is not 16-byte aligned, one to eight blocks, and plans
-that split K (the C entry without a workspace runs the same call unsplit)."""
+output rows whose start is not 16-byte aligned, every number of blocks that an
+instance has (one to eight up to 32 rows, to six up to 48, to four up to 64: the
+largest images of the sums in LDS; K is long enough there that the call stays
+off the tiles), and plans that split K (the C entry without a workspace runs the
+same call unsplit)."""
 
 from __future__ import annotations
 
@@ -56,6 +59,35 @@ def _check(got, x, packed, scale, bias, cols):
 
 SHAPES = [(300, 1024, 17), (4097, 896, 33), (129, 4224, 48), (1000, 8192, 49), (16, 128, 64), (9001, 640, 32),
           (4096, 14336, 24), (1026, 5120, 40), (8200, 1152, 64)]
+
+
+# (blocks, rows of x): ceil(rows / 4096) blocks of 16 weight rows a workgroup
+BLOCKS = [(rows, cols, m) for cols, m, most in ((2048, 1, 8), (2176, 16, 8), (4096, 32, 8), (6144, 40, 6), (8192, 64, 4))
+          for rows in (4096 * n - 77 for n in range(1, most + 1))]
+
+
+@pytest.mark.parametrize("rows,cols,m", BLOCKS)
+def test_every_number_of_blocks(rows, cols, m):
+    """bf16 and, where three limbs a row make that instance, fp32: outputs of
+    weight rows at the edges of blocks and workgroups, all rows of x."""
+
+    from qste_amd import kernels
+
+    rng = np.random.default_rng(rows + m)
+    packed = rng.integers(0, 256, size=(rows, cols // 8), dtype=np.uint8)
+    scale = (rng.random(rows) * 0.02 + 0.01).astype(np.float32)
+    bias = (rng.standard_normal(rows) * 0.1).astype(np.float32)
+    pick = np.unique(np.concatenate([np.arange(0, rows, 997), np.arange(15, rows, 1009), np.arange(max(0, rows - 140), rows)]))
+    for dtype, n in ((torch.bfloat16, m), (torch.float32, m // 3)):
+        if n == 0:
+            continue
+        print(f"skinny {rows}x{cols} m={n} {dtype}", flush=True)
+        x = torch.from_numpy(rng.standard_normal((n, cols), dtype=np.float32)).to(dtype)
+        y = kernels.packed_linear_affine(x.to(DEV), torch.from_numpy(packed).to(DEV), torch.from_numpy(scale).to(DEV),
+                                         torch.from_numpy(bias).to(DEV), cols)
+        assert torch.isfinite(y).all()
+        _check(y[:, torch.from_numpy(pick).to(DEV)], x.float().numpy(), np.ascontiguousarray(packed[pick]), scale[pick],
+               bias[pick], cols)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

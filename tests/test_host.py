@@ -126,6 +126,22 @@ def test_skinny_forward_asks_for_no_space_it_cannot_use():
     assert 0 < query(64, 8192, 4096, 2) <= 4 * 64 * 8192 * 4
 
 
+def test_backward_routes():
+    """What the route query says for layers of known kinds."""
+
+    from qste_amd.kernels import _lib
+
+    route = _lib.load().qste_linear_backward_route
+    general, limbs, pair, tiles, half, ranges = range(6)
+    assert route(8184, 3072, 768, 2, 1) == pair and route(300, 65, 1000, 2, 1) == pair
+    assert route(8184, 768, 3072, 2, 1) == half and route(8184, 768, 3072, 2, 0) == tiles
+    assert route(4384, 1372, 2155, 1, 1) == half
+    assert route(2046, 50257, 768, 2, 1) == ranges
+    assert route(256, 2048, 2048, 0, 1) == limbs
+    assert route(4, 100, 100, 2, 1) == general == route(4, 64, 96, 0, 1)
+    assert route(4, 100, 100, 7, 1) < 0 and route(-1, 100, 100, 2, 1) < 0 and route(4, 0, 100, 2, 1) < 0
+
+
 def test_fp32_forwards_of_few_tiles_keep_their_k_ranges():
     """An fp32 forward of at most 128 tiles over 12 K steps or more sums its K in
     ranges (a shorter chain is the more exact one): room for their partial sums."""
