@@ -84,15 +84,19 @@ int qste_packed_linear_affine(const void* x, int dtype, const uint8_t* packed,
 
 /* qste_packed_linear_affine with a workspace of
  * qste_packed_linear_affine_workspace_bytes(m, rows, cols, dtype) bytes
- * (0: none is used).  fp32 x then runs on the bf16 MFMA path: x splits
- * exactly into three bf16 limbs (hi + mid + lo) along K, the signs repeat
- * for each, every product is exact and the sums are the MFMA's fp32
- * accumulators -- an fp32 product, where the plain entry runs fp32 SIMT
- * code.  Where a product has few output tiles against its K (fp32 at small
- * m; bf16 / fp16 with 16 < m and at most a round of 256-row tiles), K is
+ * (0: none is used).  fp32 x then runs on the bf16 MFMA path, where its sizes
+ * make that faster: x splits exactly into three bf16 limbs (hi + mid + lo),
+ * times a power of two per row that keeps the last one in bf16's range,
+ * every product is exact and the sums are the MFMA's fp32 accumulators -- an
+ * fp32 product, where the plain entry runs fp32 SIMT code.  Where a product
+ * has few output tiles against its K (fp32; bf16 / fp16 with 16 < m), K is
  * cut into ranges whose fp32 accumulators the workspace holds, summed in
- * range order before the scale, bias and one rounding.  Other dtypes and
- * shapes behave as the plain entry.  Replaces
+ * range order before the scale, bias and one rounding.  bf16 / fp16 x whose
+ * cols no matrix path takes (a multiple of 64; of 128 on the kernel for up to
+ * 64 rows, 21 of fp32) runs on copies of x and the signs padded with zeros,
+ * where those are faster and below 4 GiB.  Both change the order of the fp32
+ * sums, so an output may differ from the plain entry's by its last place.
+ * Other shapes behave as the plain entry.  Replaces
  * qste.kernels.packed_linear_affine (loader.py:292-297); the reference's
  * route for fp32 inputs is torch's fp32 mm on expanded signs
  * (cuda.py:1531-1597). */
@@ -112,10 +116,12 @@ int qste_packed_transpose(const void* dy, int dtype, const uint8_t* packed,
                           int64_t cols, void* stream);
 
 /* qste_packed_transpose with a workspace of
- * qste_packed_transpose_workspace_bytes(m, rows, cols, dtype) bytes: fp32 dy
- * times the row scale (one fp32 rounding) runs through bf16 limbs on the
- * MFMA path as above.  Replaces qste.kernels.packed_transpose
- * (loader.py:299-304) for fp32 inputs. */
+ * qste_packed_transpose_workspace_bytes(m, rows, cols, dtype) bytes (0: none
+ * is used): fp32 dy times the row scale runs through bf16 limbs on the MFMA
+ * path as above (the limbs hold the product to 2^-26 of it and better), and
+ * bf16 / fp16 products of few output tiles (rows and cols multiples of 64) cut
+ * K into ranges summed in range order, as the layer's backward does.  Replaces
+ * qste.kernels.packed_transpose (loader.py:299-304). */
 size_t qste_packed_transpose_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int dtype);
 int qste_packed_transpose_ws(const void* dy, int dtype, const uint8_t* packed, const float* row_scale, void* dx,
                              int64_t m, int64_t rows, int64_t cols, void* workspace, size_t workspace_bytes,
@@ -132,7 +138,7 @@ int qste_packed_transpose_ws(const void* dy, int dtype, const uint8_t* packed, c
  * fallback.py:126-138). */
 size_t qste_evidence_from_packed_workspace_bytes(int64_t samples, int64_t rows, int64_t cols);
 /* The workspace for a given dtype: for fp32 dy, room for its bf16 limbs
- * (dy times the sample scale, one fp32 rounding, then split as above),
+ * (of dy times the sample scale, as above; a power of two per column of dy),
  * which qste_evidence_from_packed then uses for the MFMA path. */
 size_t qste_evidence_from_packed_workspace_bytes_dtype(int64_t samples, int64_t rows, int64_t cols, int dtype);
 int qste_evidence_from_packed(const void* dy, int dtype, const uint8_t* packed_x,
@@ -160,15 +166,19 @@ int qste_packed_row_inner(const float* matrix, const uint8_t* packed, float* out
  * Per shape, evidence and dx run in one launch or as two, and evidence
  * tiles whose K (= samples) chain is long against the launch are split over
  * K and summed in a fixed order in the workspace, so results do not depend
- * on scheduling.
+ * on scheduling; so is a dx of few output tiles that has a launch of its own.
+ * bf16 / fp16 layers whose rows or cols are no multiple of 64 run on the
+ * matrix cores from zero-padded copies (of dy and of W's signs) where that is
+ * faster, with room for them in the workspace.
  * Needs qste_linear_backward_workspace_bytes() bytes of workspace.
  * No counterpart as a single call in the reference: it fuses five of its
  * calls (cuda.py:1568-1688, functional.py:143, 193). */
 size_t qste_linear_backward_workspace_bytes(int64_t samples, int64_t rows, int64_t cols);
-/* The workspace for a given dtype: for fp32 dy it includes room for the
- * bf16 limbs of dX's and the evidence's dense operands, with which
- * qste_linear_backward runs both products on the MFMA path; given only
- * qste_linear_backward_workspace_bytes() it runs them in fp32 SIMT code. */
+/* The workspace for a given dtype (the query above: for bf16 / fp16): for fp32
+ * dy it includes room for the bf16 limbs of dX's and the evidence's dense
+ * operands, with which qste_linear_backward runs both products on the MFMA
+ * path; given less it runs them in fp32 SIMT code.  A ragged bf16 / fp16 layer
+ * given less than its padded copies take runs on the general kernels. */
 size_t qste_linear_backward_workspace_bytes_dtype(int64_t samples, int64_t rows, int64_t cols, int dtype);
 /* How qste_linear_backward runs a layer whose operands are aligned and whose
  * workspace has the size of the query for its dtype (no GPU needed): the

@@ -1043,7 +1043,7 @@ __global__ __launch_bounds__(THREADS) void forward_combine_kernel(const float* _
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// bf16 and fp16 take the MFMA path (fp32 stays on the fp32 SIMT kernel)
+// bf16 and fp16 take the MFMA path as they are (fp32 as bf16 limbs, below)
 static bool mfma_dtype(int dtype) { return dtype == QSTE_BF16 || dtype == QSTE_F16; }
 
 EvidencePlan mfma_evidence_plan(int64_t samples, int64_t rows, int64_t cols, bool with_dgrad);
@@ -1220,7 +1220,7 @@ static int launch_split(const mfma::Params& p, const SplitK& sp, float* partial,
   return static_cast<int>(hipGetLastError());
 }
 
-// The 16-bit forward with few output tiles (M past the decode GEMV's 16, a
+// The 16-bit forward with few output tiles (past 16 rows, a
 // round of 256-row tiles or less) over a long K: K ranges as for the fp32
 // limbs, their accumulators in a caller workspace, then scale, bias and one
 // rounding.  Workspace bytes, 0 where no split pays.
