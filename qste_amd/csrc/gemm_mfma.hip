@@ -1599,8 +1599,8 @@ int mfma_backward_pair(const void* dy, int64_t ldy, int dtype, const uint8_t* x_
 // are therefore those of the operands times a power of two that brings the
 // row's largest to 2^kLimbTop (limb_shift), undone in the epilogue: exact in
 // both places, and all 24 bits are kept down to 2^-206 of the largest.  The
-// largest exponent of a row is found in the pass that writes its limbs (rows
-// contiguous: a second read, from the cache), or in a pass before it (evidence,
+// largest exponent of a row is found in the pass that writes its limbs (which
+// holds the row in registers in between), or in a pass before it (evidence,
 // rows of outputs being columns of dy).
 // ---------------------------------------------------------------------------
 
