@@ -380,6 +380,22 @@ def _dequantized_grad(grad_output: Tensor, payload: Tensor, scale: Tensor, ctx, 
     return (flat * factor).view(ctx.shape), None
 
 
+def _takes_kernel_value(kind: str, dtype: torch.dtype, columns: int) -> bool:
+    """Whether the kernel computes the value beside the derivative.
+
+    tanh-GELU leaves it to torch where that is faster: fp32 rows off the kernel's
+    8-element chunks, whose stores are scalar (us, torch's value / the kernel's:
+    8000 x 1001 33.9 / 41.4, 1500 x 2801 21.9 / 25.5; 8184 x 3072 67.9 / 58.3), and fp16
+    rows too long to be held between its two passes (4000 x 20000 252.9 / 286.7,
+    300 x 20000 35.7 / 41.4; fp32 300.8 / 261.5, bf16 248.6 / 246.8)."""
+
+    if (kind, dtype) not in _KERNEL_VALUE:
+        return False
+    if kind != "gelu_tanh":
+        return True
+    return not (dtype is torch.float32 and columns % 8 or dtype is torch.float16 and columns > 16384)
+
+
 class _SmoothFn(Function):
     """Smooth activation retaining its derivative as int8 with a per-row scale."""
 
@@ -390,7 +406,7 @@ class _SmoothFn(Function):
             raise ValueError(f"unknown smooth activation {kind!r}")
         kernel_kind, kernel_param = _kernel_kind(kind, param)
         flat, shape, columns = _flatten(inputs)
-        if flat.dtype in _KERNEL_DTYPES and (kernel_kind, flat.dtype) in _KERNEL_VALUE:
+        if _takes_kernel_value(kernel_kind, flat.dtype, columns):
             out, payload, scale = kernels.smooth_activation(flat, kernel_kind, kernel_param)
             output = out.view(shape)
             if kernel_kind == "gelu_tanh" and not inputs.is_contiguous():

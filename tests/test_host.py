@@ -950,3 +950,29 @@ def test_swiglu_mlp_node_composes_the_layers(fake, monkeypatch):
         assert torch.allclose(e0[name], e1[name], rtol=1e-4, atol=1e-6), name
     for a, b in zip(s0, s1):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-6)
+
+
+def test_tanh_gelu_takes_torchs_value_off_the_kernels_rows(monkeypatch):
+    """fp32 rows off whole chunks and fp16 rows past what the kernel holds take
+    torch's value, the others the kernel's (which is told no output then)."""
+
+    import torch
+
+    import qste_amd as qste
+    from qste_amd import nn as qnn
+
+    given = []
+
+    def kernel(x, kind, param=0.0, *, output=None, derivative=None):
+        given.append(output is not None)
+        return (x if output is None else output, torch.zeros(x.shape, dtype=torch.int8), torch.ones(x.shape[0]))
+
+    monkeypatch.setattr(qnn.kernels, "smooth_activation", kernel)
+    act = qste.nn.GELU(approximate="tanh")
+    for dtype, columns, torchs in ((torch.float32, 1001, True), (torch.float32, 20000, False), (torch.float32, 3072, False),
+                                   (torch.float16, 20000, True), (torch.float16, 1001, False),
+                                   (torch.float16, 16384, False), (torch.bfloat16, 20000, False),
+                                   (torch.bfloat16, 1001, False)):
+        act(torch.randn(2, columns).to(dtype).requires_grad_(True))
+        assert given.pop() == torchs, (dtype, columns)
+    assert not given
